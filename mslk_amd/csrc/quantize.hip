@@ -15,34 +15,42 @@
 //
 // The pass is HBM-bound (2 B in + 1 B out per element for bf16), so the kernel is organised
 // around 128-bit coalesced loads that stay in registers between the amax pass and the convert
-// pass: a row is owned by a "team" of 64 lanes (one wavefront) or 256 lanes (one workgroup);
-// each lane keeps up to NV vectors of 8 elements.  Rows longer than TEAM*8*NV are streamed twice
-// (the second read hits L2 / Infinity Cache).
+// pass: a row is owned by a "team" of 4 ... 1024 lanes, each of which keeps NV vectors of 8 elements.
+// Rows beyond that are streamed twice (the second read hits L2 / Infinity Cache).
 #include "common.h"
 #include "kernels.h"
 #include "quant_math.h"
+#include "rows.h"
 
 namespace mslk_amd {
 namespace {
 
 // 8 consecutive elements of a row.
-template <int DTYPE> struct Vec8 { uint4 w; };          // 8 x 16-bit
-template <> struct Vec8<2> { uint4 lo, hi; };           // 8 x fp32
+template <int DTYPE> struct Vec8 { v4u w; };            // 8 x 16-bit
+template <> struct Vec8<2> { v4u lo, hi; };             // 8 x fp32
 
-MSLK_AMD_DEVINL void store8_stream(uint2* dst, uint2 val) { store8_write_through(dst, v2i{(int)val.x, (int)val.y}); }
+template <int DTYPE>
+MSLK_AMD_DEVINL Vec8<DTYPE> load_vec8(buffer_t row, uint32_t off) {
+  Vec8<DTYPE> v;
+  if constexpr (DTYPE == 2) {
+    v.lo = buffer_load16(row, off);
+    v.hi = buffer_load16(row, off + 16);
+  } else {
+    v.w = buffer_load16(row, off);
+  }
+  return v;
+}
 
+// Rows longer than the registers hold: 64-bit addressing, streamed twice.
 template <int DTYPE>
 MSLK_AMD_DEVINL Vec8<DTYPE> load_vec8(const void* row_ptr, int vec_idx) {
   Vec8<DTYPE> v;
-  // the input is read once (rows cached in registers) or twice in quick succession: stream it
   if constexpr (DTYPE == 2) {
-    const v4i* p = reinterpret_cast<const v4i*>(row_ptr) + 2 * (int64_t)vec_idx;
-    const v4i a = __builtin_nontemporal_load(p), b = __builtin_nontemporal_load(p + 1);
-    v.lo = make_uint4(a.x, a.y, a.z, a.w);
-    v.hi = make_uint4(b.x, b.y, b.z, b.w);
+    const v4u* p = reinterpret_cast<const v4u*>(row_ptr) + 2 * (int64_t)vec_idx;
+    v.lo = __builtin_nontemporal_load(p);
+    v.hi = __builtin_nontemporal_load(p + 1);
   } else {
-    const v4i a = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(row_ptr) + vec_idx);
-    v.w = make_uint4(a.x, a.y, a.z, a.w);
+    v.w = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(row_ptr) + vec_idx);
   }
   return v;
 }
@@ -52,16 +60,13 @@ MSLK_AMD_DEVINL Vec8<DTYPE> load_vec8(const void* row_ptr, int vec_idx) {
 template <int DTYPE>
 MSLK_AMD_DEVINL uint32_t absmax_bits(uint32_t m, const Vec8<DTYPE>& v) {
   if constexpr (DTYPE == 2) {
-    const uint32_t w[8] = {v.lo.x, v.lo.y, v.lo.z, v.lo.w, v.hi.x, v.hi.y, v.hi.z, v.hi.w};
 #pragma unroll
-    for (int i = 0; i < 8; ++i) m = max(m, w[i] & 0x7FFFFFFFu);
+    for (int i = 0; i < 4; ++i) m = max(max(m, v.lo[i] & 0x7FFFFFFFu), v.hi[i] & 0x7FFFFFFFu);
     return m;
   } else {
-    const uint32_t w[4] = {v.w.x, v.w.y, v.w.z, v.w.w};
     us2 acc = __builtin_bit_cast(us2, m);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      acc = __builtin_elementwise_max(acc, __builtin_bit_cast(us2, w[i] & 0x7FFF7FFFu));
+    for (int i = 0; i < 4; ++i) acc = __builtin_elementwise_max(acc, __builtin_bit_cast(us2, v.w[i] & 0x7FFF7FFFu));
     return __builtin_bit_cast(uint32_t, acc);
   }
 }
@@ -72,64 +77,57 @@ MSLK_AMD_DEVINL uint32_t finish_absmax_bits(uint32_t m) {
   return max(m & 0xFFFFu, m >> 16);
 }
 
-// `factor` is the multiplier `inv` of the torch-branch formula, or the divisor `scale` of the Triton one.
-// TRITON with rcp != 0: x / factor is formed as q0 = x * rcp, e = fma(-q0, factor, x), q = e == 0 ? q0 : fma(e, rcp, q0)
-// with rcp = fl32(1 / factor) -- a handful of instructions instead of a division sequence.  The e4m3 codes are those of the
-// IEEE division for every 16-bit element not above a 16-bit row maximum of at least 2^-64 (checked exhaustively on the
-// CPU, tests/test_oracle.py); the caller passes rcp = 0 for every other row, which then divides.
 // clamp(v, -448, 448) in one instruction (the median of the three; a NaN comes out as -448, like fmin(fmax(v, -448), 448))
 MSLK_AMD_DEVINL float clamp448(float v) { return __builtin_amdgcn_fmed3f(v, -448.0f, 448.0f); }
 
-// PLAIN (torch arithmetic only): the caller knows that no product of the row exceeds 448 (1 + 2^-22) and none is NaN -- a
-// finite row maximum that scale_ub has not cut -- so the hardware conversion alone gives the codes.
-template <int DTYPE, bool TRITON, bool PLAIN = false>
-MSLK_AMD_DEVINL uint2 quantize_vec8(const Vec8<DTYPE>& v, float factor, float rcp = 0.f) {
+// Four fp32 within +-464 -> four codes by the hardware conversion alone.
+MSLK_AMD_DEVINL uint32_t cvt4_plain(float a, float b, float c, float d) {
+  return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(c, d, __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false), true);
+}
+
+// How a row's elements become codes; the same for the whole row.
+enum RowMode : int {
+  kModePlain = 0,    // a finite row maximum that scale_ub has not cut: no quotient exceeds 448 (1 + 2^-22), the bare
+                     // conversion gives the codes.  Torch arithmetic: x * factor.  Triton arithmetic: x / factor with a
+                     // reciprocal and two FMAs, q0 = x r, e = fma(q0, factor, -x), q = fma(-e, r, q0) with r =
+                     // fl32(1 / factor).  The codes are those of the IEEE division for every 16-bit element under every
+                     // 16-bit row maximum of at least 2^-64 (exhaustively checked on the CPU, tests/test_oracle.py; an
+                     // exact quotient leaves e = +0, and -0 added to q0 keeps the sign of a zero).
+  kModeGeneral = 1,  // torch arithmetic with the NaN / overflow fix-up; Triton arithmetic with IEEE divisions and the clamp
+};
+template <int DTYPE, bool TRITON, int MODE>
+MSLK_AMD_DEVINL v2u quantize_vec8(const Vec8<DTYPE>& v, float factor, float rcp) {
   float f[8];
   if constexpr (DTYPE == 2) {
-    const uint32_t w[8] = {v.lo.x, v.lo.y, v.lo.z, v.lo.w, v.hi.x, v.hi.y, v.hi.z, v.hi.w};
-#pragma unroll
-    for (int i = 0; i < 8; ++i) f[i] = __uint_as_float(w[i]);
-  } else {
-    const uint32_t w[4] = {v.w.x, v.w.y, v.w.z, v.w.w};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      f[2 * i] = Traits<DTYPE>::to_f32(w[i] & 0xFFFFu);
-      f[2 * i + 1] = Traits<DTYPE>::to_f32(w[i] >> 16);
+      f[i] = __uint_as_float(v.lo[i]);
+      f[4 + i] = __uint_as_float(v.hi[i]);
     }
-  }
-  if constexpr (TRITON) {
-    if (rcp != 0.f) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float q0 = f[i] * rcp;
-        const float e = __builtin_fmaf(-q0, factor, f[i]);
-        const float q = e == 0.f ? q0 : __builtin_fmaf(e, rcp, q0);
-        f[i] = clamp448(q);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) f[i] = clamp448(f[i] / factor);
-    }
-    // Everything is within +-448 now (a NaN quotient came out of the clamp as -448, as it did with a max / min pair), so
-    // the plain hardware conversion gives the codes; the fix-up for magnitudes beyond 464 has nothing left to do.
-    uint2 r;
-    r.x = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false), true);
-    r.y = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], 0, false), true);
-    return r;
   } else {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) f[i] = f[i] * factor;
-    if constexpr (PLAIN) {
-      uint2 r;
-      r.x = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false), true);
-      r.y = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], 0, false), true);
-      return r;
+    for (int i = 0; i < 4; ++i) {
+      f[2 * i] = Traits<DTYPE>::to_f32(v.w[i] & 0xFFFFu);
+      f[2 * i + 1] = Traits<DTYPE>::to_f32(v.w[i] >> 16);
     }
   }
-  uint2 r;
-  r.x = cvt_pk_e4m3fn(f[0], f[1]) | (cvt_pk_e4m3fn(f[2], f[3]) << 16);
-  r.y = cvt_pk_e4m3fn(f[4], f[5]) | (cvt_pk_e4m3fn(f[6], f[7]) << 16);
-  return r;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    if constexpr (!TRITON) {
+      f[i] = f[i] * factor;
+    } else if constexpr (MODE == kModePlain) {
+      const float q0 = f[i] * rcp;
+      f[i] = __builtin_fmaf(-__builtin_fmaf(q0, factor, -f[i]), rcp, q0);
+    } else {
+      f[i] = clamp448(f[i] / factor);   // within +-448, so the bare conversion serves here too
+    }
+  }
+  if constexpr (TRITON || MODE == kModePlain) {
+    return v2u{cvt4_plain(f[0], f[1], f[2], f[3]), cvt4_plain(f[4], f[5], f[6], f[7])};
+  } else {
+    return v2u{cvt_pk_e4m3fn(f[0], f[1]) | (cvt_pk_e4m3fn(f[2], f[3]) << 16),
+               cvt_pk_e4m3fn(f[4], f[5]) | (cvt_pk_e4m3fn(f[6], f[7]) << 16)};
+  }
 }
 
 // Jagged rows (reference: JAGGED branch of _kernel_quantize_fp8_row, fp8_quantize.py:123-129): rows are
@@ -150,98 +148,107 @@ MSLK_AMD_DEVINL bool row_is_live(const JaggedRows& j, int64_t row) {
   return n < live;
 }
 
-template <int TEAM>
-MSLK_AMD_DEVINL uint32_t team_max(uint32_t m, uint32_t* smem, int team_in_block) {
-  constexpr int SPAN = TEAM < kWave ? TEAM : kWave;   // teams narrower than a wavefront are aligned lane groups of it
-#pragma unroll
-  for (int off = SPAN / 2; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
-  if constexpr (TEAM > kWave) {
-    constexpr int WAVES = TEAM / kWave;
-    const int wave = (threadIdx.x % TEAM) / kWave;
-    uint32_t* s = smem + team_in_block * WAVES;
-    if ((threadIdx.x & 63) == 0) s[wave] = m;
-    __syncthreads();
-    m = s[0];
-#pragma unroll
-    for (int w = 1; w < WAVES; ++w) m = max(m, s[w]);
-  }
-  return m;
-}
-
-// Reciprocal of the Triton-arithmetic divisor for rows that may use the multiply form of quantize_vec8, else 0: the row
-// maximum is a finite 16-bit value of at least 2^-64 that neither the lower bound nor scale_ub replaced.
+// Whether a row takes kModePlain; in the Triton arithmetic `rcp` is then the reciprocal of the divisor.
 template <int DTYPE, bool TRITON>
-MSLK_AMD_DEVINL float triton_fast_rcp(float amax, const float* scale_ub, float triton_eps, float divisor) {
-  if constexpr (!TRITON || DTYPE == 2) return 0.f;
-  const bool ok = scale_ub == nullptr && amax >= triton_eps && amax >= 0x1p-64f && amax < __builtin_inff();
-  return ok ? 1.0f / divisor : 0.f;
+MSLK_AMD_DEVINL bool row_is_plain(float amax, const float* scale_ub, float triton_eps, float divisor, float& rcp) {
+  rcp = 0.f;
+  if (scale_ub != nullptr || !(amax < __builtin_inff())) return false;
+  if constexpr (!TRITON) return true;
+  if constexpr (DTYPE == 2) return false;   // fp32 elements: the short division is proven for 16-bit ones only
+  if (!(amax >= triton_eps && amax >= 0x1p-64f)) return false;
+  rcp = 1.0f / divisor;
+  return true;
 }
 
-// Vector path: K % 8 == 0, row starts 16-byte aligned, output rows 8-byte aligned.
-template <int DTYPE, int TEAM, int NV, bool CACHED, bool TRITON>
-__global__ __launch_bounds__(256) void quantize_rows_vec_kernel(
+// Vector path: K % 8 == 0, row starts 16-byte aligned, output rows 8-byte aligned, at most TEAM * NV vectors of eight
+// elements per row.  TEAM lanes own a row: several rows per wavefront (TEAM < 64), one per wavefront, or one per
+// workgroup of TEAM >= 256 lanes.  Bound by HBM: all NV loads of a lane are in flight before the maximum is formed
+// (rows.h).  Against loads that waited for each other, Triton arithmetic on bf16: 4096 x 4096 11.9 -> 10.0 us (5.0 TB/s),
+// 8192 x 8192 41.8 -> 30.5 (6.6 TB/s), 131072 x 128 16.7 -> 10.8, 64 x 14336 4.9 -> 3.4 (the cost of a launch).
+template <int DTYPE, int TEAM, int NV, bool TRITON>
+__global__ __launch_bounds__(TEAM > 256 ? TEAM : 256) void quantize_rows_vec_kernel(
     const void* __restrict__ x, int64_t rows, int K, int64_t in_stride, uint8_t* __restrict__ out,
     int64_t out_stride, float* __restrict__ scale, const float* __restrict__ scale_ub, JaggedRows jag) {
-  constexpr int TEAMS = 256 / TEAM;
+  constexpr int BLOCK = TEAM > 256 ? TEAM : 256, TEAMS = BLOCK / TEAM;
   constexpr int ELEM_BYTES = (DTYPE == 2) ? 4 : 2;
-  __shared__ uint32_t smem[4];
-  const int team_in_block = threadIdx.x / TEAM;
+  constexpr int ROWS_W = TEAM < kWave ? kWave / TEAM : 1;   // rows of a wavefront
+  static_assert(TEAM <= kWave || TEAM == BLOCK, "a team is part of a wavefront, a wavefront or the workgroup");
+  __shared__ uint32_t smem[BLOCK / kWave];
   const int lane = threadIdx.x % TEAM;
-  const int64_t row = (int64_t)blockIdx.x * TEAMS + team_in_block;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t row0 = (int64_t)blockIdx.x * TEAMS + (TEAM <= kWave ? wave * ROWS_W : 0);   // first row of the wavefront
+  const int sub = TEAM < kWave ? (threadIdx.x & 63) / TEAM : 0;
+  const int64_t row = row0 + sub;
   const bool valid = row < rows;
-  const bool live = valid && row_is_live(jag, row);   // uniform over the team
-  const int nvec = K >> 3;
-  const char* row_ptr = reinterpret_cast<const char*>(x) + (valid ? row : 0) * in_stride * ELEM_BYTES;
-
+  const bool live = valid && row_is_live(jag, row);   // the same in every lane of the team
+  const int64_t base_row = row0 < rows ? row0 : 0;
+  const uint32_t nvec = (uint32_t)K >> 3;
+  // one row per descriptor, whose size ends the row; several rows per descriptor when the team is part of a wavefront
+  const buffer_t src = make_buffer(static_cast<const char*>(x) + base_row * in_stride * ELEM_BYTES,
+                                   TEAM < kWave ? 0x7FFFFFF0u : (live ? (uint32_t)K * ELEM_BYTES : 0u));
+  const buffer_t dst = make_buffer(out + base_row * out_stride, TEAM < kWave ? 0x7FFFFFF0u : (valid ? (uint32_t)K : 0u));
+  auto at = [&](int i, bool ok, uint32_t stride, uint32_t vec_bytes) {   // byte offset of vector i of this lane
+    const uint32_t v = i * TEAM + lane;
+    if constexpr (TEAM < kWave) return ok && v < nvec ? sub * stride + v * vec_bytes : kBeyondBuffer;
+    return v * vec_bytes;
+  };
   Vec8<DTYPE> cache[NV];
-  uint32_t m = 0;
-  if constexpr (CACHED) {
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int idx = i * TEAM + lane;
-      if (live && idx < nvec) {
-        cache[i] = load_vec8<DTYPE>(row_ptr, idx);
-        m = absmax_bits<DTYPE>(m, cache[i]);
-      }
-    }
-  } else {
-    if (live)
-      for (int idx = lane; idx < nvec; idx += TEAM) m = absmax_bits<DTYPE>(m, load_vec8<DTYPE>(row_ptr, idx));
-  }
-  m = team_max<TEAM>(finish_absmax_bits<DTYPE>(m), smem, team_in_block);
-  if (!valid) return;
+  for (int i = 0; i < NV; ++i) cache[i] = load_vec8<DTYPE>(src, at(i, live, (uint32_t)in_stride * ELEM_BYTES, 8 * ELEM_BYTES));
+  uint32_t m = 0;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) m = absmax_bits<DTYPE>(m, cache[i]);   // vectors beyond the row and dead rows read as zero
+  m = team_max<TEAM>(finish_absmax_bits<DTYPE>(m), smem);
 
-  float inv, sc;
+  float inv, sc, rcp;
   const float amax = Traits<DTYPE>::abs_bits_to_f32(m);
   scales_from_amax<DTYPE, TRITON>(amax, scale_ub, jag.triton_eps, inv, sc);
-  if (lane == 0) scale[row] = sc;
-  const float rcp = triton_fast_rcp<DTYPE, TRITON>(amax, scale_ub, jag.triton_eps, inv);
-
-  uint2* out_row = reinterpret_cast<uint2*>(out + row * out_stride);
-  if (!live) {   // an empty row quantizes to zero codes
-    for (int idx = lane; idx < nvec; idx += TEAM) store8_stream(out_row + idx, make_uint2(0u, 0u));
-  } else if constexpr (CACHED) {
-    // torch arithmetic: a row with a finite maximum that scale_ub did not cut needs no NaN / overflow fix-up behind the
-    // hardware conversion (uniform over the team)
-    if (!TRITON && scale_ub == nullptr && amax < __builtin_inff()) {
+  if (lane == 0 && valid) scale[row] = sc;
+  if (row_is_plain<DTYPE, TRITON>(amax, scale_ub, jag.triton_eps, inv, rcp)) {
 #pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        const int idx = i * TEAM + lane;
-        if (idx < nvec) store8_stream(out_row + idx, quantize_vec8<DTYPE, TRITON, !TRITON>(cache[i], inv, rcp));
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        const int idx = i * TEAM + lane;
-        if (idx < nvec) store8_stream(out_row + idx, quantize_vec8<DTYPE, TRITON>(cache[i], inv, rcp));
-      }
-    }
+    for (int i = 0; i < NV; ++i)
+      buffer_store8_through(dst, at(i, valid, (uint32_t)out_stride, 8), quantize_vec8<DTYPE, TRITON, kModePlain>(cache[i], inv, rcp));
   } else {
-    for (int idx = lane; idx < nvec; idx += TEAM)
-      store8_stream(out_row + idx, quantize_vec8<DTYPE, TRITON>(load_vec8<DTYPE>(row_ptr, idx), inv, rcp));
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      buffer_store8_through(dst, at(i, valid, (uint32_t)out_stride, 8), quantize_vec8<DTYPE, TRITON, kModeGeneral>(cache[i], inv, rcp));
   }
   // zero padding columns [K, out_stride)
-  for (int64_t k = K + lane; k < out_stride; k += TEAM) out[row * out_stride + k] = 0;
+  if (valid)
+    for (int64_t k = K + lane; k < out_stride; k += TEAM) out[row * out_stride + k] = 0;
+}
+
+// Vector path for rows beyond the registers: one workgroup per row, read twice (the second read hits the caches).
+template <int DTYPE, bool TRITON>
+__global__ __launch_bounds__(256) void quantize_rows_long_kernel(
+    const void* __restrict__ x, int64_t rows, int K, int64_t in_stride, uint8_t* __restrict__ out,
+    int64_t out_stride, float* __restrict__ scale, const float* __restrict__ scale_ub, JaggedRows jag) {
+  constexpr int ELEM_BYTES = (DTYPE == 2) ? 4 : 2;
+  __shared__ uint32_t smem[4];
+  const int64_t row = blockIdx.x;
+  const int nvec = row_is_live(jag, row) ? K >> 3 : 0;
+  const char* row_ptr = reinterpret_cast<const char*>(x) + row * in_stride * ELEM_BYTES;
+  uint32_t m = 0;
+  for (int idx = threadIdx.x; idx < nvec; idx += 256) m = absmax_bits<DTYPE>(m, load_vec8<DTYPE>(row_ptr, idx));
+  m = team_max<256>(finish_absmax_bits<DTYPE>(m), smem);
+  float inv, sc, rcp;
+  const float amax = Traits<DTYPE>::abs_bits_to_f32(m);
+  scales_from_amax<DTYPE, TRITON>(amax, scale_ub, jag.triton_eps, inv, sc);
+  if (threadIdx.x == 0) scale[row] = sc;
+  uint8_t* out_row = out + row * out_stride;
+  if (row_is_plain<DTYPE, TRITON>(amax, scale_ub, jag.triton_eps, inv, rcp)) {
+    for (int idx = threadIdx.x; idx < nvec; idx += 256) {
+      const v2u q = quantize_vec8<DTYPE, TRITON, kModePlain>(load_vec8<DTYPE>(row_ptr, idx), inv, rcp);
+      store8_write_through(out_row + (int64_t)idx * 8, v2i{(int)q.x, (int)q.y});
+    }
+  } else {
+    for (int idx = threadIdx.x; idx < nvec; idx += 256) {
+      const v2u q = quantize_vec8<DTYPE, TRITON, kModeGeneral>(load_vec8<DTYPE>(row_ptr, idx), inv, rcp);
+      store8_write_through(out_row + (int64_t)idx * 8, v2i{(int)q.x, (int)q.y});
+    }
+  }
+  // padding columns, and all of a dead row
+  for (int64_t k = (int64_t)nvec * 8 + threadIdx.x; k < out_stride; k += 256) out_row[k] = 0;
 }
 
 // Generic path: any K, any alignment; one workgroup per row, two passes.  Full groups of eight elements move as 16- / 32-byte
@@ -269,7 +276,7 @@ __global__ __launch_bounds__(256) void quantize_rows_generic_kernel(
     if constexpr (DTYPE == 2) m = max(m, __float_as_uint(xr[k]) & 0x7FFFFFFFu);
     else m = max(m, (uint32_t)xr[k] & 0x7FFFu);
   }
-  m = team_max<256>(m, smem, 0);
+  m = team_max<256>(m, smem);
   float inv, sc;
   scales_from_amax<DTYPE, TRITON>(Traits<DTYPE>::abs_bits_to_f32(m), scale_ub, jag.triton_eps, inv, sc);
   if (threadIdx.x == 0) scale[row] = sc;
@@ -277,7 +284,7 @@ __global__ __launch_bounds__(256) void quantize_rows_generic_kernel(
   for (int64_t idx = threadIdx.x; idx < nvec; idx += 256) {
     Vec8<DTYPE> v;
     __builtin_memcpy(&v, xb + idx * sizeof(Vec8<DTYPE>), sizeof(Vec8<DTYPE>));
-    const uint2 q = quantize_vec8<DTYPE, TRITON>(v, inv);
+    const v2u q = quantize_vec8<DTYPE, TRITON, kModeGeneral>(v, inv, 0.f);
     __builtin_memcpy(out_row + idx * 8, &q, 8);
   }
   for (int64_t k = nvec * 8 + threadIdx.x; k < out_stride; k += 256) {
@@ -377,12 +384,13 @@ __global__ void cast_e4m3fn_kernel(const float* __restrict__ in, int64_t n, uint
     out[i] = (uint8_t)(cvt_pk_e4m3fn(in[i], 0.0f) & 0xFFu);
 }
 
+template <int N> struct Int { static constexpr int value = N; };
+
 template <int DTYPE, bool TRITON>
 hipError_t launch_quantize_t(const void* x, int64_t rows, int64_t K, int64_t in_stride, uint8_t* out,
                              int64_t out_stride, float* scale, const float* scale_ub, JaggedRows jag,
                              hipStream_t s) {
   constexpr int ELEM_BYTES = (DTYPE == 2) ? 4 : 2;
-  constexpr int NV = 16;
   const bool vec_ok = (K % 8 == 0) && (K < (int64_t(1) << 31)) && ((in_stride * ELEM_BYTES) % 16 == 0) &&
                       (reinterpret_cast<uintptr_t>(x) % 16 == 0) && (out_stride % 8 == 0) &&
                       (reinterpret_cast<uintptr_t>(out) % 8 == 0);
@@ -392,36 +400,34 @@ hipError_t launch_quantize_t(const void* x, int64_t rows, int64_t K, int64_t in_
     return hipGetLastError();
   }
   const int k = (int)K;
-  // Short rows (per-head quantization: K = 64 ... 256) in large numbers: 8 / 16 / 32 lanes per row, one 16-byte load each,
-  // so that a wavefront covers 8 / 4 / 2 rows instead of idling three quarters of its lanes (131072 x 128 bf16: 37 -> 12 us).
-  if (K <= 256 && rows >= 4096) {
-    if (K <= 64)
-      quantize_rows_vec_kernel<DTYPE, 8, 1, true, TRITON><<<(unsigned)((rows + 31) / 32), 256, 0, s>>>(x, rows, k, in_stride, out, out_stride, scale, scale_ub, jag);
-    else if (K <= 128)
-      quantize_rows_vec_kernel<DTYPE, 16, 1, true, TRITON><<<(unsigned)((rows + 15) / 16), 256, 0, s>>>(x, rows, k, in_stride, out, out_stride, scale, scale_ub, jag);
-    else
-      quantize_rows_vec_kernel<DTYPE, 32, 1, true, TRITON><<<(unsigned)((rows + 7) / 8), 256, 0, s>>>(x, rows, k, in_stride, out, out_stride, scale, scale_ub, jag);
+  const int64_t nvec = K / 8;
+  auto team = [&](auto t, auto n) {
+    constexpr int TEAM = decltype(t)::value, NV = decltype(n)::value, TEAMS = TEAM > 256 ? 1 : 256 / TEAM;
+    quantize_rows_vec_kernel<DTYPE, TEAM, NV, TRITON><<<(unsigned)((rows + TEAMS - 1) / TEAMS), TEAM > 256 ? TEAM : 256, 0, s>>>(
+        x, rows, k, in_stride, out, out_stride, scale, scale_ub, jag);
     return hipGetLastError();
+  };
+  // From 2048 rows on the chip is full with a wavefront or less per row: as many lanes as give each one to four vectors,
+  // the per-row work (reduction, divisions) then being shared by more elements.  131072 x 128 bf16, Triton arithmetic, by
+  // lanes per row: 4 15.3, 8 10.8, 16 11.4, 32 16.2 us; 32768 x 1024: 64 x 2 vectors 16.8, 256 29.9; 8192 x 2048: 64 x 4
+  // 9.9, 256 10.8.  Longer rows take a workgroup: 8192 x 4096: 256 x 2 16.7, 64 x 8 17.7, 512 19.4; 8192 x 8192: 256 x 4
+  // 30.5, 512 x 2 30.6, 1024 39.9; 4096 x 16384: 512 x 4 31.1, 256 x 8 31.5, 1024 x 2 33.0.
+  // (The bound on the strides keeps the byte offsets of a wavefront's up to eight rows below 2^31.)
+  if (rows >= 2048 && nvec <= 256 && in_stride * ELEM_BYTES < (1 << 26) && out_stride < (1 << 26)) {
+    if (nvec <= 8) return team(Int<8>{}, Int<1>{});
+    if (nvec <= 16) return team(Int<8>{}, Int<2>{});
+    if (nvec <= 32) return team(Int<16>{}, Int<2>{});
+    if (nvec <= 64) return team(Int<32>{}, Int<2>{});
+    if (nvec <= 128) return team(Int<64>{}, Int<2>{});
+    return team(Int<64>{}, Int<4>{});
   }
-  // One wavefront per row once there are enough rows to fill the chip; otherwise a workgroup per row.
-  if (K <= kWave * 8 * NV && rows >= 2048) {
-    const unsigned blocks = (unsigned)((rows + 3) / 4);
-    if (K <= kWave * 8 * 4)
-      quantize_rows_vec_kernel<DTYPE, 64, 4, true, TRITON><<<blocks, 256, 0, s>>>(x, rows, k, in_stride, out, out_stride, scale, scale_ub, jag);
-    else if (K <= kWave * 8 * 8)
-      quantize_rows_vec_kernel<DTYPE, 64, 8, true, TRITON><<<blocks, 256, 0, s>>>(x, rows, k, in_stride, out, out_stride, scale, scale_ub, jag);
-    else
-      quantize_rows_vec_kernel<DTYPE, 64, NV, true, TRITON><<<blocks, 256, 0, s>>>(x, rows, k, in_stride, out, out_stride, scale, scale_ub, jag);
-  } else if (K <= 256 * 8 * 4) {
-    quantize_rows_vec_kernel<DTYPE, 256, 4, true, TRITON><<<(unsigned)rows, 256, 0, s>>>(x, rows, k, in_stride, out, out_stride, scale, scale_ub, jag);
-  } else if (K <= 256 * 8 * NV) {
-    quantize_rows_vec_kernel<DTYPE, 256, NV, true, TRITON><<<(unsigned)rows, 256, 0, s>>>(x, rows, k, in_stride, out, out_stride, scale, scale_ub, jag);
-  } else if (DTYPE != 2 && K <= 256 * 8 * 32) {
-    // 16-bit rows up to 65536 elements still fit the registers of one workgroup (32 x 16 bytes per lane)
-    quantize_rows_vec_kernel<DTYPE, 256, (DTYPE != 2 ? 32 : 1), true, TRITON><<<(unsigned)rows, 256, 0, s>>>(x, rows, k, in_stride, out, out_stride, scale, scale_ub, jag);
-  } else {
-    quantize_rows_vec_kernel<DTYPE, 256, 1, false, TRITON><<<(unsigned)rows, 256, 0, s>>>(x, rows, k, in_stride, out, out_stride, scale, scale_ub, jag);
-  }
+  if (nvec <= 256) return team(Int<256>{}, Int<1>{});
+  if (nvec <= 512) return team(Int<256>{}, Int<2>{});
+  if (nvec <= 1024) return team(Int<256>{}, Int<4>{});
+  if (nvec <= 2048) return team(Int<512>{}, Int<4>{});
+  if (nvec <= 4096) return team(Int<1024>{}, Int<4>{});
+  if (DTYPE != 2 && nvec <= 8192) return team(Int<1024>{}, Int<(DTYPE != 2 ? 8 : 1)>{});
+  quantize_rows_long_kernel<DTYPE, TRITON><<<(unsigned)rows, 256, 0, s>>>(x, rows, k, in_stride, out, out_stride, scale, scale_ub, jag);
   return hipGetLastError();
 }
 
