@@ -14,11 +14,12 @@
 // The two divisions of the scale are IEEE-correct; sigmoid is rcp(1 + exp(-x)) on the hardware
 // transcendental units, accurate to a few fp32 ulp.
 //
-// HBM-bound (silu: 4 B in + 1 B out per element for 16-bit inputs; gather: 2 B in + 1 B out).  One
-// workgroup of 256 lanes owns a row; the produced fp32 values stay in registers between the
+// HBM-bound (silu: 4 B in + 1 B out per element for 16-bit inputs; gather: 2 B in + 1 B out).  A wavefront or a
+// workgroup owns a row; the produced fp32 values stay in registers between the
 // maximum pass and the convert pass for rows of up to 16384 elements.
 #include "common.h"
 #include "kernels.h"
+#include "rows.h"
 
 namespace mslk_amd {
 namespace {
@@ -63,8 +64,7 @@ MSLK_AMD_DEVINL float silu_mul(float a, float b) {
 
 // 8 consecutive 16-bit elements -> fp32
 template <int DTYPE>
-MSLK_AMD_DEVINL void unpack8(const v4i& v, float (&f)[8]) {
-  const uint32_t w[4] = {(uint32_t)v.x, (uint32_t)v.y, (uint32_t)v.z, (uint32_t)v.w};
+MSLK_AMD_DEVINL void unpack8(const v4u& w, float (&f)[8]) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     f[2 * i] = elem_to_f32<DTYPE>(w[i] & 0xFFFFu);
@@ -99,19 +99,27 @@ MSLK_AMD_DEVINL RowSource resolve_row(const FusedQuantArgs& p, int64_t row) {
   return r;
 }
 
+// Eight elements of the row from its 16 input bytes (32 for the gated product).
 template <int OP, int DTYPE>
-MSLK_AMD_DEVINL void produce8(const RowSource& r, int vec, float (&y)[8]) {
+MSLK_AMD_DEVINL void produce8(const v4u& va, const v4u& vb, float score, float (&y)[8]) {
   float a[8];
-  unpack8<DTYPE>(__builtin_nontemporal_load(reinterpret_cast<const v4i*>(r.a) + vec), a);
+  unpack8<DTYPE>(va, a);
   if constexpr (OP == kFusedSiluMul) {
     float b[8];
-    unpack8<DTYPE>(__builtin_nontemporal_load(reinterpret_cast<const v4i*>(r.b) + vec), b);
+    unpack8<DTYPE>(vb, b);
 #pragma unroll
     for (int i = 0; i < 8; ++i) y[i] = silu_mul(a[i], b[i]);
   } else {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = a[i] * r.score;
+    for (int i = 0; i < 8; ++i) y[i] = a[i] * score;
   }
+}
+template <int OP, int DTYPE>
+MSLK_AMD_DEVINL void produce8(const RowSource& r, int vec, float (&y)[8]) {
+  const v4u va = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(r.a) + vec);
+  v4u vb = va;
+  if constexpr (OP == kFusedSiluMul) vb = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(r.b) + vec);
+  produce8<OP, DTYPE>(va, vb, r.score, y);
 }
 
 template <int OP, int DTYPE>
@@ -119,14 +127,6 @@ MSLK_AMD_DEVINL float produce1(const FusedQuantArgs& p, const RowSource& r, int 
   const float a = elem_to_f32<DTYPE>(reinterpret_cast<const uint16_t*>(r.a)[k]);
   if constexpr (OP == kFusedSiluMul) return silu_mul(a, elem_to_f32<DTYPE>(reinterpret_cast<const uint16_t*>(r.b)[k]));
   else return a * r.score;
-}
-
-MSLK_AMD_DEVINL uint32_t block_max_bits(uint32_t m, uint32_t* smem) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
-  if ((threadIdx.x & 63) == 0) smem[threadIdx.x >> 6] = m;
-  __syncthreads();
-  return max(max(smem[0], smem[1]), max(smem[2], smem[3]));
 }
 
 // |y| as raw bits orders like the value for non-negative floats and puts every NaN above +inf.
@@ -138,76 +138,93 @@ MSLK_AMD_DEVINL void row_scales(uint32_t max_bits, const float* scale_ub, float&
   inv = 1.0f / s;
 }
 
-MSLK_AMD_DEVINL uint2 quantize8_saturating(const float (&y)[8], float s) {
+MSLK_AMD_DEVINL v2u quantize8_saturating(const float (&y)[8], float s) {
   float f[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) f[i] = __builtin_amdgcn_fmed3f(y[i] * s, -kMaxFp8, kMaxFp8);   // clamp; a NaN comes out as -448, as from fmin(fmax())
   // within +-448 the hardware conversion alone gives the codes (no NaN / overflow fix-up to apply)
-  uint2 r;
+  v2u r;
   r.x = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false), true);
   r.y = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], 0, false), true);
   return r;
 }
 
-// Vector path: D % 8 == 0, input rows 16-byte aligned, output rows 8-byte aligned.  NV > 0: the lane
-// keeps NV x 8 produced values in registers; NV == 0: rows of any length, produced twice.
-// TEAM = 256: one workgroup per row; TEAM = 64: one wavefront per row, four rows per workgroup (rows of MoE
-// intermediate sizes, 768 ... 2048 elements, leave most of a 256-lane team idle).
-template <int OP, int DTYPE, int NV, int TEAM = 256>
+// Vector path: D % 8 == 0, input rows 16-byte aligned, output rows 8-byte aligned, at most TEAM * NV vectors of eight per
+// row, whose produced values stay in registers.  Bound by HBM: all loads of a lane are in flight before the first value is
+// formed (rows.h).  Against loads that waited for each other, bf16: gather 8192 x 5120 27.4 -> 21.8 us (5.8 TB/s), 32768 x 2048
+// 39.1 -> 33.1 (6.1 TB/s), 16384 x 1408 16.2 -> 13.6; the gated product, which had two loads per vector in flight, 8192 x
+// 4096 27.4 -> 27.1 (6.2 TB/s), 32768 x 2048 53.7 -> 49.6 (6.8 TB/s).
+// TEAM = 64: one wavefront per row, four rows per workgroup (rows of MoE intermediate sizes in large numbers); otherwise
+// one workgroup of TEAM lanes per row.
+template <int OP, int DTYPE, int TEAM, int NV>
 __global__ __launch_bounds__(256) void fused_quant_vec_kernel(FusedQuantArgs p) {
+  static_assert(TEAM == kWave || TEAM == 256, "a wavefront or a workgroup of four per row");
   __shared__ uint32_t smem[4];
-  const int64_t row = TEAM == 256 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (TEAM != 256 && row >= p.rows) return;      // uniform over the wavefront; this variant has no workgroup barrier
+  const int64_t row = TEAM == kWave ? (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : (int64_t)blockIdx.x;
+  if (TEAM == kWave && row >= p.rows) return;    // uniform over the wavefront; this variant has no workgroup barrier
   const RowSource r = resolve_row<OP>(p, row);   // uniform over the team
   if (!r.live) return;
-  const int nvec = p.D >> 3;
-  const int lane = TEAM == 256 ? (int)threadIdx.x : (int)(threadIdx.x & 63);
+  const int lane = threadIdx.x % TEAM;
+  const buffer_t src_a = make_buffer(r.a, (uint32_t)p.D * 2);
+  const buffer_t src_b = make_buffer(OP == kFusedSiluMul ? r.b : r.a, (uint32_t)p.D * 2);
+  v4u va[NV], vb[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    va[i] = buffer_load16(src_a, (uint32_t)(i * TEAM + lane) * 16);
+    if constexpr (OP == kFusedSiluMul) vb[i] = buffer_load16(src_b, (uint32_t)(i * TEAM + lane) * 16);
+  }
+  float y[NV][8];
   uint32_t m = 0;
-  float cache[NV > 0 ? NV : 1][8];
-  if constexpr (NV > 0) {
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int vec = i * TEAM + lane;
-      if (vec < nvec) {
-        produce8<OP, DTYPE>(r, vec, cache[i]);
+  for (int i = 0; i < NV; ++i) {   // vectors beyond the row read as zero and produce zero
+    produce8<OP, DTYPE>(va[i], vb[i], r.score, y[i]);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) m = max(m, __float_as_uint(cache[i][e]) & 0x7FFFFFFFu);
-      }
-    }
-  } else {
-    for (int vec = lane; vec < nvec; vec += TEAM) {
-      float y[8];
-      produce8<OP, DTYPE>(r, vec, y);
+    for (int e = 0; e < 8; ++e) m = max(m, __float_as_uint(y[i][e]) & 0x7FFFFFFFu);
+  }
+  if constexpr (OP == kFusedGatherScale) {
+    // (0 * score is NaN for an infinite or NaN score: a vector beyond the row must not enter the maximum then)
+    if (!(__builtin_fabsf(r.score) < __builtin_inff())) {
+      m = 0;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) m = max(m, __float_as_uint(y[e]) & 0x7FFFFFFFu);
+      for (int i = 0; i < NV; ++i)
+        if (i * TEAM + lane < (p.D >> 3))
+#pragma unroll
+          for (int e = 0; e < 8; ++e) m = max(m, __float_as_uint(y[i][e]) & 0x7FFFFFFFu);
     }
   }
-  if constexpr (TEAM == 256) {
-    m = block_max_bits(m, smem);
-  } else {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
-  }
+  m = team_max<TEAM>(m, smem);
   float s, inv;
   row_scales(m, p.scale_ub, s, inv);
   if (lane == 0) p.out_scale[row] = inv;
-  uint2* out_row = reinterpret_cast<uint2*>(p.out + row * (int64_t)p.D);
-  if constexpr (NV > 0) {
+  const buffer_t dst = make_buffer(p.out + row * (int64_t)p.D, (uint32_t)p.D);
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int vec = i * TEAM + lane;
-      if (vec < nvec) {
-        const uint2 q = quantize8_saturating(cache[i], s);
-        store8_write_through(reinterpret_cast<v2i*>(out_row + vec), v2i{(int)q.x, (int)q.y});
-      }
-    }
-  } else {
-    for (int vec = lane; vec < nvec; vec += TEAM) {
-      float y[8];
-      produce8<OP, DTYPE>(r, vec, y);
-      const uint2 q = quantize8_saturating(y, s);
-      store8_write_through(reinterpret_cast<v2i*>(out_row + vec), v2i{(int)q.x, (int)q.y});
-    }
+  for (int i = 0; i < NV; ++i) buffer_store8_through(dst, (uint32_t)(i * TEAM + lane) * 8, quantize8_saturating(y[i], s));
+}
+
+// Rows of any length: as above, produced twice.
+template <int OP, int DTYPE>
+__global__ __launch_bounds__(256) void fused_quant_long_kernel(FusedQuantArgs p) {
+  __shared__ uint32_t smem[4];
+  const int64_t row = blockIdx.x;
+  const RowSource r = resolve_row<OP>(p, row);
+  if (!r.live) return;
+  const int nvec = p.D >> 3;
+  uint32_t m = 0;
+  float y[8];
+  for (int vec = threadIdx.x; vec < nvec; vec += 256) {
+    produce8<OP, DTYPE>(r, vec, y);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) m = max(m, __float_as_uint(y[e]) & 0x7FFFFFFFu);
+  }
+  m = team_max<256>(m, smem);
+  float s, inv;
+  row_scales(m, p.scale_ub, s, inv);
+  if (threadIdx.x == 0) p.out_scale[row] = inv;
+  uint8_t* out_row = p.out + row * (int64_t)p.D;
+  for (int vec = threadIdx.x; vec < nvec; vec += 256) {
+    produce8<OP, DTYPE>(r, vec, y);
+    const v2u q = quantize8_saturating(y, s);
+    store8_write_through(out_row + (int64_t)vec * 8, v2i{(int)q.x, (int)q.y});
   }
 }
 
@@ -220,7 +237,7 @@ __global__ __launch_bounds__(256) void fused_quant_generic_kernel(FusedQuantArgs
   if (!r.live) return;
   uint32_t m = 0;
   for (int k = threadIdx.x; k < p.D; k += 256) m = max(m, __float_as_uint(produce1<OP, DTYPE>(p, r, k)) & 0x7FFFFFFFu);
-  m = block_max_bits(m, smem);
+  m = team_max<256>(m, smem);
   float s, inv;
   row_scales(m, p.scale_ub, s, inv);
   if (threadIdx.x == 0) p.out_scale[row] = inv;
@@ -238,23 +255,27 @@ hipError_t launch_fused_t(const FusedQuantArgs& p, hipStream_t s) {
                       reinterpret_cast<uintptr_t>(p.out) % 8 == 0;
   if (!vec_ok) {
     fused_quant_generic_kernel<OP, DTYPE><<<rows, 256, 0, s>>>(p);
-  } else if (p.D <= 2048 && p.rows >= 2048) {
-    // enough rows to fill the chip with one wavefront each
-    const unsigned blocks = (unsigned)((p.rows + 3) / 4);
-    if (p.D <= 512) fused_quant_vec_kernel<OP, DTYPE, 1, 64><<<blocks, 256, 0, s>>>(p);
-    else if (p.D <= 1024) fused_quant_vec_kernel<OP, DTYPE, 2, 64><<<blocks, 256, 0, s>>>(p);
-    else fused_quant_vec_kernel<OP, DTYPE, 4, 64><<<blocks, 256, 0, s>>>(p);
-  } else if (p.D <= 2048) {
-    fused_quant_vec_kernel<OP, DTYPE, 1><<<rows, 256, 0, s>>>(p);
-  } else if (p.D <= 4096) {
-    fused_quant_vec_kernel<OP, DTYPE, 2><<<rows, 256, 0, s>>>(p);
-  } else if (p.D <= 8192) {
-    fused_quant_vec_kernel<OP, DTYPE, 4><<<rows, 256, 0, s>>>(p);
-  } else if (p.D <= 16384) {
-    fused_quant_vec_kernel<OP, DTYPE, 8><<<rows, 256, 0, s>>>(p);
-  } else {
-    fused_quant_vec_kernel<OP, DTYPE, 0><<<rows, 256, 0, s>>>(p);
+    return hipGetLastError();
   }
+  auto team = [&](auto t, auto n) {
+    constexpr int TEAM = decltype(t)::value, NV = decltype(n)::value;
+    fused_quant_vec_kernel<OP, DTYPE, TEAM, NV><<<TEAM == kWave ? (rows + 3) / 4 : rows, 256, 0, s>>>(p);
+    return hipGetLastError();
+  };
+  // As few vectors as hold the row: one beyond its end costs the arithmetic all the same (32768 x 768, gated product: 64 x 2
+  // 22.2, 64 x 4 35.1 us).  In large numbers short rows take a wavefront each (gather, 32768 x 2048: 64 x 4 33.1, 256 45.1);
+  // the gated product, which computes more per byte, only up to two vectors (32768 x 2048: 256 49.6, 64 x 4 52.3).
+  if (p.rows >= 2048 && p.D <= (OP == kFusedSiluMul ? 1024 : 2048)) {
+    if (p.D <= 512) return team(Int<64>{}, Int<1>{});
+    if (p.D <= 1024) return team(Int<64>{}, Int<2>{});
+    return team(Int<64>{}, Int<(OP == kFusedSiluMul ? 2 : 4)>{});
+  }
+  if (p.D <= 2048) return team(Int<256>{}, Int<1>{});
+  if (p.D <= 4096) return team(Int<256>{}, Int<2>{});
+  if (p.D <= 6144) return team(Int<256>{}, Int<3>{});
+  if (p.D <= 8192) return team(Int<256>{}, Int<4>{});
+  if (p.D <= 16384) return team(Int<256>{}, Int<8>{});
+  fused_quant_long_kernel<OP, DTYPE><<<rows, 256, 0, s>>>(p);
   return hipGetLastError();
 }
 

@@ -384,8 +384,6 @@ __global__ void cast_e4m3fn_kernel(const float* __restrict__ in, int64_t n, uint
     out[i] = (uint8_t)(cvt_pk_e4m3fn(in[i], 0.0f) & 0xFFu);
 }
 
-template <int N> struct Int { static constexpr int value = N; };
-
 template <int DTYPE, bool TRITON>
 hipError_t launch_quantize_t(const void* x, int64_t rows, int64_t K, int64_t in_stride, uint8_t* out,
                              int64_t out_stride, float* scale, const float* scale_ub, JaggedRows jag,

@@ -14,6 +14,8 @@ typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 typedef __amdgpu_buffer_rsrc_t buffer_t;
 
+template <int N> struct Int { static constexpr int value = N; };   // a template argument carried by a value
+
 constexpr uint32_t kBeyondBuffer = 0x80000000u;   // an offset no descriptor made here reaches (sizes stay below 2^31)
 constexpr int kCacheNt = 2, kCacheSc1 = 16;       // cache policy bits of the buffer instructions: non-temporal, system scope
 
