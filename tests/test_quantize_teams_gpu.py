@@ -61,3 +61,13 @@ def test_dead_rows_and_padding_columns(groups, per_group, K):
     q = q.cpu().view(torch.uint8)
     assert torch.equal(q[..., :K], rq.view(torch.uint8)) and not q[..., K:].any()
     assert torch.equal(s.cpu(), rs)
+
+
+@pytest.mark.parametrize("rows,K", [(1, 8), (300, 8), (257, 24), (1000, 576), (3, 65544), (129, 1000), (70001, 16)])
+def test_dequantized_rows_take_their_own_scale(rows, K):
+    """The row of a chunk comes from a multiply and a shift: chunk counts per row of one, a power of two and neither."""
+    g = torch.Generator().manual_seed(rows + K)
+    q = torch.randint(0, 0x7E, (rows, K), generator=g, dtype=torch.uint8).view(torch.float8_e4m3fn)
+    s = torch.rand(rows, generator=g) + 0.5
+    y = mslk_amd.dequantize_fp8_row(q.to(DEV), s.to(DEV))
+    assert torch.equal(y.cpu(), O.dequantize_fp8_row_bf16(q, s))
