@@ -5,7 +5,7 @@ Importing the package registers `torch.ops.mslk.f8f8bf16_rowwise`, `..._rowwise_
 `..._rowwise_grouped_mm`, `..._rowwise_batched` and
 `torch.ops.mslk.quantize_fp8_row` / `dequantize_fp8_row`, all backed by hand-written HIP kernels in libmslk_amd.so.
 """
-from . import _lib  # noqa: F401
+from . import _lib, quantize  # noqa: F401
 from .quantize import (quantize_fp8_row, quantize_fp8_per_row, dequantize_fp8_row,  # noqa: F401
                        FP8_DTYPE)  # noqa: F401
 from . import gemm  # noqa: F401  (registers torch.ops.mslk.*)
@@ -16,6 +16,21 @@ from .gemm import (f8f8bf16_rowwise, f8f8bf16_rowwise_out, quantize_f8f8bf16_row
                    f8f8bf16_rowwise_grouped_cat, f8f8bf16_rowwise_grouped_stacked,
                    f8f8bf16_rowwise_grouped_mm, f8f8bf16_rowwise_grouped_dynamic,
                    f8f8bf16_rowwise_batched)
+
+
+def _register_missing(error: RuntimeError) -> None:
+    """The build is missing: every operator with a native kernel raises `error` when it is used on a GPU."""
+    def fail(*_args, **_kwargs):
+        raise error
+
+    for library, names in ((quantize._triton_library, ["quantize_fp8_row"]),
+                           (quantize._library, ["quantize_fp8_per_row", "dequantize_fp8_row"] + list(moe._OPS)
+                            + [n for n in gemm._SCHEMAS if n not in gemm._PYTHON_IMPLS])):
+        for name in names:
+            library.impl(name, fail, "CUDA", allow_override=True)
+
+
+_lib.load_torch_ops(_register_missing)   # every schema is defined by now
 
 __all__ = ["quantize_fp8_row", "quantize_fp8_per_row", "dequantize_fp8_row", "silu_mul_quant", "gather_scale_quant_dense_tokens", "f8f8bf16_rowwise", "f8f8bf16_rowwise_out", "quantize_f8f8bf16_rowwise", "f8f8f16_rowwise", "f8f8bf16_rowwise_preshuffle", "f8f8f16_rowwise_preshuffle", "preshuffle_b_mfma", "ck_preshuffle",
            "f8f8bf16_rowwise_grouped", "f8f8bf16_rowwise_grouped_cat", "f8f8bf16_rowwise_grouped_stacked",

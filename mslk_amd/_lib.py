@@ -12,6 +12,9 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 # MSLK_AMD_LIBRARY overrides the location of the built library (e.g. an out-of-tree build).
 LIB_PATH = os.environ.get("MSLK_AMD_LIBRARY") or os.path.join(_HERE, "libmslk_amd.so")
 
+# The operators as native PyTorch kernels on top of it (csrc/torch_ops.cpp).
+TORCH_OPS_PATH = os.path.join(_HERE, "_torch_ops.so")
+
 _lib = None
 
 # name -> (restype, argtypes); mirrors include/mslk_amd.h one to one
@@ -66,13 +69,16 @@ SIGNATURES = {
 }
 
 
+def _missing(path: str) -> RuntimeError:
+    return RuntimeError(f"mslk_amd: {path} is missing. Build it with `python -m mslk_amd.build` "
+                        "(hipcc --offload-arch=gfx950); there is no CPU or PyTorch fallback.")
+
+
 def lib() -> ctypes.CDLL:
     global _lib
     if _lib is None:
         if not os.path.exists(LIB_PATH):
-            raise RuntimeError(
-                f"mslk_amd: {LIB_PATH} is missing. Build it with `python -m mslk_amd.build` "
-                "(hipcc --offload-arch=gfx950); there is no CPU or PyTorch fallback.")
+            raise _missing(LIB_PATH)
         L = ctypes.CDLL(LIB_PATH)
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(L, name)
@@ -86,3 +92,19 @@ def check(rc: int) -> None:
     """Turn a non-zero return code into the RuntimeError a TORCH_CHECK would have raised."""
     if rc != 0:
         raise RuntimeError(lib().mslk_amd_last_error().decode())
+
+
+def load_torch_ops(register_missing) -> None:
+    """Loads the native operator kernels, which registers them with the dispatcher, and binds them to the C ABI.  When the
+    build is missing, `register_missing(error)` is called instead, to make the operators raise `error` when they are used."""
+    for path in (LIB_PATH, TORCH_OPS_PATH):
+        if not os.path.exists(path):
+            register_missing(_missing(path))
+            return
+    import torch
+    torch.ops.load_library(TORCH_OPS_PATH)
+    bind = ctypes.CDLL(TORCH_OPS_PATH).mslk_amd_torch_bind
+    bind.restype, bind.argtypes = c_char_p, [c_char_p]
+    error = bind(os.fsencode(LIB_PATH))
+    if error is not None:
+        raise RuntimeError(f"mslk_amd: cannot bind {LIB_PATH}: {error.decode()}")

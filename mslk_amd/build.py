@@ -1,4 +1,4 @@
-"""Builds mslk_amd/libmslk_amd.so with hipcc for gfx950:  python -m mslk_amd.build [--force]"""
+"""Builds mslk_amd/libmslk_amd.so with hipcc for gfx950 and mslk_amd/_torch_ops.so on top of it:  python -m mslk_amd.build [--force]"""
 from __future__ import annotations
 
 import os
@@ -9,7 +9,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 
 
 def build(force: bool = False, jobs: int = 8) -> str:
-    cmd = ["make", "-C", os.path.join(_HERE, "csrc"), f"-j{jobs}"]
+    cmd = ["make", "-C", os.path.join(_HERE, "csrc"), f"-j{jobs}", f"PYTHON={sys.executable}"]
     if force:
         cmd.append("-B")
     subprocess.check_call(cmd)
