@@ -46,6 +46,29 @@ MSLK_AMD_DEVINL int64_t uniform64(int64_t v) {
   return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
+// x + y for 0 <= x, y < 2^31, at most 2^31 - 1 (one unsigned addition cannot wrap): sizes that add up to more than a tensor
+// holds always end beyond it.
+MSLK_AMD_DEVINL int saturating_sum(int x, int y) {
+  const uint32_t u = (uint32_t)x + (uint32_t)y;
+  return (int)(u > 0x7FFFFFFFu ? 0x7FFFFFFFu : u);
+}
+// Inclusive prefix sum over the 64 lanes of non-negative values by data-parallel moves: inside each row of 16 lanes, then
+// the last lane of rows 0 and 2 added to rows 1 and 3, then lane 31 to rows 2 and 3.  Lanes without a source add zero.
+template <bool SATURATE, int CTRL, int ROWS>
+MSLK_AMD_DEVINL int prefix_step(int v) {
+  const int o = __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
+  return SATURATE ? saturating_sum(v, o) : v + o;
+}
+template <bool SATURATE>
+MSLK_AMD_DEVINL int wave_prefix_sum(int v) {
+  v = prefix_step<SATURATE, 0x111, 0xF>(v);   // one lane to the right
+  v = prefix_step<SATURATE, 0x112, 0xF>(v);   // two
+  v = prefix_step<SATURATE, 0x114, 0xF>(v);   // four
+  v = prefix_step<SATURATE, 0x118, 0xF>(v);   // eight
+  v = prefix_step<SATURATE, 0x142, 0xA>(v);   // lane 15 of a row to the next row
+  return prefix_step<SATURATE, 0x143, 0xC>(v);   // lane 31 to the upper half
+}
+
 // Workgroup -> (group, tile of the group) where the groups are K slices: every group has the same `per` output tiles, but a
 // tile costs what its slice is long.  The list runs over the groups in order of falling slice length (the longest tiles
 // start first, the short ones fill the end), and is dealt to the XCDs in runs of per / 8 tiles, so that every XCD gets the
@@ -109,103 +132,97 @@ MSLK_AMD_DEVINL bool find_group(const DeviceGroups& p, int t, GroupSpan& sp) {
       return true;
     }
   } else {
-    // The G extents are read 64 at a time, one per lane, and turned into tile ranges by a wave-level
-    // prefix sum, so the lookup costs one memory round trip instead of G dependent ones.  The total tile count is formed
-    // first: XCD x (workgroup id mod 8) then takes a contiguous slice of the tile list, so that the row tiles of a group
-    // that share a weight panel run on one XCD and find it in its L2 (without the slices the device-extent layouts
-    // fetched 1.6 times what the host-extent kernel fetches for the same 16 experts).
+    // The G extents are read 64 at a time, one per lane, and turned into tile ranges by a wave-level prefix sum, so the
+    // lookup costs one memory round trip for up to 128 groups (the first two chunks are fetched together and stay in
+    // registers) instead of G dependent ones.  A workgroup holds its CU's whole LDS, so nothing else runs under the lookup:
+    // with more round trips for the groups beyond 64 and sums through LDS shuffles (a hundred cycles per step) 128 experts x
+    // 2048 x 768 took 65.5 us over 8192 rows and 120.0 over 32768 (now 56.3 and 114.8), 64 x 4096 x 1024 over 16384 128.4
+    // (120.1), 16 x 8192 x 5120 over 8192 324 (323).
+    // The total tile count is formed first: XCD x (workgroup id mod 8) then takes a contiguous slice of the tile list, so
+    // that the row tiles of a group that share a weight panel run on one XCD and find it in its L2 (without the slices the
+    // device-extent layouts fetched 1.6 times what the host-extent kernel fetches for the same 16 experts).
     const int fixed_tiles = LAYOUT == kGroupsOffsetsN ? tiles_m : tiles_n;
     const int blk = LAYOUT == kGroupsOffsetsN ? BN : BM;
     const int64_t total = LAYOUT == kGroupsOffsetsN ? p.N : p.M;
     const int lane = threadIdx.x & 63;
     // Every quantity fits 32 bits (the host checks the dimensions and the grid): sizes beyond the tensor mark the group bad.
-    struct Chunk { int start, len, tiles, incl; bool bad; };
+    struct Extent { int64_t size; int begin, end; };
+    struct Chunk { int start, len, tiles, incl; unsigned long long bad; };
+    auto fetch = [&](int base) {
+      Extent x{0, 0, 0};
+      const int gi = base + lane;
+      if (gi < p.G) {
+        if constexpr (LAYOUT == kGroupsSizesM) {
+          x.size = static_cast<const int64_t*>(p.layout)[gi];
+        } else {
+          x.begin = gi ? static_cast<const int32_t*>(p.layout)[gi - 1] : 0;
+          x.end = static_cast<const int32_t*>(p.layout)[gi];
+        }
+      }
+      return x;
+    };
     // `seen_bad` carries "an earlier group was inconsistent" from chunk to chunk: such a group and every group after it
     // own no tiles, so the tile count, the XCD slices and the lookup all stop at the first bad group and every tile
     // of the groups in front of it gets a workgroup (the grid is sized for consistent extents).
-    auto load_chunk = [&](int base, int& carry_len, bool& seen_bad) {
+    auto chunk_of = [&](const Extent& x, int base, int& carry_len, bool& seen_bad) {
       Chunk c;
-      const int gi = base + lane;
-      const bool in = gi < p.G;
-      c.start = 0;
-      c.len = 0;
-      c.bad = false;
+      const bool in = base + lane < p.G;
+      bool bad;
       if constexpr (LAYOUT == kGroupsSizesM) {
-        int64_t len64 = 0;
-        if (in) len64 = static_cast<const int64_t*>(p.layout)[gi];
-        c.bad = len64 < 0 || len64 > total;
-        c.len = c.bad ? 0 : (int)len64;
-        // running sum that saturates at 2^31 - 1 instead of wrapping (the terms are below 2^31, so one unsigned addition
-        // cannot wrap): sizes that add up to more than the tensor holds always end beyond it and mark their group bad
-        auto sat_add = [](int x, int y) {
-          const uint32_t u = (uint32_t)x + (uint32_t)y;
-          return (int)(u > 0x7FFFFFFFu ? 0x7FFFFFFFu : u);
-        };
-        int incl_len = c.len;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-          const int v = __shfl_up(incl_len, d, 64);
-          if (lane >= d) incl_len = sat_add(incl_len, v);
-        }
-        const int end = sat_add(carry_len, incl_len);
+        bad = x.size < 0 || x.size > total;
+        c.len = bad ? 0 : (int)x.size;
+        const int end = saturating_sum(carry_len, wave_prefix_sum<true>(c.len));
         c.start = end - c.len;
-        carry_len = sat_add(carry_len, __shfl(incl_len, 63, 64));
-        c.bad = c.bad || (in && (end > total || end == 0x7FFFFFFF));
+        carry_len = __builtin_amdgcn_readlane(end, 63);
+        bad = bad || (in && (end > total || end == 0x7FFFFFFF));
       } else {
-        const int32_t* off = static_cast<const int32_t*>(p.layout);
-        if (in) {
-          c.start = gi ? off[gi - 1] : 0;
-          const int64_t len64 = (int64_t)off[gi] - c.start;
-          c.bad = len64 < 0 || c.start < 0 || (int64_t)c.start + len64 > total;
-          c.len = c.bad ? 0 : (int)len64;
-        }
+        const int64_t len64 = (int64_t)x.end - x.begin;
+        bad = len64 < 0 || x.begin < 0 || x.end > total;
+        c.start = x.begin;
+        c.len = bad ? 0 : (int)len64;
       }
-      const unsigned long long bad_lanes = __ballot(c.bad);
-      const bool after_bad = seen_bad || (bad_lanes != 0 && lane >= __ffsll((long long)bad_lanes) - 1);
-      seen_bad = seen_bad || bad_lanes != 0;
+      c.bad = __ballot(bad);
+      const bool after_bad = seen_bad || (c.bad != 0 && lane >= __ffsll((long long)c.bad) - 1);
+      seen_bad = seen_bad || c.bad != 0;
       c.tiles = (in && !after_bad) ? ((c.len + blk - 1) / blk) * fixed_tiles : 0;
-      c.incl = c.tiles;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int v = __shfl_up(c.incl, d, 64);
-        if (lane >= d) c.incl += v;
-      }
+      c.incl = wave_prefix_sum<false>(c.tiles);
       return c;
     };
-    int64_t total_tiles = 0;
+    auto tiles_of = [&](const Chunk& c) { return __builtin_amdgcn_readlane(c.incl, 63); };
+    const Extent x0 = fetch(0), x1 = fetch(64);
     int carry_len = 0;
     bool seen_bad = false;
-    Chunk first = load_chunk(0, carry_len, seen_bad);
-    const bool first_bad = seen_bad;
-    total_tiles = __shfl(first.incl, 63, 64);
-    for (int base = 64; base < p.G && !seen_bad; base += 64) total_tiles += __shfl(load_chunk(base, carry_len, seen_bad).incl, 63, 64);
+    const Chunk c0 = chunk_of(x0, 0, carry_len, seen_bad);
+    const Chunk c1 = chunk_of(x1, 64, carry_len, seen_bad);   // no groups there: no tiles
+    const int carry_len2 = carry_len;
+    const bool seen_bad2 = seen_bad;
+    int64_t total_tiles = (int64_t)tiles_of(c0) + tiles_of(c1);
+    for (int base = 128; base < p.G && !seen_bad; base += 64) total_tiles += tiles_of(chunk_of(fetch(base), base, carry_len, seen_bad));
     const int64_t per_xcd = (total_tiles + kXcds - 1) / kXcds;
     const int64_t slot = t / kXcds;                       // `t` arrives as the workgroup id
     const int64_t tile = (int64_t)(t % kXcds) * per_xcd + slot;
     if (slot >= per_xcd || tile >= total_tiles) return false;
     int64_t carry_tiles = 0;
-    carry_len = 0;
-    seen_bad = first_bad;
-    for (int base = 0; base < p.G; base += 64) {
-      Chunk c = first;
-      if (base == 0) carry_len = __shfl(first.start + first.len, 63, 64);   // sizes: rows of the first 64 groups
-      else c = load_chunk(base, carry_len, seen_bad);
+    auto find_in = [&](const Chunk& c, int base) {
       const int64_t excl = carry_tiles + c.incl - c.tiles;
-      const bool hit = c.tiles > 0 && tile >= excl && tile < excl + c.tiles;
-      const unsigned long long hit_mask = __ballot(hit), bad_mask = __ballot(c.bad);
-      if (hit_mask != 0) {
-        const int src = __ffsll((long long)hit_mask) - 1;
-        if (bad_mask & ((1ull << src) - 1ull)) return false;   // a group before this one is inconsistent: touch nothing
-        // the results are the same in every lane: say so, so that the tile's addresses live in scalar registers
-        sp.gi = base + src;
-        sp.o0 = __builtin_amdgcn_readfirstlane(__shfl(c.start, src, 64));
-        sp.len = __builtin_amdgcn_readfirstlane(__shfl(c.len, src, 64));
-        sp.t = (int)(tile - uniform64(__shfl(excl, src, 64)));
-        return true;
+      const unsigned long long hit = __ballot(c.tiles > 0 && tile >= excl && tile < excl + c.tiles);
+      if (hit == 0) {
+        carry_tiles += tiles_of(c);
+        return false;
       }
-      if (bad_mask != 0) return false;
-      carry_tiles += __shfl(c.incl, 63, 64);
-    }
+      const int src = __ffsll((long long)hit) - 1;
+      // the results are the same in every lane: out of scalar registers, so that the tile's addresses live there
+      sp.gi = base + src;
+      sp.o0 = __builtin_amdgcn_readlane(c.start, src);
+      sp.len = __builtin_amdgcn_readlane(c.len, src);
+      sp.t = (int)(uniform64(tile - carry_tiles) - __builtin_amdgcn_readlane(c.incl - c.tiles, src));
+      return true;
+    };
+    if (find_in(c0, 0) || find_in(c1, 64)) return true;
+    carry_len = carry_len2;
+    seen_bad = seen_bad2;
+    for (int base = 128; base < p.G && !seen_bad; base += 64)
+      if (find_in(chunk_of(fetch(base), base, carry_len, seen_bad), base)) return true;
     return false;
   }
 }
