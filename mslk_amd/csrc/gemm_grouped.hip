@@ -53,8 +53,8 @@ __global__ __launch_bounds__(256) void grouped_tiled_kernel(GroupTable tab) {
 // Host-side schedule of a TensorList launch.  Workgroup ids go round the eight XCDs, and inside an XCD the hardware
 // hands the next workgroup to the first CU that is free -- so an XCD finishes when its share of the WORK is done, and
 // the launch when the slowest XCD is.  Equal tile COUNTS per XCD are not equal work: a tile of an expert with one row
-// tile fetches its whole weight block from HBM alone (measured about 67 us at K = 5120), a tile out of a panel of four
-// row tiles shares it (59 us), and a ragged tile with a quarter of the rows takes about three quarters of a full one.
+// tile fetches its whole weight block from HBM alone (measured about 67 us for 256 x 256 at K = 5120), a tile out of a
+// panel of four row tiles shares it (59 us), and a ragged tile with a quarter of the rows takes about three quarters of a full one.
 // The groups are therefore cut into panels of up to kGroupM row tiles (all column tiles of those rows: the unit inside
 // which operand tiles are shared through the L2), every panel gets a cost from that model, the panels are dealt to the
 // XCDs longest first onto the least loaded one -- every XCD gets dear and cheap panels alike; all the weight-bound ones
@@ -64,9 +64,8 @@ __global__ __launch_bounds__(256) void grouped_tiled_kernel(GroupTable tab) {
 // ordered column by column, so the two XCDs get column ranges of it.  A panel is just another group descriptor (same
 // weights, row range of the activations and of the output); when the panels would not fit the descriptor table, whole
 // groups are dealt.
-hipError_t launch_grouped_tiled(const GroupTable& in, hipStream_t s) {
-  if (in.total_tiles <= 0 || in.count <= 0) return hipSuccess;
-  constexpr int BM = 256, BN = 256;
+template <int BM, int BN>
+static hipError_t launch_grouped_shape(const GroupTable& in, hipStream_t s) {
   struct Chunk { int group, row0, rows, tiles; float cost, cheapest; };
   Chunk chunks[kMaxGroupsPerLaunch];
   auto tile_cost = [](int rows, int sharing) {   // relative time of one tile: rows valid, `sharing` row tiles use its weights
@@ -132,11 +131,11 @@ hipError_t launch_grouped_tiled(const GroupTable& in, hipStream_t s) {
   t.total_tiles = tiles;
   // XCD x works on tiles [xcd_begin[x], xcd_begin[x + 1]).  Two plans: the deal (whole panels per XCD), and the same list
   // cut into eight runs of equal cost, a cut falling wherever the running cost reaches the next eighth.  Each is priced as
-  // the slowest XCD's passes over its CUs (tiles / CUs of an XCD, rounded up) times the mean cost of its tiles; the deal
-  // keeps every XCD at whole panels -- multiples of the column count, which full passes are made of -- and wins whenever
+  // the slowest XCD's passes over its CUs (tiles / workgroups an XCD runs at once, rounded up) times the mean cost of its
+  // tiles; the deal keeps every XCD at whole panels -- multiples of the column count, which full passes are made of -- and wins whenever
   // there are panels enough (measured: cutting cfg4 evenly by cost costs 7 %, because the cuts leave partial passes);
   // the even cut wins when the deal leaves XCDs idle (one group of 1024 rows: 189 -> 47 us).
-  const int cus_per_xcd = device_compute_units() / kXcds;
+  const int wgs_per_xcd = device_compute_units() / kXcds * (TileShape<BM, BN>::LDS_BYTES <= 80 * 1024 ? 2 : 1);   // workgroups at once
   int plan_a[kXcds + 1], plan_b[kXcds + 1];
   plan_a[0] = plan_b[0] = 0;
   plan_a[kXcds] = plan_b[kXcds] = tiles;
@@ -168,7 +167,7 @@ hipError_t launch_grouped_tiled(const GroupTable& in, hipStream_t s) {
         const int to = t.g[k].tile_begin + c.tiles < hi ? t.g[k].tile_begin + c.tiles : hi;
         cost += (double)c.cost / c.tiles * (to - from);
       }
-      const int passes = (hi - lo + cus_per_xcd - 1) / cus_per_xcd;
+      const int passes = (hi - lo + wgs_per_xcd - 1) / wgs_per_xcd;
       const double time = cost / (hi - lo) * passes;
       if (time > worst) worst = time;
     }
@@ -179,8 +178,20 @@ hipError_t launch_grouped_tiled(const GroupTable& in, hipStream_t s) {
   int longest = 0;
   for (int i = 0; i < kXcds; ++i)
     if (t.xcd_begin[i + 1] - t.xcd_begin[i] > longest) longest = t.xcd_begin[i + 1] - t.xcd_begin[i];
-  grouped_tiled_kernel<256, 256><<<longest * kXcds, 256, 0, s>>>(t);
+  grouped_tiled_kernel<BM, BN><<<longest * kXcds, 256, 0, s>>>(t);
   return hipGetLastError();
+}
+
+hipError_t launch_grouped_tiled(const GroupTable& in, hipStream_t s) {
+  if (in.total_tiles <= 0 || in.count <= 0) return hipSuccess;
+  int64_t rows = 0, groups = 0, tiles128 = 0;
+  for (int g = 0; g < in.count; ++g) {
+    rows += in.g[g].M;
+    groups += in.g[g].M > 0;
+    tiles128 += (int64_t)((in.g[g].M + 127) / 128) * ((in.g[g].N + 127) / 128);
+  }
+  // (as lists 32 experts x 4096 x 1024 with 64 rows each: 35.7 against 42.7 us, 16 x 4096 x 5120 91.2 / 102.8)
+  return small_row_groups(rows, groups, tiles128) ? launch_grouped_shape<128, 128>(in, s) : launch_grouped_shape<256, 256>(in, s);
 }
 
 // Whether every operand row of the problem can be fetched by the 16-byte DMA path.

@@ -335,13 +335,31 @@ hipError_t launch_device_shape(const DeviceGroups& p, hipStream_t s) {
   return hipGetLastError();
 }
 
+// 128 x 128 or 256 x 256 tiles for groups of rows (sizes known on the host or not).  Two 128 x 128 workgroups share a CU, so
+// one hides the other's first round trip and its epilogue; a 256 x 256 tile reads half as many operand bytes per product, and
+// a ragged one costs what its rows cost.  The small tiles win where they all run at once (8 experts x 1536 x 2048 over 4096
+// rows, 432 tiles: 19.8 against 27.5 us; 1 x 8192 x 5120 over 1024, 512 tiles: 47.0 / 54.4; but 2 x 4096 x 4096 over 2048, 544
+// tiles: 52.4 / 43.1; 8 x 4096 x 2048 over 2048, 640 tiles: 37.9 / 27.0) and up to 128 rows per group, where the weight
+// stream is the bound and half the rows of a 256-row tile are padding (64 x 2048 x 2048, by rows per group: 64 60.2 / 75.7,
+// 128 78.6 / 78.4, 192 98.8 / 87.4, 256 110.5 / 104.7, 320 129.9 / 116.1; 16 x 4096 x 5120: 64 93.6 / 106.3, 128 107.4 /
+// 109.4, 192 116.9 / 111.2, 320 156.2 / 124.8).  256 x 128 tiles were slower than either, 128 x 256 ones 5 % faster than
+// 128 x 128 for few rows and K >= 4096 and slower otherwise.
+inline bool small_row_groups(int64_t rows, int64_t groups, int64_t tiles128) {
+  return rows <= 128 * groups || tiles128 <= 2 * device_compute_units();
+}
+
 template <int LAYOUT, int BIAS>
 hipError_t launch_device_layout(const DeviceGroups& p, hipStream_t s) {
-  // Tile shape from the average group: 256 x 256 once such tiles give every CU work.
   const int64_t G = p.G > 0 ? p.G : 1;
-  int64_t Mg = p.M, Ng = p.N;
-  if (LAYOUT == kGroupsSizesM || LAYOUT == kGroupsOffsetsM) Mg = (p.M + G - 1) / G;
-  if (LAYOUT == kGroupsOffsetsN) Ng = (p.N + G - 1) / G;
+  if constexpr (LAYOUT == kGroupsSizesM || LAYOUT == kGroupsOffsetsM) {
+    // The sizes are not known here: a group ends in half a tile on average.  Operands that take the scalar tile want many
+    // workgroups (8 experts x 4096 x 1000 over 4096 rows: 32.0 ms, with 256 x 256 tiles 67.7).
+    const int64_t M = p.M, N = p.N, tiles_m = G == 1 ? (M + 127) / 128 : (M + 64 * G) / 128, tiles128 = tiles_m * ((N + 127) / 128);
+    if (p.unaligned || small_row_groups(M, G, tiles128)) return launch_device_shape<LAYOUT, 128, 128, BIAS>(p, s);
+    return launch_device_shape<LAYOUT, 256, 256, BIAS>(p, s);
+  }
+  // Tile shape from the average group: 256 x 256 once such tiles give every CU work.
+  const int64_t Mg = p.M, Ng = LAYOUT == kGroupsOffsetsN ? (p.N + G - 1) / G : p.N;
   const int64_t big = G * ((Mg + 255) / 256) * ((Ng + 255) / 256);
   const int64_t pad = ((Mg + 255) / 256 * 256) * ((Ng + 255) / 256 * 256);
   const bool use_big = big >= 192 && pad * 4 <= Mg * Ng * 5;   // at most 25 % padding
