@@ -18,19 +18,23 @@ from .gemm import (f8f8bf16_rowwise, f8f8bf16_rowwise_out, quantize_f8f8bf16_row
                    f8f8bf16_rowwise_batched)
 
 
-def _register_missing(error: RuntimeError) -> None:
-    """The build is missing: every operator with a native kernel raises `error` when it is used on a GPU."""
+def _native_schemas():
+    """Name -> schema of every operator with a native GPU kernel."""
+    schemas = {**quantize.SCHEMAS, **{f"mslk::{n}": n + schema for n, (schema, _) in moe._OPS.items()},
+               **{f"mslk::{n}": n + schema for n, schema in gemm._SCHEMAS.items() if n not in gemm._PYTHON_IMPLS}}
+    return schemas
+
+
+def _register_missing(name: str, error: RuntimeError) -> None:
+    """The build is missing: the operator raises `error` when it is used on a GPU."""
     def fail(*_args, **_kwargs):
         raise error
 
-    for library, names in ((quantize._triton_library, ["quantize_fp8_row"]),
-                           (quantize._library, ["quantize_fp8_per_row", "dequantize_fp8_row"] + list(moe._OPS)
-                            + [n for n in gemm._SCHEMAS if n not in gemm._PYTHON_IMPLS])):
-        for name in names:
-            library.impl(name, fail, "CUDA", allow_override=True)
+    namespace, operator = name.split("::")
+    {"triton": quantize._triton_library, "mslk": quantize._library}[namespace].impl(operator, fail, "CUDA", allow_override=True)
 
 
-_lib.load_torch_ops(_register_missing)   # every schema is defined by now
+_lib.load_torch_ops(_native_schemas(), _register_missing)   # every schema is defined by now
 
 __all__ = ["quantize_fp8_row", "quantize_fp8_per_row", "dequantize_fp8_row", "silu_mul_quant", "gather_scale_quant_dense_tokens", "f8f8bf16_rowwise", "f8f8bf16_rowwise_out", "quantize_f8f8bf16_rowwise", "f8f8f16_rowwise", "f8f8bf16_rowwise_preshuffle", "f8f8f16_rowwise_preshuffle", "preshuffle_b_mfma", "ck_preshuffle",
            "f8f8bf16_rowwise_grouped", "f8f8bf16_rowwise_grouped_cat", "f8f8bf16_rowwise_grouped_stacked",

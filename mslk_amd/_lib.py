@@ -94,17 +94,48 @@ def check(rc: int) -> None:
         raise RuntimeError(lib().mslk_amd_last_error().decode())
 
 
-def load_torch_ops(register_missing) -> None:
-    """Loads the native operator kernels, which registers them with the dispatcher, and binds them to the C ABI.  When the
-    build is missing, `register_missing(error)` is called instead, to make the operators raise `error` when they are used."""
+def _types(schema) -> tuple:
+    """The types of a schema's arguments and results: what a kernel has to agree with (names and defaults do not matter)."""
+    def text(values):
+        return tuple(str(v.type).replace("SymInt", "int") for v in values)
+    return text(schema.arguments), text(schema.returns)
+
+
+def fits(name: str, schema: str) -> bool:
+    """Whether the operator `name` ("namespace::operator"), which another library may have defined, takes a kernel of `schema`."""
+    import torch
+    namespace, operator = name.split("::")
+    overload = getattr(getattr(getattr(torch.ops, namespace), operator), "default", None)
+    return overload is not None and _types(overload._schema) == _types(torch._C.parse_schema(schema))
+
+
+def load_torch_ops(schemas, register_missing) -> None:
+    """Makes the native functions the GPU kernels of the operators of `schemas` (name -> schema, all of them defined by now, by
+    this package or by a library loaded before it).  An operator that was defined with other types keeps the kernel it has.
+    When the build is missing, `register_missing(name, error)` is called for each instead, to make the operators raise `error`
+    when they are used."""
+    import warnings
+    names = []
+    for name, schema in schemas.items():
+        if fits(name, schema):
+            names.append(name)
+        else:
+            warnings.warn(f"mslk_amd: {name} is already defined with other argument or result types than {schema}; its GPU "
+                          "kernel stays as it is")
     for path in (LIB_PATH, TORCH_OPS_PATH):
         if not os.path.exists(path):
-            register_missing(_missing(path))
+            for name in names:
+                register_missing(name, _missing(path))
             return
     import torch
     torch.ops.load_library(TORCH_OPS_PATH)
-    bind = ctypes.CDLL(TORCH_OPS_PATH).mslk_amd_torch_bind
-    bind.restype, bind.argtypes = c_char_p, [c_char_p]
-    error = bind(os.fsencode(LIB_PATH))
+    ops = ctypes.CDLL(TORCH_OPS_PATH)
+    ops.mslk_amd_torch_bind.restype, ops.mslk_amd_torch_bind.argtypes = c_char_p, [c_char_p]
+    ops.mslk_amd_torch_register.restype, ops.mslk_amd_torch_register.argtypes = c_char_p, [c_char_p, c_char_p]
+    error = ops.mslk_amd_torch_bind(os.fsencode(LIB_PATH))
     if error is not None:
         raise RuntimeError(f"mslk_amd: cannot bind {LIB_PATH}: {error.decode()}")
+    for name in names:
+        error = ops.mslk_amd_torch_register(*(part.encode() for part in name.split("::")))
+        if error is not None:
+            raise RuntimeError(f"mslk_amd: cannot register the kernel of {name}: {error.decode()}")

@@ -17,7 +17,9 @@
 #include <dlfcn.h>
 #include <torch/library.h>
 
+#include <cstring>
 #include <optional>
+#include <string>
 #include <tuple>
 #include <vector>
 
@@ -546,24 +548,40 @@ Tensor grouped_mm_op(const Tensor& XQ, const Tensor& WQ, const Tensor& x_scale, 
   return output;
 }
 
-TORCH_LIBRARY_IMPL(triton, CUDA, m) { m.impl("quantize_fp8_row", quantize_fp8_row); }
-
-TORCH_LIBRARY_IMPL(mslk, CUDA, m) {
-  m.impl("quantize_fp8_per_row", quantize_fp8_per_row);
-  m.impl("dequantize_fp8_row", dequantize_fp8_row);
-  m.impl("silu_mul_quant", silu_mul_quant);
-  m.impl("gather_scale_quant_dense_tokens", gather_scale_quant_dense_tokens);
-  m.impl("f8f8bf16_rowwise", rowwise_op<false, false>);
-  m.impl("f8f8f16_rowwise", rowwise_op<true, false>);
-  m.impl("f8f8bf16_rowwise_preshuffle", rowwise_op<false, true>);
-  m.impl("f8f8f16_rowwise_preshuffle", rowwise_op<true, true>);
-  m.impl("f8f8bf16_rowwise_out", rowwise_out_op);
-  m.impl("quantize_f8f8bf16_rowwise", quantize_rowwise);
-  m.impl("f8f8bf16_rowwise_grouped", grouped_op);
-  m.impl("f8f8bf16_rowwise_grouped_cat", grouped_cat_op);
-  m.impl("f8f8bf16_rowwise_grouped_stacked", grouped_stacked_op);
-  m.impl("f8f8bf16_rowwise_grouped_mm", grouped_mm_op);
+// Registered as boxed functions, one operator at a time and when the package asks for it.  A library loaded earlier may have
+// defined an operator (the package then only replaces its GPU kernel): a kernel registered with its C++ type is refused where
+// that library's own kernels take, say, Tensor by value instead of by reference, and an exception in a static initializer
+// ends the process.  Calls from Python are boxed anyway.
+template <auto FN>
+void boxed(const c10::OperatorHandle& op, c10::DispatchKeySet keys, torch::jit::Stack* stack) {
+  static const c10::KernelFunction kernel = c10::KernelFunction::makeFromUnboxedFunction(TORCH_FN(FN));
+  kernel.callBoxed(op, keys, stack);
 }
+struct Kernel {
+  const char *ns, *name;
+  torch::CppFunction (*make)();
+};
+template <auto FN>
+constexpr Kernel kernel(const char* ns, const char* name) {
+  return {ns, name, [] { return torch::CppFunction::makeFromBoxedFunction<&boxed<FN>>(); }};
+}
+const Kernel kernels[] = {
+    kernel<quantize_fp8_row>("triton", "quantize_fp8_row"),
+    kernel<quantize_fp8_per_row>("mslk", "quantize_fp8_per_row"),
+    kernel<dequantize_fp8_row>("mslk", "dequantize_fp8_row"),
+    kernel<silu_mul_quant>("mslk", "silu_mul_quant"),
+    kernel<gather_scale_quant_dense_tokens>("mslk", "gather_scale_quant_dense_tokens"),
+    kernel<rowwise_op<false, false>>("mslk", "f8f8bf16_rowwise"),
+    kernel<rowwise_op<true, false>>("mslk", "f8f8f16_rowwise"),
+    kernel<rowwise_op<false, true>>("mslk", "f8f8bf16_rowwise_preshuffle"),
+    kernel<rowwise_op<true, true>>("mslk", "f8f8f16_rowwise_preshuffle"),
+    kernel<rowwise_out_op>("mslk", "f8f8bf16_rowwise_out"),
+    kernel<quantize_rowwise>("mslk", "quantize_f8f8bf16_rowwise"),
+    kernel<grouped_op>("mslk", "f8f8bf16_rowwise_grouped"),
+    kernel<grouped_cat_op>("mslk", "f8f8bf16_rowwise_grouped_cat"),
+    kernel<grouped_stacked_op>("mslk", "f8f8bf16_rowwise_grouped_stacked"),
+    kernel<grouped_mm_op>("mslk", "f8f8bf16_rowwise_grouped_mm"),
+};
 
 // What the Python functions call directly: the checks in front of a launch, for tensors on any device.
 TORCH_LIBRARY_FRAGMENT(mslk_amd, m) {
@@ -574,14 +592,36 @@ TORCH_LIBRARY_FRAGMENT(mslk_amd, m) {
 
 }  // namespace
 
-// Binds the entry points of the library at `path`; returns an error message or null.
+// Binds the entry points of the library at `path`, all of them or none; returns an error message or null.
 extern "C" const char* mslk_amd_torch_bind(const char* path) {
   void* lib = dlopen(path, RTLD_NOW | RTLD_LOCAL);
   if (lib == nullptr) return dlerror();
+  Api bound;
 #define X(name)                                                                              \
-  api.name = reinterpret_cast<decltype(api.name)>(dlsym(lib, #name));                          \
-  if (api.name == nullptr) return "the library does not export " #name;
+  bound.name = reinterpret_cast<decltype(bound.name)>(dlsym(lib, #name));                      \
+  if (bound.name == nullptr) return "the library does not export " #name;
   MSLK_AMD_ENTRY_POINTS(X)
 #undef X
+  api = bound;
   return nullptr;
+}
+
+// Makes the native function the GPU kernel of operator `name` in namespace `ns`, whose schema has to have the types of the
+// one the package defines; after mslk_amd_torch_bind().  Returns an error message or null.
+extern "C" const char* mslk_amd_torch_register(const char* ns, const char* name) {
+  static std::string error;   // calls come from the import of the package, one at a time
+  if (api.mslk_amd_last_error == nullptr) return "mslk_amd_torch_bind() comes first";
+  for (const Kernel& k : kernels) {
+    if (std::strcmp(k.ns, ns) != 0 || std::strcmp(k.name, name) != 0) continue;
+    try {
+      // kept until the process ends: the registration goes with the object
+      auto* library = new torch::Library(torch::Library::IMPL, ns, c10::DispatchKey::CUDA, __FILE__, __LINE__);
+      library->impl(name, k.make());
+      return nullptr;
+    } catch (const std::exception& e) {
+      error = e.what();
+      return error.c_str();
+    }
+  }
+  return "no native kernel of this name";
 }

@@ -39,25 +39,28 @@ def _quantize_fp8_per_row_fake(input, bs=None, scale_ub=None, output_dtype=None,
 # path is known by (the legacy FBGEMM operator's signature), always with the torch branch's arithmetic.
 _library = torch.library.Library("mslk", "FRAGMENT")
 _triton_library = torch.library.Library("triton", "FRAGMENT")
-_QUANTIZE_ROW_SCHEMA = ("quantize_fp8_row(Tensor a, Tensor? scale_ub=None, Tensor? zero_start_index_M=None, "
-                        "bool use_triton=True, Device? output_device=None, SymInt? align_rows_to=None, "
-                        "float? eps_opt=0.001953125) -> (Tensor, Tensor)")
-_QUANTIZE_PER_ROW_SCHEMA = ("quantize_fp8_per_row(Tensor input, Tensor? bs=None, Tensor? scale_ub=None, "
-                            "ScalarType? output_dtype=None, bool stochastic_rounding=False) -> (Tensor, Tensor)")
+SCHEMAS = {
+    "triton::quantize_fp8_row": "quantize_fp8_row(Tensor a, Tensor? scale_ub=None, Tensor? zero_start_index_M=None, "
+                                "bool use_triton=True, Device? output_device=None, SymInt? align_rows_to=None, "
+                                "float? eps_opt=0.001953125) -> (Tensor, Tensor)",
+    "mslk::quantize_fp8_per_row": "quantize_fp8_per_row(Tensor input, Tensor? bs=None, Tensor? scale_ub=None, "
+                                  "ScalarType? output_dtype=None, bool stochastic_rounding=False) -> (Tensor, Tensor)",
+    "mslk::dequantize_fp8_row": "dequantize_fp8_row(Tensor xq, Tensor x_scale) -> Tensor",
+}
 
 
 def _register_quantize() -> None:
-    if not hasattr(torch.ops.triton, "quantize_fp8_row"):
-        _triton_library.define(_QUANTIZE_ROW_SCHEMA)
-        torch.library.register_fake("triton::quantize_fp8_row", _quantize_fp8_row_fake, lib=_triton_library)
-    if not hasattr(torch.ops.mslk, "quantize_fp8_per_row"):
-        _library.define(_QUANTIZE_PER_ROW_SCHEMA)
-        torch.library.register_fake("mslk::quantize_fp8_per_row", _quantize_fp8_per_row_fake, lib=_library)
-    if not hasattr(torch.ops.mslk, "dequantize_fp8_row"):
-        _library.define("dequantize_fp8_row(Tensor xq, Tensor x_scale) -> Tensor")
-        torch.library.register_fake(
-            "mslk::dequantize_fp8_row",
-            lambda xq, x_scale: torch.empty(xq.shape, dtype=torch.bfloat16, device=xq.device), lib=_library)
+    fakes = {
+        "quantize_fp8_row": _quantize_fp8_row_fake,
+        "quantize_fp8_per_row": _quantize_fp8_per_row_fake,
+        "dequantize_fp8_row": lambda xq, x_scale: torch.empty(xq.shape, dtype=torch.bfloat16, device=xq.device),
+    }
+    for name, schema in SCHEMAS.items():
+        namespace, operator = name.split("::")
+        library = _triton_library if namespace == "triton" else _library
+        if not hasattr(getattr(torch.ops, namespace), operator):
+            library.define(schema)
+            torch.library.register_fake(name, fakes[operator], lib=library)
 
 
 _register_quantize()
