@@ -192,6 +192,21 @@ __global__ __launch_bounds__(TEAM > 256 ? TEAM : 256) void quantize_rows_vec_ker
     if constexpr (TEAM < kWave) return ok && v < nvec ? sub * stride + v * vec_bytes : kBeyondBuffer;
     return v * vec_bytes;
   };
+  auto pad = [&] {   // zero padding columns [K, out_stride)
+    if (valid)
+      for (int64_t k = K + lane; k < out_stride; k += TEAM) out[row * out_stride + k] = 0;
+  };
+  // A wavefront without a live row (where rows are as wide as a workgroup, the whole workgroup): zero codes, whatever scale_ub
+  // makes of the scale (0 / 0 is no zero), and nothing read or reduced.
+  if (__ballot(live) == 0) {
+    float inv, sc;
+    scales_from_amax<DTYPE, TRITON>(0.f, scale_ub, jag.triton_eps, inv, sc);
+    if (lane == 0 && valid) scale[row] = sc;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) buffer_store8_through(dst, at(i, valid, (uint32_t)out_stride, 8), v2u{0, 0});
+    pad();
+    return;
+  }
   Vec8<DTYPE> cache[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) cache[i] = load_vec8<DTYPE>(src, at(i, live, (uint32_t)in_stride * ELEM_BYTES, 8 * ELEM_BYTES));
@@ -210,12 +225,13 @@ __global__ __launch_bounds__(TEAM > 256 ? TEAM : 256) void quantize_rows_vec_ker
       buffer_store8_through(dst, at(i, valid, (uint32_t)out_stride, 8), quantize_vec8<DTYPE, TRITON, kModePlain>(cache[i], inv, rcp));
   } else {
 #pragma unroll
-    for (int i = 0; i < NV; ++i)
-      buffer_store8_through(dst, at(i, valid, (uint32_t)out_stride, 8), quantize_vec8<DTYPE, TRITON, kModeGeneral>(cache[i], inv, rcp));
+    for (int i = 0; i < NV; ++i) {
+      v2u q = quantize_vec8<DTYPE, TRITON, kModeGeneral>(cache[i], inv, rcp);
+      if (TEAM < kWave && !live) q = v2u{0, 0};   // a dead row beside live ones of the wavefront
+      buffer_store8_through(dst, at(i, valid, (uint32_t)out_stride, 8), q);
+    }
   }
-  // zero padding columns [K, out_stride)
-  if (valid)
-    for (int64_t k = K + lane; k < out_stride; k += TEAM) out[row * out_stride + k] = 0;
+  pad();
 }
 
 // Vector path for rows beyond the registers: one workgroup per row, read twice (the second read hits the caches).
@@ -247,8 +263,8 @@ __global__ __launch_bounds__(256) void quantize_rows_long_kernel(
       store8_write_through(out_row + (int64_t)idx * 8, v2i{(int)q.x, (int)q.y});
     }
   }
-  // padding columns, and all of a dead row
-  for (int64_t k = (int64_t)nvec * 8 + threadIdx.x; k < out_stride; k += 256) out_row[k] = 0;
+  // padding columns, and all of a dead row (out_stride and the row's start are multiples of 8)
+  for (int64_t k = (int64_t)nvec * 8 + threadIdx.x * 8; k < out_stride; k += 256 * 8) store8_write_through(out_row + k, v2i{0, 0});
 }
 
 // Generic path: any K, any alignment; one workgroup per row, two passes.  Full groups of eight elements move as 16- / 32-byte

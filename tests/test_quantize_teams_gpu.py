@@ -63,6 +63,21 @@ def test_dead_rows_and_padding_columns(groups, per_group, K):
     assert torch.equal(s.cpu(), rs)
 
 
+@pytest.mark.parametrize("groups,per_group,K", [(700, 3, 64), (400, 6, 264), (300, 7, 1024), (3, 7, 4104), (3, 7, 65544), (5, 4, 100)])
+@pytest.mark.parametrize("triton", [True, False])
+def test_dead_rows_are_zero_codes_whatever_scale_ub_is(groups, per_group, K, triton):
+    """A bound of zero or below makes the scale zero or negative: 0 / 0 and 0 times a negative factor are no zero codes."""
+    g = torch.Generator().manual_seed(K)
+    x = torch.randn(groups, per_group, K, generator=g).bfloat16().to(DEV)
+    live = torch.randint(0, per_group + 1, (groups,), generator=g)
+    live[0] = 0
+    dead = torch.arange(per_group)[None, :] >= live[:, None]
+    for bound in (0.0, -1.0):
+        q, _ = mslk_amd.quantize_fp8_row(x, torch.tensor([bound], device=DEV), live.to(DEV), triton, None, 128)
+        q = q.cpu().view(torch.uint8)
+        assert not q[dead].any() and not q[..., K:].any(), (bound, K)
+
+
 @pytest.mark.parametrize("rows,K", [(1, 8), (300, 8), (257, 24), (1000, 576), (3, 65544), (129, 1000), (70001, 16)])
 def test_dequantized_rows_take_their_own_scale(rows, K):
     """The row of a chunk comes from a multiply and a shift: chunk counts per row of one, a power of two and neither."""
