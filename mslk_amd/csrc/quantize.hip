@@ -410,8 +410,9 @@ hipError_t launch_quantize_t(const void* x, int64_t rows, int64_t K, int64_t in_
   // lanes per row: 4 15.3, 8 10.8, 16 11.4, 32 16.2 us; 32768 x 1024: 64 x 2 vectors 16.8, 256 29.9; 8192 x 2048: 64 x 4
   // 9.9, 256 10.8.  Longer rows take a workgroup: 8192 x 4096: 256 x 2 16.7, 64 x 8 17.7, 512 19.4; 8192 x 8192: 256 x 4
   // 30.5, 512 x 2 30.6, 1024 39.9; 4096 x 16384: 512 x 4 31.1, 256 x 8 31.5, 1024 x 2 33.0.
-  // (The bound on the strides keeps the byte offsets of a wavefront's up to eight rows below 2^31.)
-  if (rows >= 2048 && nvec <= 256 && in_stride * ELEM_BYTES < (1 << 26) && out_stride < (1 << 26)) {
+  // (The bounds on the strides keep the byte offsets of a wavefront's up to eight rows between 0 and 2^31; a C caller may walk
+  // the input backwards.)
+  if (rows >= 2048 && nvec <= 256 && in_stride >= 0 && in_stride * ELEM_BYTES < (1 << 26) && out_stride < (1 << 26)) {
     if (nvec <= 8) return team(Int<8>{}, Int<1>{});
     if (nvec <= 16) return team(Int<8>{}, Int<2>{});
     if (nvec <= 32) return team(Int<16>{}, Int<2>{});

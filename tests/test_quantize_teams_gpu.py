@@ -49,6 +49,18 @@ def test_row_lengths_around_every_step_of_the_dispatch(rows, Ks, dtype):
             _check(got, want, f"{rows} x {K} {dtype} triton={triton}")
 
 
+@pytest.mark.parametrize("rows,K", [(2051, 64), (2051, 520), (2051, 1024), (2051, 2048), (300, 520), (5, 65544)])
+def test_rows_in_reverse_order_through_the_c_abi(rows, K):
+    """A negative row stride, from the last row on: several rows of a wavefront, a wavefront or a workgroup per row."""
+    from mslk_amd import _lib
+    x = torch.randn(rows, K, device=DEV).bfloat16()
+    q, s = torch.empty(rows, K, dtype=torch.uint8, device=DEV), torch.empty(rows, device=DEV)
+    _lib.check(_lib.lib().mslk_amd_quantize_fp8_row(x[-1].data_ptr(), 0, rows, K, -K, q.data_ptr(), K, s.data_ptr(), None,
+                                                    torch.cuda.current_stream().cuda_stream))
+    want, want_scale = mslk_amd.quantize_fp8_row(x.flip(0), use_triton=False)
+    assert torch.equal(q, want.view(torch.uint8)) and torch.equal(s, want_scale)
+
+
 @pytest.mark.parametrize("groups,per_group,K", [(500, 5, 120), (3, 7, 4104), (130, 16, 1000)])
 def test_dead_rows_and_padding_columns(groups, per_group, K):
     """Several rows of a wavefront with different live counts; columns up to the next multiple of 128 are zero."""
