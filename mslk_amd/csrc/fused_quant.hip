@@ -160,8 +160,8 @@ template <int OP, int DTYPE, int TEAM, int NV>
 __global__ __launch_bounds__(256) void fused_quant_vec_kernel(FusedQuantArgs p) {
   static_assert(TEAM == kWave || TEAM == 256, "a wavefront or a workgroup of four per row");
   __shared__ uint32_t smem[4];
-  const int64_t row = TEAM == kWave ? (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : (int64_t)blockIdx.x;
-  if (TEAM == kWave && row >= p.rows) return;    // uniform over the wavefront; this variant has no workgroup barrier
+  const int64_t row = TEAM == kWave ? row_block() * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : row_block();
+  if (row >= p.rows) return;                     // uniform over the team, the wavefront or (with the barrier) the workgroup
   const RowSource r = resolve_row<OP>(p, row);   // uniform over the team
   if (!r.live) return;
   const int lane = threadIdx.x % TEAM;
@@ -259,7 +259,7 @@ hipError_t launch_fused_t(const FusedQuantArgs& p, hipStream_t s) {
   }
   auto team = [&](auto t, auto n) {
     constexpr int TEAM = decltype(t)::value, NV = decltype(n)::value;
-    fused_quant_vec_kernel<OP, DTYPE, TEAM, NV><<<TEAM == kWave ? (rows + 3) / 4 : rows, 256, 0, s>>>(p);
+    fused_quant_vec_kernel<OP, DTYPE, TEAM, NV><<<row_grid(TEAM == kWave ? (p.rows + 3) / 4 : p.rows), 256, 0, s>>>(p);
     return hipGetLastError();
   };
   // As few vectors as hold the row: one beyond its end costs the arithmetic all the same (32768 x 768, gated product: 64 x 2

@@ -191,7 +191,8 @@ hipError_t launch_grouped_tiled(const GroupTable& in, hipStream_t s) {
     tiles128 += (int64_t)((in.g[g].M + 127) / 128) * ((in.g[g].N + 127) / 128);
   }
   // (as lists 32 experts x 4096 x 1024 with 64 rows each: 35.7 against 42.7 us, 16 x 4096 x 5120 91.2 / 102.8)
-  return small_row_groups(rows, groups, tiles128) ? launch_grouped_shape<128, 128>(in, s) : launch_grouped_shape<256, 256>(in, s);
+  const bool launchable = tiles128 <= kMaxWorkgroups / kXcds;   // (one XCD may be given most of them, and its share sets the grid)
+  return launchable && small_row_groups(rows, groups, tiles128) ? launch_grouped_shape<128, 128>(in, s) : launch_grouped_shape<256, 256>(in, s);
 }
 
 // Whether every operand row of the problem can be fetched by the 16-byte DMA path.

@@ -344,6 +344,8 @@ hipError_t launch_device_shape(const DeviceGroups& p, hipStream_t s) {
 // 128 78.6 / 78.4, 192 98.8 / 87.4, 256 110.5 / 104.7, 320 129.9 / 116.1; 16 x 4096 x 5120: 64 93.6 / 106.3, 128 107.4 /
 // 109.4, 192 116.9 / 111.2, 320 156.2 / 124.8).  256 x 128 tiles were slower than either, 128 x 256 ones 5 % faster than
 // 128 x 128 for few rows and K >= 4096 and slower otherwise.
+// (Twice or four times the workgroups: not beyond kMaxWorkgroups, past which HIP refuses a launch that the larger tiles fit.)
+constexpr int64_t kMaxWorkgroups = (int64_t(1) << 24) - 1;   // 256 lanes each, 2^32 work-items
 inline bool small_row_groups(int64_t rows, int64_t groups, int64_t tiles128) {
   return rows <= 128 * groups || tiles128 <= 2 * device_compute_units();
 }
@@ -355,7 +357,8 @@ hipError_t launch_device_layout(const DeviceGroups& p, hipStream_t s) {
     // The sizes are not known here: a group ends in half a tile on average.  Operands that take the scalar tile want many
     // workgroups (8 experts x 4096 x 1000 over 4096 rows: 32.0 ms, with 256 x 256 tiles 67.7).
     const int64_t M = p.M, N = p.N, tiles_m = G == 1 ? (M + 127) / 128 : (M + 64 * G) / 128, tiles128 = tiles_m * ((N + 127) / 128);
-    if (p.unaligned || small_row_groups(M, G, tiles128)) return launch_device_shape<LAYOUT, 128, 128, BIAS>(p, s);
+    const bool launchable = ((M + 127) / 128 + G) * ((N + 127) / 128) + kXcds <= kMaxWorkgroups;
+    if (launchable && (p.unaligned || small_row_groups(M, G, tiles128))) return launch_device_shape<LAYOUT, 128, 128, BIAS>(p, s);
     return launch_device_shape<LAYOUT, 256, 256, BIAS>(p, s);
   }
   // Tile shape from the average group: 256 x 256 once such tiles give every CU work.

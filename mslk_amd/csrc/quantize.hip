@@ -176,7 +176,7 @@ __global__ __launch_bounds__(TEAM > 256 ? TEAM : 256) void quantize_rows_vec_ker
   __shared__ uint32_t smem[BLOCK / kWave];
   const int lane = threadIdx.x % TEAM;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t row0 = (int64_t)blockIdx.x * TEAMS + (TEAM <= kWave ? wave * ROWS_W : 0);   // first row of the wavefront
+  const int64_t row0 = row_block() * TEAMS + (TEAM <= kWave ? wave * ROWS_W : 0);   // first row of the wavefront
   const int sub = TEAM < kWave ? (threadIdx.x & 63) / TEAM : 0;
   const int64_t row = row0 + sub;
   const bool valid = row < rows;
@@ -323,28 +323,31 @@ __global__ __launch_bounds__(256) void quantize_rows_generic_kernel(
 // A lane converts 8 consecutive codes of one row (K % 8 == 0), so that the 64 stores of a wavefront are 1 KiB without a gap
 // (16 codes per lane as two stores left every store instruction with half of each 32 bytes: 8192 x 8192 42.3 -> 32.8 us
 // = 6.1 TB/s, 131072 x 128 10.5 -> 9.6; two or four chunks per lane 33.7 and 34.2).  The row is the chunk's index divided by
-// the chunks of a row, by a multiply and a shift prepared on the host; WIDE divides in 64 bits, from 2^31 chunks on.
+// the chunks of a row, by a multiply and a shift prepared on the host.  WIDE, from 2^31 chunks on (16 GiB of codes): divides in
+// 64 bits and walks the tensor with a grid of bounded size, since one lane per chunk would reach the 2^32 work-items that
+// HIP refuses.
 struct RowDivider { uint32_t magic, shift; };   // n / d = umulhi(n, magic) >> shift for n < 2^31, d > 1; magic 0: d = 1
 template <bool WIDE>
 __global__ __launch_bounds__(256) void dequantize_rows_vec_kernel(const uint8_t* __restrict__ xq,
                                                                   const float* __restrict__ scale, int64_t chunks,
                                                                   int64_t chunks_per_row, RowDivider div, uint16_t* __restrict__ out) {
-  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (c >= chunks) return;
-  const v2u q = __builtin_nontemporal_load(reinterpret_cast<const v2u*>(xq) + c);
-  int64_t row;
-  if constexpr (WIDE) row = c / chunks_per_row;
-  else row = div.magic == 0 ? (uint32_t)c : __umulhi((uint32_t)c, div.magic) >> div.shift;
-  const float sc = scale[row];
-  v4u o;
+  for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < chunks; c += (int64_t)gridDim.x * 256) {
+    const v2u q = __builtin_nontemporal_load(reinterpret_cast<const v2u*>(xq) + c);
+    int64_t row;
+    if constexpr (WIDE) row = c / chunks_per_row;
+    else row = div.magic == 0 ? (uint32_t)c : __umulhi((uint32_t)c, div.magic) >> div.shift;
+    const float sc = scale[row];
+    v4u o;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)q[j], false);
-    const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)q[j], true);
-    o[2 * j] = pack_bf16x2(lo[0] * sc, lo[1] * sc);
-    o[2 * j + 1] = pack_bf16x2(hi[0] * sc, hi[1] * sc);
+    for (int j = 0; j < 2; ++j) {
+      const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)q[j], false);
+      const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)q[j], true);
+      o[2 * j] = pack_bf16x2(lo[0] * sc, lo[1] * sc);
+      o[2 * j + 1] = pack_bf16x2(hi[0] * sc, hi[1] * sc);
+    }
+    __builtin_nontemporal_store(o, reinterpret_cast<v4u*>(out) + c);
+    if constexpr (!WIDE) break;   // one chunk per lane
   }
-  __builtin_nontemporal_store(o, reinterpret_cast<v4u*>(out) + c);
 }
 
 // Any K, any alignment: a lane takes 8 consecutive codes of the flat tensor; when they lie in one row they move as an
@@ -401,7 +404,7 @@ hipError_t launch_quantize_t(const void* x, int64_t rows, int64_t K, int64_t in_
   const int64_t nvec = K / 8;
   auto team = [&](auto t, auto n) {
     constexpr int TEAM = decltype(t)::value, NV = decltype(n)::value, TEAMS = TEAM > 256 ? 1 : 256 / TEAM;
-    quantize_rows_vec_kernel<DTYPE, TEAM, NV, TRITON><<<(unsigned)((rows + TEAMS - 1) / TEAMS), TEAM > 256 ? TEAM : 256, 0, s>>>(
+    quantize_rows_vec_kernel<DTYPE, TEAM, NV, TRITON><<<row_grid((rows + TEAMS - 1) / TEAMS), TEAM > 256 ? TEAM : 256, 0, s>>>(
         x, rows, k, in_stride, out, out_stride, scale, scale_ub, jag);
     return hipGetLastError();
   };
@@ -462,7 +465,7 @@ hipError_t launch_dequantize_fp8_row(const void* xq, const float* scale, int64_t
     const int64_t chunks = total / 8, per_row = K / 8, blocks = (chunks + 255) / 256;
     RowDivider div{0, 0};
     if (chunks >= (int64_t(1) << 31)) {
-      dequantize_rows_vec_kernel<true><<<(unsigned)blocks, 256, 0, s>>>(in, scale, chunks, per_row, div, dst);
+      dequantize_rows_vec_kernel<true><<<1u << 16, 256, 0, s>>>(in, scale, chunks, per_row, div, dst);
     } else {
       if (per_row > 1) {   // 2^shift < d <= 2^(shift + 1): magic = ceil(2^(32 + shift) / d) < 2^32, exact for n < 2^31
         while ((int64_t(2) << div.shift) < per_row) ++div.shift;

@@ -19,6 +19,14 @@ template <int N> struct Int { static constexpr int value = N; };   // a template
 constexpr uint32_t kBeyondBuffer = 0x80000000u;   // an offset no descriptor made here reaches (sizes stay below 2^31)
 constexpr int kCacheNt = 2, kCacheSc1 = 16;       // cache policy bits of the buffer instructions: non-temporal, system scope
 
+// HIP refuses a launch of 2^32 or more work-items along one dimension: of workgroups of 1024 lanes that hold a row each, 2^22
+// rows.  From 2^21 workgroups on the grid goes on along y, the last line of it beyond the rows.
+constexpr int64_t kRowGridX = int64_t(1) << 21;
+inline dim3 row_grid(int64_t blocks) {
+  return blocks <= kRowGridX ? dim3((unsigned)blocks) : dim3((unsigned)kRowGridX, (unsigned)((blocks + kRowGridX - 1) / kRowGridX));
+}
+MSLK_AMD_DEVINL int64_t row_block() { return (int64_t)blockIdx.y * kRowGridX + blockIdx.x; }
+
 // `base` and `bytes` have to be the same in every lane of the wavefront.
 MSLK_AMD_DEVINL buffer_t make_buffer(const void* base, uint32_t bytes) {
   const uint64_t v = reinterpret_cast<uint64_t>(base);
