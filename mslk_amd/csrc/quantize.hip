@@ -176,7 +176,7 @@ __global__ __launch_bounds__(TEAM > 256 ? TEAM : 256) void quantize_rows_vec_ker
   __shared__ uint32_t smem[BLOCK / kWave];
   const int lane = threadIdx.x % TEAM;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t row0 = row_block() * TEAMS + (TEAM <= kWave ? wave * ROWS_W : 0);   // first row of the wavefront
+  const int64_t row0 = (TEAM <= kWave ? (int64_t)blockIdx.x : row_block()) * TEAMS + (TEAM <= kWave ? wave * ROWS_W : 0);   // first row of the wavefront
   const int sub = TEAM < kWave ? (threadIdx.x & 63) / TEAM : 0;
   const int64_t row = row0 + sub;
   const bool valid = row < rows;
@@ -207,6 +207,10 @@ __global__ __launch_bounds__(TEAM > 256 ? TEAM : 256) void quantize_rows_vec_ker
     pad();
     return;
   }
+  // Whether the wavefront owns any part of vector i: one wholly beyond the row reads as zero, but is not worth its arithmetic
+  // (1024 x 16392 with scale_ub, Triton arithmetic: 17.5 -> 12.9 us; 2047 x 64, three of four wavefronts without a vector:
+  // 4.3 -> 3.8).
+  auto used = [&](int i) { return (uint32_t)(i * TEAM + (TEAM > kWave ? wave * kWave : 0)) < nvec; };
   Vec8<DTYPE> cache[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) cache[i] = load_vec8<DTYPE>(src, at(i, live, (uint32_t)in_stride * ELEM_BYTES, 8 * ELEM_BYTES));
@@ -222,10 +226,11 @@ __global__ __launch_bounds__(TEAM > 256 ? TEAM : 256) void quantize_rows_vec_ker
   if (row_is_plain<DTYPE, TRITON>(amax, scale_ub, jag.triton_eps, inv, rcp)) {
 #pragma unroll
     for (int i = 0; i < NV; ++i)
-      buffer_store8_through(dst, at(i, valid, (uint32_t)out_stride, 8), quantize_vec8<DTYPE, TRITON, kModePlain>(cache[i], inv, rcp));
+      if (used(i)) buffer_store8_through(dst, at(i, valid, (uint32_t)out_stride, 8), quantize_vec8<DTYPE, TRITON, kModePlain>(cache[i], inv, rcp));
   } else {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
+      if (!used(i)) break;
       v2u q = quantize_vec8<DTYPE, TRITON, kModeGeneral>(cache[i], inv, rcp);
       if (TEAM < kWave && !live) q = v2u{0, 0};   // a dead row beside live ones of the wavefront
       buffer_store8_through(dst, at(i, valid, (uint32_t)out_stride, 8), q);
@@ -404,7 +409,7 @@ hipError_t launch_quantize_t(const void* x, int64_t rows, int64_t K, int64_t in_
   const int64_t nvec = K / 8;
   auto team = [&](auto t, auto n) {
     constexpr int TEAM = decltype(t)::value, NV = decltype(n)::value, TEAMS = TEAM > 256 ? 1 : 256 / TEAM;
-    quantize_rows_vec_kernel<DTYPE, TEAM, NV, TRITON><<<row_grid((rows + TEAMS - 1) / TEAMS), TEAM > 256 ? TEAM : 256, 0, s>>>(
+    quantize_rows_vec_kernel<DTYPE, TEAM, NV, TRITON><<<TEAM <= kWave ? dim3((unsigned)((rows + TEAMS - 1) / TEAMS)) : row_grid(rows), TEAM > 256 ? TEAM : 256, 0, s>>>(
         x, rows, k, in_stride, out, out_stride, scale, scale_ub, jag);
     return hipGetLastError();
   };
@@ -413,16 +418,20 @@ hipError_t launch_quantize_t(const void* x, int64_t rows, int64_t K, int64_t in_
   // lanes per row: 4 15.3, 8 10.8, 16 11.4, 32 16.2 us; 32768 x 1024: 64 x 2 vectors 16.8, 256 29.9; 8192 x 2048: 64 x 4
   // 9.9, 256 10.8.  Longer rows take a workgroup: 8192 x 4096: 256 x 2 16.7, 64 x 8 17.7, 512 19.4; 8192 x 8192: 256 x 4
   // 30.5, 512 x 2 30.6, 1024 39.9; 4096 x 16384: 512 x 4 31.1, 256 x 8 31.5, 1024 x 2 33.0.
+  // Between two steps a workgroup has too many lanes without a vector: 2048 < K <= 2560 takes a wavefront of five (8192 x 2560
+  // 9.8, as 256 x 2 11.6; 131072 x 2056 125 / 153, but 131072 x 2560 in torch arithmetic 167 / 157), and 64 < K <= 128 in fp32,
+  // whose vectors are twice as wide, 16 lanes of one (1048576 x 72: 77, as 8 x 2 93).
   // (The bounds on the strides keep the byte offsets of a wavefront's up to eight rows between 0 and 2^31; a C caller may walk
   // the input backwards.)
   if (rows >= 2048 && nvec <= 256 && in_stride >= 0 && in_stride * ELEM_BYTES < (1 << 26) && out_stride < (1 << 26)) {
     if (nvec <= 8) return team(Int<8>{}, Int<1>{});
-    if (nvec <= 16) return team(Int<8>{}, Int<2>{});
+    if (nvec <= 16) return DTYPE == 2 ? team(Int<16>{}, Int<1>{}) : team(Int<8>{}, Int<2>{});
     if (nvec <= 32) return team(Int<16>{}, Int<2>{});
     if (nvec <= 64) return team(Int<32>{}, Int<2>{});
     if (nvec <= 128) return team(Int<64>{}, Int<2>{});
     return team(Int<64>{}, Int<4>{});
   }
+  if (rows >= 2048 && nvec > 256 && nvec <= 320) return team(Int<64>{}, Int<5>{});
   if (nvec <= 256) return team(Int<256>{}, Int<1>{});
   if (nvec <= 512) return team(Int<256>{}, Int<2>{});
   if (nvec <= 1024) return team(Int<256>{}, Int<4>{});

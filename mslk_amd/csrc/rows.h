@@ -25,7 +25,7 @@ constexpr int64_t kRowGridX = int64_t(1) << 21;
 inline dim3 row_grid(int64_t blocks) {
   return blocks <= kRowGridX ? dim3((unsigned)blocks) : dim3((unsigned)kRowGridX, (unsigned)((blocks + kRowGridX - 1) / kRowGridX));
 }
-MSLK_AMD_DEVINL int64_t row_block() { return (int64_t)blockIdx.y * kRowGridX + blockIdx.x; }
+MSLK_AMD_DEVINL int64_t row_block() { return blockIdx.y * (uint32_t)kRowGridX + blockIdx.x; }
 
 // `base` and `bytes` have to be the same in every lane of the wavefront.
 MSLK_AMD_DEVINL buffer_t make_buffer(const void* base, uint32_t bytes) {

@@ -14,7 +14,7 @@ def _slices(rows, step=GRID_X // 4):
     return [slice(b, min(b + step, rows)) for b in range(0, rows, step)]
 
 
-@pytest.mark.parametrize("K,per_workgroup", [(2056, 1), (1032, 4)])
+@pytest.mark.parametrize("K,per_workgroup", [(2568, 1), (1032, 4)])
 def test_quantizer_with_more_workgroups_than_one_line_of_the_grid(K, per_workgroup):
     rows = GRID_X * per_workgroup + 3 * per_workgroup + (1 if per_workgroup > 1 else 0)
     x = torch.randn(rows, K, device=DEV, dtype=torch.bfloat16)

@@ -36,7 +36,7 @@ LARGE = [2056, 4096, 4104, 8192, 8200, 16384, 16392, 32768, 32776, 65536, 65544]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("rows,Ks", [(2051, SMALL), (2047, SMALL[:6]), (5, SMALL + LARGE)])
+@pytest.mark.parametrize("rows,Ks", [(2051, SMALL), (2051, [2056, 2560, 2568]), (2047, SMALL[:6]), (5, SMALL + LARGE)])
 def test_row_lengths_around_every_step_of_the_dispatch(rows, Ks, dtype):
     g = torch.Generator().manual_seed(rows)
     for K in Ks:
