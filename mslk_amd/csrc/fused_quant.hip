@@ -160,7 +160,7 @@ template <int OP, int DTYPE, int TEAM, int NV>
 __global__ __launch_bounds__(256) void fused_quant_vec_kernel(FusedQuantArgs p) {
   static_assert(TEAM == kWave || TEAM == 256, "a wavefront or a workgroup of four per row");
   __shared__ uint32_t smem[4];
-  const int64_t row = TEAM == kWave ? row_block() * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : row_block();
+  const int64_t row = TEAM == kWave ? (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : row_block();
   if (row >= p.rows) return;                     // uniform over the team, the wavefront or (with the barrier) the workgroup
   const RowSource r = resolve_row<OP>(p, row);   // uniform over the team
   if (!r.live) return;
@@ -173,10 +173,19 @@ __global__ __launch_bounds__(256) void fused_quant_vec_kernel(FusedQuantArgs p) 
     va[i] = buffer_load16(src_a, (uint32_t)(i * TEAM + lane) * 16);
     if constexpr (OP == kFusedSiluMul) vb[i] = buffer_load16(src_b, (uint32_t)(i * TEAM + lane) * 16);
   }
+  // Whether the wavefront owns any part of vector i.  One wholly beyond the row reads as zero and is not worth the arithmetic of
+  // the gated product (131072 x 2056: 286 -> 227 us, 2047 x 8200: 18.9 -> 14.0).  (The empty instruction keeps the loads where
+  // they are: the compiler would move each into the branch that uses it, one round trip each; and the wait is there for the
+  // loads of the branches not taken, before their registers are used again -- the compiler would put it between the stores.)
+  constexpr bool SKIP = OP == kFusedSiluMul && TEAM > kWave && NV > 1;
+  const int wave_first = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * kWave;
+  auto used = [&](int i) { return !SKIP || i * TEAM + wave_first < p.D >> 3; };
+  if constexpr (SKIP) asm volatile("" : : : "memory");
   float y[NV][8];
   uint32_t m = 0;
 #pragma unroll
-  for (int i = 0; i < NV; ++i) {   // vectors beyond the row read as zero and produce zero
+  for (int i = 0; i < NV; ++i) {   // lanes beyond the row read as zero and produce zero
+    if (!used(i)) break;
     produce8<OP, DTYPE>(va[i], vb[i], r.score, y[i]);
 #pragma unroll
     for (int e = 0; e < 8; ++e) m = max(m, __float_as_uint(y[i][e]) & 0x7FFFFFFFu);
@@ -192,13 +201,17 @@ __global__ __launch_bounds__(256) void fused_quant_vec_kernel(FusedQuantArgs p) 
           for (int e = 0; e < 8; ++e) m = max(m, __float_as_uint(y[i][e]) & 0x7FFFFFFFu);
     }
   }
+  if constexpr (SKIP) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
   m = team_max<TEAM>(m, smem);
   float s, inv;
   row_scales(m, p.scale_ub, s, inv);
   if (lane == 0) p.out_scale[row] = inv;
   const buffer_t dst = make_buffer(p.out + row * (int64_t)p.D, (uint32_t)p.D);
 #pragma unroll
-  for (int i = 0; i < NV; ++i) buffer_store8_through(dst, (uint32_t)(i * TEAM + lane) * 8, quantize8_saturating(y[i], s));
+  for (int i = 0; i < NV; ++i) {
+    if (!used(i)) break;
+    buffer_store8_through(dst, (uint32_t)(i * TEAM + lane) * 8, quantize8_saturating(y[i], s));
+  }
 }
 
 // Rows of any length: as above, produced twice.
@@ -259,16 +272,18 @@ hipError_t launch_fused_t(const FusedQuantArgs& p, hipStream_t s) {
   }
   auto team = [&](auto t, auto n) {
     constexpr int TEAM = decltype(t)::value, NV = decltype(n)::value;
-    fused_quant_vec_kernel<OP, DTYPE, TEAM, NV><<<row_grid(TEAM == kWave ? (p.rows + 3) / 4 : p.rows), 256, 0, s>>>(p);
+    fused_quant_vec_kernel<OP, DTYPE, TEAM, NV><<<TEAM == kWave ? dim3((rows + 3) / 4) : row_grid(p.rows), 256, 0, s>>>(p);
     return hipGetLastError();
   };
   // As few vectors as hold the row: one beyond its end costs the arithmetic all the same (32768 x 768, gated product: 64 x 2
-  // 22.2, 64 x 4 35.1 us).  In large numbers short rows take a wavefront each (gather, 32768 x 2048: 64 x 4 33.1, 256 45.1);
-  // the gated product, which computes more per byte, only up to two vectors (32768 x 2048: 256 49.6, 64 x 4 52.3).
-  if (p.rows >= 2048 && p.D <= (OP == kFusedSiluMul ? 1024 : 2048)) {
+  // 22.2, 64 x 4 35.1 us).  In large numbers short rows take a wavefront each (gather, 32768 x 2048: 64 x 4 33.1, 256 45.1).
+  // The gated product computes more per byte, so that lanes without a vector cost it more: a wavefront for up to two vectors
+  // whatever the number of rows (2047 x 512 fp16: 3.9, as 256 x 1 4.7), in large numbers for up to three (131072 x 1408
+  // fp16: 139, as 256 x 1 171), but not for four (32768 x 2048: 256 49.6, 64 x 4 52.3).
+  if (OP == kFusedSiluMul ? p.D <= 1024 || (p.rows >= 2048 && p.D <= 1536) : p.rows >= 2048 && p.D <= 2048) {
     if (p.D <= 512) return team(Int<64>{}, Int<1>{});
     if (p.D <= 1024) return team(Int<64>{}, Int<2>{});
-    return team(Int<64>{}, Int<(OP == kFusedSiluMul ? 2 : 4)>{});
+    return team(Int<64>{}, Int<(OP == kFusedSiluMul ? 3 : 4)>{});
   }
   if (p.D <= 2048) return team(Int<256>{}, Int<1>{});
   if (p.D <= 4096) return team(Int<256>{}, Int<2>{});

@@ -13,7 +13,7 @@ DEV = "cuda:0"
 STEPS = [8, 512, 520, 1024, 1032, 2048, 2056, 4096, 4104, 6144, 6152, 8192, 8200, 16384, 16392]
 
 
-@pytest.mark.parametrize("rows,Ds", [(7, STEPS), (2053, STEPS[:7])])
+@pytest.mark.parametrize("rows,Ds", [(7, STEPS), (2053, STEPS[:7]), (2053, [1536, 1544])])
 def test_gather_and_gated_product_around_every_step(rows, Ds):
     g = torch.Generator().manual_seed(rows)
     for D in Ds:
