@@ -5,6 +5,7 @@
 #pragma once
 #include "gemm_tile.h"
 #include "kernels.h"
+#include "rows.h"
 
 namespace mslk_amd {
 namespace {
@@ -70,39 +71,82 @@ MSLK_AMD_DEVINL int wave_prefix_sum(int v) {
 }
 
 // Workgroup -> (group, tile of the group) where the groups are K slices: every group has the same `per` output tiles, but a
-// tile costs what its slice is long.  The list runs over the groups in order of falling slice length (the longest tiles
-// start first, the short ones fill the end), and is dealt to the XCDs in runs of per / 8 tiles, so that every XCD gets the
-// same share of every group and a run still holds neighbouring tiles that share operand rows in the L2.  (An equal cut of
-// the list in group order gives one XCD the whole of the longest group: eight [4096 x 2048] gradients over 16384 rows,
-// group sizes falling like 1 / rank^1.1: 363 -> 156 us.)
-// Groups beyond the first 64 keep their order behind the sorted ones.
+// tile costs what its slice is long.  Two orders:
+// - in group order, every XCD an equal run of tiles: whole groups, whose operands only that XCD's L2 fetches;
+// - groups by falling length (the longest tiles start first, the short ones fill the end), dealt to the XCDs in runs of
+//   per / 8 tiles, so that every XCD gets the same share of every group and a run still holds neighbouring tiles.  Groups
+//   beyond the first 64 keep their order behind the sorted ones.
+// The second where the first gives one XCD much more than the others: eight [4096 x 2048] gradients over 16384 rows, group
+// sizes falling like 1 / rank^1.1, 363 -> 156 us, because one XCD owned the whole longest group.  The first otherwise: with
+// equal groups the second, whose operands every XCD fetches, is slower (16 x [1024 x 1024] over 16384 rows: 19.5 / 23.6 us,
+// 16 x [1408 x 2880] 81 / 91, 32 x [4096 x 2048] over 8192 152 / 177), and so it is with few tiles per group (32 x [1024 x
+// 1024] over 32768 rows of sizes like 1 / rank^1.1: 89 / 104).
+// Every workgroup decides alike from the lengths (k_slices_in_order).
 MSLK_AMD_DEVINL int k_slice_run(int per) { return per > kXcds ? (per + kXcds - 1) / kXcds : 1; }
-MSLK_AMD_DEVINL bool k_slice_tile(const DeviceGroups& p, int wg, int per, int& group, int& tile, int64_t& begin, int64_t& end) {
+
+// Whether the first order serves.  A tile costs its slice's length plus kTileCost, which is about what its output takes.  Of G / 8
+// groups an XCD gets in the first order the longest one sets the pace; the order serves while that XCD has at most a fifth
+// more than its share (beyond 64 groups, where the second sorts only some of them, a half).  It also serves where the second
+// order leaves a run of fewer than four neighbouring tiles, or none wait for a CU.
+MSLK_AMD_DEVINL bool k_slices_in_order(const DeviceGroups& p, int per, int per_xcd, int lane_begin, int lane_end) {
+  constexpr float kTileCost = 512.f;
+  if (p.G == 1 || per < 32 || per_xcd <= 32) return true;
   const int32_t* off = static_cast<const int32_t*>(p.layout);
   const int lane = threadIdx.x & 63;
-  const int run = k_slice_run(per), slot = wg / kXcds;
-  const int at = (slot / run * kXcds + wg % kXcds) * run + slot % run;
-  const int rank = at / per;
-  if (rank >= p.G) return false;
-  tile = __builtin_amdgcn_readfirstlane(at - rank * per);
-  int gi = rank;
-  if (rank < 64) {
-    // lane i holds the length of group i; its rank is the number of groups in front of it
-    const int n = p.G < 64 ? p.G : 64;
-    int len = -1;
-    if (lane < n) len = (int)((uint32_t)off[lane] - (lane ? (uint32_t)off[lane - 1] : 0u));
-    int ahead = 0;
-    for (int j = 0; j < n; ++j) {
-      const int other = __builtin_amdgcn_readlane(len, j);
-      ahead += (other > len || (other == len && j < lane)) ? 1 : 0;
+  auto length = [](int begin, int end) {   // of a consistent slice; anything else counts as none
+    const int len = (int)((uint32_t)end - (uint32_t)begin);
+    return len < 0 ? 0 : len;
+  };
+  int longest = length(lane_begin, lane_end);
+  for (int gi = 64 + lane; gi < p.G; gi += 64) {
+    const int len = length(off[gi - 1], off[gi]);
+    longest = len > longest ? len : longest;
+  }
+  const float most = (float)team_max<64>((uint32_t)longest, nullptr) + kTileCost, groups = (float)p.G;
+  const float all = (float)p.K + groups * kTileCost;
+  return (most * groups - all) * 8.f <= (p.G <= 64 ? 0.2f : 0.5f) * (groups < 8.f ? 8.f : groups) * all;
+}
+
+MSLK_AMD_DEVINL bool k_slice_tile(const DeviceGroups& p, int wg, int per, int& group, int& tile, int64_t& begin, int64_t& end) {
+  const int32_t* off = static_cast<const int32_t*>(p.layout);
+  const int lane = threadIdx.x & 63, total = p.G * per, per_xcd = (total + kXcds - 1) / kXcds;
+  const int lane_begin = lane && lane < p.G ? off[lane - 1] : 0, lane_end = lane < p.G ? off[lane] : 0;
+  int gi;
+  if (k_slices_in_order(p, per, per_xcd, lane_begin, lane_end)) {
+    const int at = wg % kXcds * per_xcd + wg / kXcds;
+    if (wg / kXcds >= per_xcd || at >= total) return false;
+    gi = at / per;
+    tile = __builtin_amdgcn_readfirstlane(at - gi * per);
+  } else {
+    const int run = k_slice_run(per), slot = wg / kXcds;
+    const int at = (slot / run * kXcds + wg % kXcds) * run + slot % run;
+    gi = at / per;
+    if (gi >= p.G) return false;
+    tile = __builtin_amdgcn_readfirstlane(at - gi * per);
+    if (gi < 64) {   // the group of rank gi: lane i holds the length of group i, its rank is the number of groups in front of it
+      const int n = p.G < 64 ? p.G : 64;
+      const int raw = (int)((uint32_t)lane_end - (uint32_t)lane_begin);
+      const int len = lane < n ? (raw < 0 ? -1 : raw) : INT32_MIN;   // lanes without a group are in front of none
+      int ahead = 0;
+      for (int j = 0; j < n; j += 8) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const int other = __builtin_amdgcn_readlane(len, j + k);
+          ahead += (other > len || (other == len && j + k < lane)) ? 1 : 0;
+        }
+      }
+      gi = __ffsll((long long)__ballot(lane < n && ahead == gi)) - 1;
     }
-    const unsigned long long hit = __ballot(lane < n && ahead == rank);
-    gi = __ffsll((long long)hit) - 1;
   }
   gi = __builtin_amdgcn_readfirstlane(gi);
   group = gi;
-  begin = gi ? off[gi - 1] : 0;
-  end = off[gi];
+  if (gi < 64) {
+    begin = __builtin_amdgcn_readlane(lane_begin, gi);
+    end = __builtin_amdgcn_readlane(lane_end, gi);
+  } else {
+    begin = off[gi - 1];
+    end = off[gi];
+  }
   return true;
 }
 
@@ -320,7 +364,8 @@ hipError_t launch_device_shape(const DeviceGroups& p, hipStream_t s) {
   const int64_t tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
   int64_t grid;
   if (LAYOUT == kGroupsOffsetsK) {
-    const int64_t per = tiles_m * tiles_n, run = per > kXcds ? (per + kXcds - 1) / kXcds : 1;   // k_slice_tile(): whole runs for every XCD
+    // k_slice_tile(): whole runs for every XCD, which is no less than an eighth of the list for each
+    const int64_t per = tiles_m * tiles_n, run = per > kXcds ? (per + kXcds - 1) / kXcds : 1;
     grid = ((p.G * per + run - 1) / run + kXcds - 1) / kXcds * kXcds * run;
   } else if (LAYOUT == kGroupsUniform || LAYOUT == kGroupsPrepadM) {
     grid = (p.G * tiles_m * tiles_n + kXcds - 1) / kXcds * kXcds;

@@ -35,3 +35,15 @@ def _run(ks, M, N):
 ])
 def test_every_tile_of_every_slice(ks, M, N):
     _run(ks, M, N)
+
+
+@pytest.mark.parametrize("ks,M,N", [
+    ([128] * 6, 1000, 1104),                               # 72 tiles per group, more than a tile per CU: groups in order ...
+    ([16, 48, 1024, 16, 0, 16], 1000, 1104),               # ... and by falling length, dealt to the XCDs
+    ([112, 128, 96, 128, 128, 112, 128], 1000, 1104),      # nearly equal: in order, XCDs begin inside a group
+    ([16] * 65 + [4096], 1408, 1400),                      # the longest slice behind the first 64 groups
+    ([16 * (i % 3) for i in range(66)], 1408, 1400),
+    ([32] * 40, 640, 640),                                 # 25 tiles per group: too few to deal out
+])
+def test_both_orders_of_the_slices(ks, M, N):
+    _run(ks, M, N)
