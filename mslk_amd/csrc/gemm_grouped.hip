@@ -182,17 +182,28 @@ static hipError_t launch_grouped_shape(const GroupTable& in, hipStream_t s) {
   return hipGetLastError();
 }
 
+// As for groups whose sizes only the device knows (small_row_groups), with what the sizes say besides: where 128 x 128 tiles need
+// more passes over the chip than 256 x 256 ones they lose if the larger ones need a single pass (32 x 2048 x 14336, 512 rows
+// of sizes like 1 / rank^1.1: 528 and 256 tiles, 217 / 156 us; 8 x 5120 x 4096, one group of 912 rows and seven of 16: 65 / 42),
+// and from K = 4096 on (16 x 5120 x 4096 over 2048 rows, one group of 1808: 108 / 89).  Shorter K gain from the two
+// workgroups of a CU also over several passes (64 x 4096 x 1024 over 4096 rows, one of 3088: 0.8 of the time).
 hipError_t launch_grouped_tiled(const GroupTable& in, hipStream_t s) {
   if (in.total_tiles <= 0 || in.count <= 0) return hipSuccess;
-  int64_t rows = 0, groups = 0, tiles128 = 0;
+  int64_t rows = 0, groups = 0, tiles128 = 0, tiles256 = 0, K = 0;
   for (int g = 0; g < in.count; ++g) {
-    rows += in.g[g].M;
-    groups += in.g[g].M > 0;
-    tiles128 += (int64_t)((in.g[g].M + 127) / 128) * ((in.g[g].N + 127) / 128);
+    const GroupDesc& d = in.g[g];
+    rows += d.M;
+    groups += d.M > 0;
+    tiles128 += (int64_t)((d.M + 127) / 128) * ((d.N + 127) / 128);
+    tiles256 += (int64_t)((d.M + 255) / 256) * ((d.N + 255) / 256);
+    K = d.K > K ? d.K : K;
   }
-  // (as lists 32 experts x 4096 x 1024 with 64 rows each: 35.7 against 42.7 us, 16 x 4096 x 5120 91.2 / 102.8)
+  const int64_t cus = device_compute_units();
+  const bool more_passes = (tiles128 + 2 * cus - 1) / (2 * cus) > (tiles256 + cus - 1) / cus && (tiles256 <= cus || K >= 4096);
   const bool launchable = tiles128 <= kMaxWorkgroups / kXcds;   // (one XCD may be given most of them, and its share sets the grid)
-  return launchable && small_row_groups(rows, groups, tiles128) ? launch_grouped_shape<128, 128>(in, s) : launch_grouped_shape<256, 256>(in, s);
+  // (as lists 32 experts x 4096 x 1024 with 64 rows each: 35.7 against 42.7 us, 16 x 4096 x 5120 91.2 / 102.8)
+  if (launchable && !more_passes && small_row_groups(rows, groups, tiles128)) return launch_grouped_shape<128, 128>(in, s);
+  return launch_grouped_shape<256, 256>(in, s);
 }
 
 // Whether every operand row of the problem can be fetched by the 16-byte DMA path.

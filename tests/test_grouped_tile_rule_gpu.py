@@ -18,6 +18,8 @@ DEV, F8 = "cuda:0", torch.float8_e4m3fn
     ([16 * (i % 5) + 1 for i in range(70)], 1032, 512),              # a list of more groups than one launch holds
     ([1024], 8192, 512),                                             # 512 small tiles
     ([1025], 8192, 512),                                             # 576
+    ([130] + [2] * 7, 8192, 512),                                    # as a list: two passes of small tiles, one of large ones
+    ([130] + [2] * 8, 8192, 512),                                    # two passes of either: small ones
     ([37, 410, 200], 1000, 520),                                     # K % 16 != 0: scalar tiles
 ])
 def test_rows_of_every_group(sizes, N, K):
