@@ -399,11 +399,17 @@ template <int LAYOUT, int BIAS>
 hipError_t launch_device_layout(const DeviceGroups& p, hipStream_t s) {
   const int64_t G = p.G > 0 ? p.G : 1;
   if constexpr (LAYOUT == kGroupsSizesM || LAYOUT == kGroupsOffsetsM) {
-    // The sizes are not known here: a group ends in half a tile on average.  Operands that take the scalar tile want many
+    // The sizes are not known here: a group ends in half a tile on average.  Where they may instead fill their tiles and those all
+    // run at once (equal groups of a multiple of 128 rows), the small tiles win by a third and lose a fifth when the sizes are
+    // skewed after all (8 x 4096 x 4096 over 2048 rows: equal 32 / 46 us, sizes like 1 / rank^1.1 59 / 48): the large ones are
+    // taken, except for short K, where the small ones win or tie either way (8 x 1024 x 512 over 8192: 8.5 / 11.9 and 12.0 / 13.7;
+    // 8 x 2048 x 768 over 4096: 10.1 / 14.0 and 14.8 / 15.7, but 16 of them 18.9 / 16.0).  Operands that take the scalar tile want many
     // workgroups (8 experts x 4096 x 1000 over 4096 rows: 32.0 ms, with 256 x 256 tiles 67.7).
     const int64_t M = p.M, N = p.N, tiles_m = G == 1 ? (M + 127) / 128 : (M + 64 * G) / 128, tiles128 = tiles_m * ((N + 127) / 128);
     const bool launchable = ((M + 127) / 128 + G) * ((N + 127) / 128) + kXcds <= kMaxWorkgroups;
-    if (launchable && (p.unaligned || small_row_groups(M, G, tiles128))) return launch_device_shape<LAYOUT, 128, 128, BIAS>(p, s);
+    const int64_t full_tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
+    const bool short_k = p.K < 768 && full_tiles128 <= 2 * device_compute_units();
+    if (launchable && (p.unaligned || short_k || small_row_groups(M, G, tiles128))) return launch_device_shape<LAYOUT, 128, 128, BIAS>(p, s);
     return launch_device_shape<LAYOUT, 256, 256, BIAS>(p, s);
   }
   // Tile shape from the average group: 256 x 256 once such tiles give every CU work.

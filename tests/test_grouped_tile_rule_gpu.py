@@ -18,6 +18,8 @@ DEV, F8 = "cuda:0", torch.float8_e4m3fn
     ([16 * (i % 5) + 1 for i in range(70)], 1032, 512),              # a list of more groups than one launch holds
     ([1024], 8192, 512),                                             # 512 small tiles
     ([1025], 8192, 512),                                             # 576
+    ([2048] * 4, 1024, 512),                                         # sizes on the device, full tiles of a short K: small ones
+    ([2049, 2047, 2000, 2096], 1024, 768),                           # a longer K: large ones
     ([130] + [2] * 7, 8192, 512),                                    # as a list: two passes of small tiles, one of large ones
     ([130] + [2] * 8, 8192, 512),                                    # two passes of either: small ones
     ([37, 410, 200], 1000, 520),                                     # K % 16 != 0: scalar tiles
