@@ -87,6 +87,16 @@ def _bias_args(bias: Optional[torch.Tensor], N: int, device: torch.device):
     return b.data_ptr(), (1 if b.dtype == torch.float32 else 2), b
 
 
+def _op(name: str, *args):
+    """The registered operator, outside of autograd: these products have no derivative, and autograd's fallback for such an
+    operator would make its results, and an output it writes, part of the graph of any input that requires a gradient."""
+    op = getattr(torch.ops.mslk, name)
+    if not torch.is_grad_enabled():
+        return op(*args)
+    with torch.no_grad():
+        return op(*args)
+
+
 def _rowwise_impl(XQ, WQ, x_scale, w_scale, bias, use_fast_accum, output=None, out_dtype=torch.bfloat16,
                   preshuffled=False):
     return torch.ops.mslk_amd.rowwise(XQ, WQ, x_scale, w_scale, bias, use_fast_accum, output, out_dtype == torch.float16, preshuffled)
@@ -105,7 +115,7 @@ def quantize_f8f8bf16_rowwise(X, WQ, w_scale, bias=None):
     (Y, XQ, x_scale) -- the pair every decode step of a caller of the reference issues (bench/gemm/gemm_ops.py:593-673).
     For 1 <= M <= 4 rows of bf16 with K % 128 == 0 (K >= 1024) it is ONE launch (every workgroup quantizes the rows itself; XQ and
     x_scale are the bits the stand-alone quantizer returns); other shapes run the two kernels."""
-    return torch.ops.mslk.quantize_f8f8bf16_rowwise(X, WQ, w_scale, bias)
+    return _op("quantize_f8f8bf16_rowwise", X, WQ, w_scale, bias)
 
 
 def f8f8f16_rowwise(XQ, WQ, x_scale, w_scale, bias=None, use_fast_accum=True):
@@ -160,20 +170,20 @@ def f8f8bf16_rowwise_grouped(XQ, WQ, x_scale, w_scale) -> List[torch.Tensor]:
     _check_grouped(XQ, WQ, x_scale, w_scale)
     if len(XQ) == 0:
         return []
-    return torch.ops.mslk.f8f8bf16_rowwise_grouped(list(XQ), list(WQ), list(x_scale), list(w_scale))
+    return _op("f8f8bf16_rowwise_grouped", list(XQ), list(WQ), list(x_scale), list(w_scale))
 
 
 def f8f8bf16_rowwise_grouped_cat(XQ, WQ, x_scale, w_scale) -> torch.Tensor:
     """Same computation, outputs concatenated along M (all groups must share N)."""
     _check_grouped(XQ, WQ, x_scale, w_scale)
     _check(len(XQ) > 0, "at least one group is required")
-    return torch.ops.mslk.f8f8bf16_rowwise_grouped_cat(list(XQ), list(WQ), list(x_scale), list(w_scale))
+    return _op("f8f8bf16_rowwise_grouped_cat", list(XQ), list(WQ), list(x_scale), list(w_scale))
 
 
 def f8f8bf16_rowwise_grouped_stacked(XQ, WQ, x_scale, w_scale, M_sizes) -> torch.Tensor:
     """XQ [total_M, K], WQ [G, N, K], x_scale [total_M], w_scale [G, N], M_sizes int64 [G] on the GPU
     (fp8_rowwise_grouped_gemm.hip:607-655).  M_sizes is never read on the host."""
-    return torch.ops.mslk.f8f8bf16_rowwise_grouped_stacked(XQ, WQ, x_scale, w_scale, M_sizes)
+    return _op("f8f8bf16_rowwise_grouped_stacked", XQ, WQ, x_scale, w_scale, M_sizes)
 
 
 def f8f8bf16_rowwise_grouped_mm(XQ, WQ, x_scale, w_scale, offsets, output) -> torch.Tensor:
@@ -187,7 +197,7 @@ def f8f8bf16_rowwise_grouped_mm(XQ, WQ, x_scale, w_scale, offsets, output) -> to
       XQ [G, M, K],    WQ [G, N, K]    no offsets       output [G, M, N]
       XQ [M, total_K], WQ [N, total_K] offsets over K   output [G, M, N]
     """
-    return torch.ops.mslk.f8f8bf16_rowwise_grouped_mm(XQ, WQ, x_scale, w_scale, offsets, output)
+    return _op("f8f8bf16_rowwise_grouped_mm", XQ, WQ, x_scale, w_scale, offsets, output)
 
 
 def f8f8bf16_rowwise_grouped_dynamic(XQ, WQ, x_scale, w_scale, zero_start_index_M, zeroing_output_tensor=True) -> torch.Tensor:
