@@ -583,13 +583,6 @@ const Kernel kernels[] = {
     kernel<grouped_mm_op>("mslk", "f8f8bf16_rowwise_grouped_mm"),
 };
 
-// What the Python functions call directly: the checks in front of a launch, for tensors on any device.
-TORCH_LIBRARY_FRAGMENT(mslk_amd, m) {
-  m.def("rowwise(Tensor XQ, Tensor WQ, Tensor x_scale, Tensor w_scale, Tensor? bias, bool use_fast_accum, Tensor? output, bool out_f16, "
-        "bool preshuffled) -> Tensor", rowwise);
-  m.def("check_grouped(Tensor[] XQ, Tensor[] WQ, Tensor[] x_scale, Tensor[] w_scale) -> ()", check_grouped);
-}
-
 }  // namespace
 
 // Binds the entry points of the library at `path`, all of them or none; returns an error message or null.

@@ -99,7 +99,17 @@ def _op(name: str, *args):
 
 def _rowwise_impl(XQ, WQ, x_scale, w_scale, bias, use_fast_accum, output=None, out_dtype=torch.bfloat16,
                   preshuffled=False):
-    return torch.ops.mslk_amd.rowwise(XQ, WQ, x_scale, w_scale, bias, use_fast_accum, output, out_dtype == torch.float16, preshuffled)
+    if not XQ.is_cuda:   # what the operator's kernel checks in front of this, in its order (without a GPU tensor there is no kernel)
+        _check(XQ.dtype == WQ.dtype, f"XQ and WQ dtypes must match, got {XQ.dtype} vs {WQ.dtype}")
+        _check(XQ.dtype == FP8_DTYPE, f"XQ and WQ must be {FP8_DTYPE} on gfx950, got {XQ.dtype}")
+        _check(x_scale.dtype == torch.float32 and w_scale.dtype == torch.float32, "Scales must be float32.")
+        _check(use_fast_accum, "AMD does not support disabling use_fast_accum.")
+        _check(False, "XQ must be a contiguous GPU tensor")
+    if output is not None:
+        _op("f8f8bf16_rowwise_out", XQ, WQ, x_scale, w_scale, output, bias, use_fast_accum)
+        return output
+    name = ("f8f8f16_rowwise" if out_dtype == torch.float16 else "f8f8bf16_rowwise") + ("_preshuffle" if preshuffled else "")
+    return _op(name, XQ, WQ, x_scale, w_scale, bias, use_fast_accum)
 
 
 def f8f8bf16_rowwise(XQ, WQ, x_scale, w_scale, bias=None, use_fast_accum=True):
@@ -115,6 +125,10 @@ def quantize_f8f8bf16_rowwise(X, WQ, w_scale, bias=None):
     (Y, XQ, x_scale) -- the pair every decode step of a caller of the reference issues (bench/gemm/gemm_ops.py:593-673).
     For 1 <= M <= 4 rows of bf16 with K % 128 == 0 (K >= 1024) it is ONE launch (every workgroup quantizes the rows itself; XQ and
     x_scale are the bits the stand-alone quantizer returns); other shapes run the two kernels."""
+    if not X.is_cuda:
+        _check(WQ.dtype == FP8_DTYPE, f"WQ must be {FP8_DTYPE} on gfx950, got {WQ.dtype}")
+        _check(w_scale.dtype == torch.float32, "Scales must be float32.")
+        _check(False, "WQ must be a contiguous 2-D GPU tensor")
     return _op("quantize_f8f8bf16_rowwise", X, WQ, w_scale, bias)
 
 
@@ -160,8 +174,11 @@ def ck_preshuffle(src: torch.Tensor, NXdl: int = 16) -> torch.Tensor:
 
 
 def _check_grouped(XQ: Sequence[torch.Tensor], WQ, x_scale, w_scale) -> None:
-    """The argument checks of the TensorList ops."""
-    torch.ops.mslk_amd.check_grouped(list(XQ), list(WQ), list(x_scale), list(w_scale))
+    """The argument checks of the TensorList ops in front of their kernel; the kernel makes the others."""
+    _check(len(XQ) == len(WQ) == len(x_scale) == len(w_scale), "All inputs must have the same number of groups.")
+    if len(XQ) > 0 and not XQ[0].is_cuda:
+        _check(XQ[0].dtype == FP8_DTYPE, f"XQ and WQ must be {FP8_DTYPE} on gfx950, got {XQ[0].dtype}")
+        _check(False, "XQ tensors must be contiguous GPU tensors")
 
 
 def f8f8bf16_rowwise_grouped(XQ, WQ, x_scale, w_scale) -> List[torch.Tensor]:
@@ -183,6 +200,7 @@ def f8f8bf16_rowwise_grouped_cat(XQ, WQ, x_scale, w_scale) -> torch.Tensor:
 def f8f8bf16_rowwise_grouped_stacked(XQ, WQ, x_scale, w_scale, M_sizes) -> torch.Tensor:
     """XQ [total_M, K], WQ [G, N, K], x_scale [total_M], w_scale [G, N], M_sizes int64 [G] on the GPU
     (fp8_rowwise_grouped_gemm.hip:607-655).  M_sizes is never read on the host."""
+    _check(XQ.is_cuda, "XQ/WQ must be contiguous GPU tensors")
     return _op("f8f8bf16_rowwise_grouped_stacked", XQ, WQ, x_scale, w_scale, M_sizes)
 
 
@@ -197,6 +215,7 @@ def f8f8bf16_rowwise_grouped_mm(XQ, WQ, x_scale, w_scale, offsets, output) -> to
       XQ [G, M, K],    WQ [G, N, K]    no offsets       output [G, M, N]
       XQ [M, total_K], WQ [N, total_K] offsets over K   output [G, M, N]
     """
+    _check(XQ.is_cuda, "XQ/WQ must be contiguous GPU tensors")
     return _op("f8f8bf16_rowwise_grouped_mm", XQ, WQ, x_scale, w_scale, offsets, output)
 
 
