@@ -25,16 +25,12 @@ def _native_schemas():
     return schemas
 
 
-def _register_missing(name: str, error: RuntimeError) -> None:
-    """The build is missing: the operator raises `error` when it is used on a GPU."""
-    def fail(*_args, **_kwargs):
-        raise error
-
+def _register_stub(name, kernel) -> None:
     namespace, operator = name.split("::")
-    {"triton": quantize._triton_library, "mslk": quantize._library}[namespace].impl(operator, fail, "CUDA", allow_override=True)
+    {"triton": quantize._triton_library, "mslk": quantize._library}[namespace].impl(operator, kernel, "CUDA", allow_override=True)
 
 
-_lib.load_torch_ops(_native_schemas(), _register_missing)   # every schema is defined by now
+_lib.load_torch_ops(_native_schemas(), _register_stub)   # every schema is defined by now
 
 __all__ = ["quantize_fp8_row", "quantize_fp8_per_row", "dequantize_fp8_row", "silu_mul_quant", "gather_scale_quant_dense_tokens", "f8f8bf16_rowwise", "f8f8bf16_rowwise_out", "quantize_f8f8bf16_rowwise", "f8f8f16_rowwise", "f8f8bf16_rowwise_preshuffle", "f8f8f16_rowwise_preshuffle", "preshuffle_b_mfma", "ck_preshuffle",
            "f8f8bf16_rowwise_grouped", "f8f8bf16_rowwise_grouped_cat", "f8f8bf16_rowwise_grouped_stacked",

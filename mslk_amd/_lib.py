@@ -109,27 +109,15 @@ def fits(name: str, schema: str) -> bool:
     return overload is not None and _types(overload._schema) == _types(torch._C.parse_schema(schema))
 
 
-def load_torch_ops(schemas, register_missing) -> None:
-    """Makes the native functions the GPU kernels of the operators of `schemas` (name -> schema, all of them defined by now, by
-    this package or by a library loaded before it).  An operator that was defined with other types keeps the kernel it has.
-    When the build is missing, `register_missing(name, error)` is called for each instead, to make the operators raise `error`
-    when they are used."""
-    import warnings
-    names = []
-    for name, schema in schemas.items():
-        if fits(name, schema):
-            names.append(name)
-        else:
-            warnings.warn(f"mslk_amd: {name} is already defined with other argument or result types than {schema}; its GPU "
-                          "kernel stays as it is")
+def _register_native(names) -> None:
+    """Binds the native functions to the C ABI and makes them the GPU kernels of the operators `names`."""
     for path in (LIB_PATH, TORCH_OPS_PATH):
         if not os.path.exists(path):
-            for name in names:
-                register_missing(name, _missing(path))
-            return
-    import torch
-    torch.ops.load_library(TORCH_OPS_PATH)
-    ops = ctypes.CDLL(TORCH_OPS_PATH)
+            raise _missing(path)
+    try:
+        ops = ctypes.CDLL(TORCH_OPS_PATH)
+    except OSError as e:   # built against another PyTorch
+        raise RuntimeError(f"mslk_amd: cannot load {TORCH_OPS_PATH}: {e}") from e
     ops.mslk_amd_torch_bind.restype, ops.mslk_amd_torch_bind.argtypes = c_char_p, [c_char_p]
     ops.mslk_amd_torch_register.restype, ops.mslk_amd_torch_register.argtypes = c_char_p, [c_char_p, c_char_p]
     error = ops.mslk_amd_torch_bind(os.fsencode(LIB_PATH))
@@ -139,3 +127,31 @@ def load_torch_ops(schemas, register_missing) -> None:
         error = ops.mslk_amd_torch_register(*(part.encode() for part in name.split("::")))
         if error is not None:
             raise RuntimeError(f"mslk_amd: cannot register the kernel of {name}: {error.decode()}")
+
+
+def load_torch_ops(schemas, register_stub) -> None:
+    """Makes the native functions the GPU kernels of the operators of `schemas` (name -> schema, all of them defined by now, by
+    this package or by a library loaded before it).  An operator that was defined with other types keeps the kernel it has.
+    Where the build is missing or incomplete (or another library named by MSLK_AMD_LIBRARY is), `register_stub(name, kernel)`
+    is called for each instead: a kernel that tries again when it is used, and raises what is wrong."""
+    import warnings
+    names = []
+    for name, schema in schemas.items():
+        if fits(name, schema):
+            names.append(name)
+        else:
+            warnings.warn(f"mslk_amd: {name} is already defined with other argument or result types than {schema}; its GPU "
+                          "kernel stays as it is")
+    try:
+        _register_native(names)
+    except RuntimeError:
+        def stub(name):
+            def kernel(*args, **kwargs):
+                import torch
+                _register_native(names)   # takes the place of the stubs
+                namespace, operator = name.split("::")
+                return getattr(getattr(torch.ops, namespace), operator)(*args, **kwargs)
+            return kernel
+
+        for name in names:
+            register_stub(name, stub(name))

@@ -592,7 +592,10 @@ extern "C" const char* mslk_amd_torch_bind(const char* path) {
   Api bound;
 #define X(name)                                                                              \
   bound.name = reinterpret_cast<decltype(bound.name)>(dlsym(lib, #name));                      \
-  if (bound.name == nullptr) return "the library does not export " #name;
+  if (bound.name == nullptr) {                                                                 \
+    dlclose(lib);                                                                              \
+    return "the library does not export " #name;                                               \
+  }
   MSLK_AMD_ENTRY_POINTS(X)
 #undef X
   api = bound;

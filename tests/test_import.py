@@ -1,6 +1,7 @@
 """Importing the package beside another library that defined some of its operators first: the GPU kernels are replaced where
 the types agree, other operators keep what they have, and the import never takes the process down.  CPU, one process each."""
 import os
+import shutil
 import subprocess
 import sys
 
@@ -57,4 +58,46 @@ import mslk_amd
 assert "CUDA: registered at torch_ops.cpp" in torch._C._dispatch_dump("mslk::f8f8bf16_rowwise")
 print("imported")
 ''')
+    assert r.returncode == 0 and "imported" in r.stdout, r.stderr[-3000:]
+
+
+CALL = """
+cuda = torch._C.DispatchKeySet(torch._C.DispatchKey.CUDA)   # the GPU's kernel, on CPU tensors
+def call():
+    try:
+        torch.ops.mslk.f8f8bf16_rowwise.default.redispatch(cuda, *[torch.zeros(1, 16)] * 4, None, True)
+    except RuntimeError as e:
+        return str(e)
+"""
+
+
+def test_a_process_that_imported_before_the_build_finds_it_later(tmp_path):
+    package = shutil.copytree(os.path.join(ROOT, "mslk_amd"), tmp_path / "mslk_amd", ignore=shutil.ignore_patterns("*.so", "csrc"))
+    r = _run(f'''
+import shutil, sys, torch
+sys.path.insert(0, {str(tmp_path)!r})
+import mslk_amd
+assert mslk_amd.__file__.startswith({str(tmp_path)!r})
+{CALL}
+assert "libmslk_amd.so is missing" in call(), call()
+shutil.copy({os.path.join(ROOT, "mslk_amd", "libmslk_amd.so")!r}, {str(package)!r})
+assert "_torch_ops.so is missing" in call(), call()
+shutil.copy({os.path.join(ROOT, "mslk_amd", "_torch_ops.so")!r}, {str(package)!r})
+call()   # replaces the kernels and calls the operator again, which has none for the CPU
+assert "must be torch.float8_e4m3fn" in call(), call()      # the native checks
+print("imported")
+''')
+    assert r.returncode == 0 and "imported" in r.stdout, r.stderr[-3000:]
+
+
+def test_a_library_without_an_entry_point_leaves_no_kernel_over_null_pointers(tmp_path):
+    source, library = tmp_path / "older.c", tmp_path / "libolder.so"
+    source.write_text('const char* mslk_amd_last_error(void) { return ""; }')
+    subprocess.run(["gcc", "-shared", "-fPIC", str(source), "-o", str(library)], check=True)
+    r = _run(f'''
+import torch, mslk_amd
+{CALL}
+assert "cannot bind" in call() and "does not export" in call(), call()
+print("imported")
+''', MSLK_AMD_LIBRARY=str(library))
     assert r.returncode == 0 and "imported" in r.stdout, r.stderr[-3000:]
