@@ -9,7 +9,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 
 
 def build(force: bool = False, jobs: int = 8) -> str:
-    cmd = ["make", "-C", os.path.join(_HERE, "csrc"), f"-j{jobs}", f"PYTHON={sys.executable}"]
+    cmd = ["make", "-C", os.path.join(_HERE, "csrc"), f"-j{jobs}", "all", f"PYTHON={sys.executable}"]
     if force:
         cmd.append("-B")
     subprocess.check_call(cmd)

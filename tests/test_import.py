@@ -101,3 +101,9 @@ assert "cannot bind" in call() and "does not export" in call(), call()
 print("imported")
 ''', MSLK_AMD_LIBRARY=str(library))
     assert r.returncode == 0 and "imported" in r.stdout, r.stderr[-3000:]
+
+
+def test_the_c_library_alone_is_built_without_pytorch():
+    make = ["make", "-n", "-B", "-C", os.path.join(ROOT, "mslk_amd", "csrc"), "PYTHON=/nonexistent"]
+    r = subprocess.run(make, capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and "libmslk_amd.so" in r.stdout and "torch" not in r.stdout, r.stdout[-500:] + r.stderr
