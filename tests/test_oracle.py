@@ -378,10 +378,10 @@ def test_elementwise_criterion_counts_what_it_should():
 
 
 def test_reciprocal_fma_division_gives_the_codes_of_the_ieee_division():
-    """The quantizer's Triton-arithmetic mode replaces x / s by r = 1 / s, q0 = x r, e = fma(-q0, s, x), q = e == 0 ? q0 :
-    fma(e, r, q0) in rows whose maximum is a bf16 / fp16 value of at least 2^-64.  Exhaustive over every such maximum and every
-    element not above it (2 x 10^9 pairs, split over threads): the e4m3 codes are the same.  Below 2^-64 the forms do differ
-    (which is why the kernel divides there)."""
+    """The quantizer's Triton-arithmetic mode replaces x / s by r = 1 / s, q0 = x r, e = fma(q0, s, -x), q = fma(-e, r, q0),
+    converted without a clamp, in rows whose maximum is a bf16 / fp16 value of at least 2^-64.  Exhaustive over every such
+    maximum and every element not above it (2 x 10^9 pairs, split over threads): the e4m3 codes are the same.  Below 2^-64 the
+    forms do differ (which is why the kernel divides there)."""
     from concurrent.futures import ThreadPoolExecutor
     jobs = []
     bf16_lo, bf16_hi = 0x1F80, 0x7F80                      # 2^-64 ... the first non-finite bf16
