@@ -3,7 +3,7 @@
 Importing the package registers `torch.ops.mslk.f8f8bf16_rowwise`, `..._rowwise_out`,
 `..._rowwise_grouped`, `..._rowwise_grouped_cat`, `..._rowwise_grouped_stacked`,
 `..._rowwise_grouped_mm`, `..._rowwise_batched` and
-`torch.ops.mslk.quantize_fp8_row` / `dequantize_fp8_row`, all backed by hand-written HIP kernels in libmslk_amd.so.
+`torch.ops.triton.quantize_fp8_row`, `torch.ops.mslk.quantize_fp8_per_row` / `dequantize_fp8_row`, all backed by hand-written HIP kernels in libmslk_amd.so.
 """
 from . import _lib, quantize  # noqa: F401
 from .quantize import (quantize_fp8_row, quantize_fp8_per_row, dequantize_fp8_row,  # noqa: F401

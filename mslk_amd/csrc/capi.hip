@@ -278,7 +278,7 @@ int mslk_amd_quantize_f8f8bf16_rowwise(const void* x, int x_dtype, int64_t x_row
   if (bias_dtype < 0 || bias_dtype > 2) return fail("%s: bad bias dtype code %d", op, bias_dtype);
   if ((bias_dtype != 0) != (bias != nullptr)) return fail("%s: bias pointer and bias dtype disagree", op);
   if (!mslk_amd_quantize_f8f8bf16_rowwise_supported(M, N, K))
-    return fail("%s: the one-launch path needs 1 <= M <= 4 and K a multiple of 1024 (got M=%lld, N=%lld, K=%lld); "
+    return fail("%s: the one-launch path needs 1 <= M <= 4 and K a multiple of 128, at least 1024 (got M=%lld, N=%lld, K=%lld); "
                 "use mslk_amd_quantize_fp8_row followed by mslk_amd_f8f8bf16_rowwise", op, (long long)M, (long long)N, (long long)K);
   if (!x || !wq || !w_scale || !y) return fail("%s: null pointer", op);
   GemmProblem p{nullptr, (const uint8_t*)wq, nullptr, w_scale, bias, (uint16_t*)y, (int)M, (int)N, (int)K, bias_dtype, 0, 0};

@@ -178,8 +178,8 @@ MSLK_AMD_DEVINL bool find_group(const DeviceGroups& p, int t, GroupSpan& sp) {
   } else {
     // The G extents are read 64 at a time, one per lane, and turned into tile ranges by a wave-level prefix sum, so the
     // lookup costs one memory round trip for up to 128 groups (the first two chunks are fetched together and stay in
-    // registers) instead of G dependent ones.  A workgroup holds its CU's whole LDS, so nothing else runs under the lookup:
-    // with more round trips for the groups beyond 64 and sums through LDS shuffles (a hundred cycles per step) 128 experts x
+    // registers) instead of G dependent ones.  A workgroup of 256 x 256 tiles holds its CU's whole LDS, so nothing else runs
+    // under its lookup (two of 128 x 128 share a CU): with more round trips for the groups beyond 64 and sums through LDS shuffles (a hundred cycles per step) 128 experts x
     // 2048 x 768 took 65.5 us over 8192 rows and 120.0 over 32768 (now 56.3 and 114.8), 64 x 4096 x 1024 over 16384 128.4
     // (120.1), 16 x 8192 x 5120 over 8192 324 (323).
     // The total tile count is formed first: XCD x (workgroup id mod 8) then takes a contiguous slice of the tile list, so

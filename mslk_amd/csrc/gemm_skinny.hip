@@ -386,7 +386,7 @@ hipError_t launch_lds(const GemmProblem& p, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Decode with the activation quantizer fused in: bf16 activations in, M <= 4, K % 1024 == 0.
+// Decode with the activation quantizer fused in: bf16 activations in, M <= 4, K % 128 == 0 from 1024 on.
 //
 // The reference quantizes the activations with one launch and multiplies with a second
 // (bench/gemm/gemm_ops.py:593-673); at decode sizes the first launch costs about a third of the pair.  Here every

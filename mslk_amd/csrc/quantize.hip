@@ -15,7 +15,7 @@
 //
 // The pass is HBM-bound (2 B in + 1 B out per element for bf16), so the kernel is organised
 // around 128-bit coalesced loads that stay in registers between the amax pass and the convert
-// pass: a row is owned by a "team" of 4 ... 1024 lanes, each of which keeps NV vectors of 8 elements.
+// pass: a row is owned by a "team" of 8 ... 1024 lanes, each of which keeps NV vectors of 8 elements.
 // Rows beyond that are streamed twice (the second read hits L2 / Infinity Cache).
 #include "common.h"
 #include "kernels.h"
