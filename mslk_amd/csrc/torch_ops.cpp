@@ -125,6 +125,8 @@ std::tuple<Tensor, Tensor> quantize_launch(const Tensor& a, const OptTensor& sca
   const int code = float_code(a.scalar_type());
   TORCH_CHECK(code >= 0, "quantize_fp8_row: unsupported input dtype ", a.scalar_type(), " (bf16, fp16, fp32 are supported)");
   TORCH_CHECK(a.dim() >= 1, "quantize_fp8_row: input must have at least one dimension");
+  // (an optional operand on a GPU is enough to get here)
+  TORCH_CHECK(a.is_cuda(), "quantize_fp8_row: input must be a GPU tensor");
   // same restriction as the reference's GPU path (fp8_quantize.py:235)
   TORCH_CHECK(a.dim() <= 4, "Only up to 4 dimension input tensor is supported if use_triton is True");
   const int64_t K = a.size(-1), rows = rows_of(a);
@@ -250,6 +252,7 @@ std::tuple<Tensor, Tensor> silu_mul_quant(const Tensor& x0, const Tensor& x1, co
   const int code = float_code(x0.scalar_type());
   TORCH_CHECK(code == MSLK_AMD_DTYPE_BF16 || code == MSLK_AMD_DTYPE_F16, "silu_mul_quant: inputs must be bfloat16 or float16, got ", x0.scalar_type());
   TORCH_CHECK(x1.device() == x0.device(), "x0 and x1 must be on the same device");
+  TORCH_CHECK(x0.is_cuda(), "silu_mul_quant: inputs must be GPU tensors");
   const int64_t T = x0.size(0), D = x0.size(1);
   Tensor out = empty_on({T, D}, kF8, x0), out_scale = empty_on({T}, at::kFloat, x0);
   if (T == 0 || D == 0) return {out, out_scale};
@@ -273,6 +276,7 @@ std::tuple<Tensor, Tensor> gather_scale_quant_dense_tokens(const Tensor& x, cons
   TORCH_CHECK(is_index(token_indices) && is_index(expert_indices), "indices must be int32 or int64");
   TORCH_CHECK(token_indices.device() == x.device() && expert_indices.device() == x.device() && scores.device() == x.device(),
               "all operands must be on the same device");
+  TORCH_CHECK(x.is_cuda(), "gather_scale_quant_dense_tokens: inputs must be GPU tensors");
   Tensor out = empty_on({a, D}, kF8, x), out_scale = empty_on({a}, at::kFloat, x);
   if (a == 0 || D == 0) return {out, out_scale};
   const Scalars s = scalars_of(scale_ub, valid_token_count, x);
@@ -472,6 +476,8 @@ Tensor grouped_stacked_op(const Tensor& XQ, const Tensor& WQ, const Tensor& x_sc
   TORCH_CHECK(K == WQ.size(2), "XQ and WQ must share K");
   TORCH_CHECK(M_sizes.numel() == G, "M_sizes must have one entry per group");
   TORCH_CHECK(x_scale.numel() == total_M && w_scale.numel() == G * N, "scale sizes must match total_M and G*N");
+  TORCH_CHECK(WQ.device() == XQ.device() && x_scale.device() == XQ.device() && w_scale.device() == XQ.device() && M_sizes.device() == XQ.device(),
+              "all operands must be on the same device");
   Tensor Y = empty_on({total_M, N}, at::kBFloat16, XQ);
   if (total_M == 0 || N == 0 || G == 0) return Y;
   if (K == 0) return Y.zero_();

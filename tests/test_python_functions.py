@@ -89,3 +89,29 @@ def test_dense_functions_compile_into_one_graph(name):
 
     x = torch.randn(40, 256, device="cuda:0", dtype=BF16)
     assert torch.equal(torch.compile(linear, backend="aot_eager", fullgraph=True)(x), linear(x))
+
+
+@pytest.mark.parametrize("name,args", [
+    ("mslk::silu_mul_quant", lambda: (torch.zeros(2, 8, dtype=BF16), torch.zeros(2, 8, dtype=BF16))),
+    ("mslk::gather_scale_quant_dense_tokens", lambda: (torch.zeros(2, 8, dtype=BF16), torch.zeros(2, dtype=torch.int32),
+                                                       torch.zeros(2, dtype=torch.int32), torch.zeros(2, 3))),
+    ("triton::quantize_fp8_row", lambda: (torch.zeros(2, 8, dtype=BF16),)),
+])
+def test_kernels_refuse_cpu_inputs_that_reach_them(name, args):
+    """An optional operand on a GPU is enough to pick the GPU's kernel; here it is called directly."""
+    namespace, operator = name.split("::")
+    overload = getattr(getattr(torch.ops, namespace), operator).default
+    optional = [a.default_value for a in overload._schema.arguments[len(args()):]]
+    with pytest.raises(RuntimeError, match="must be (a )?GPU tensor"):
+        overload.redispatch(torch._C.DispatchKeySet(torch._C.DispatchKey.CUDA), *args(), *optional)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("elsewhere", ["x_scale", "w_scale"])
+def test_stacked_form_refuses_scales_in_host_memory(elsewhere):
+    operands = {"XQ": torch.zeros(8, 512, device="cuda:0").to(F8), "WQ": torch.zeros(2, 512, 512, device="cuda:0").to(F8),
+                "x_scale": torch.ones(8, device="cuda:0"), "w_scale": torch.ones(2, 512, device="cuda:0"),
+                "M_sizes": torch.tensor([3, 5], device="cuda:0")}
+    operands[elsewhere] = operands[elsewhere].cpu()
+    with pytest.raises(RuntimeError, match="same device"):
+        torch.ops.mslk.f8f8bf16_rowwise_grouped_stacked(**operands)
