@@ -198,7 +198,7 @@ __global__ __launch_bounds__(TEAM > 256 ? TEAM : 256) void quantize_rows_vec_ker
   };
   // A wavefront without a live row (where rows are as wide as a workgroup, the whole workgroup): zero codes, whatever scale_ub
   // makes of the scale (0 / 0 is no zero), and nothing read or reduced.
-  if (__ballot(live) == 0) {
+  if (jag.zero_start != nullptr && __ballot(live) == 0) {
     float inv, sc;
     scales_from_amax<DTYPE, TRITON>(0.f, scale_ub, jag.triton_eps, inv, sc);
     if (lane == 0 && valid) scale[row] = sc;
