@@ -165,7 +165,10 @@ MSLK_AMD_DEVINL bool row_is_plain(float amax, const float* scale_ub, float trito
 // workgroup of TEAM >= 256 lanes.  Bound by HBM: all NV loads of a lane are in flight before the maximum is formed
 // (rows.h).  Against loads that waited for each other, Triton arithmetic on bf16: 4096 x 4096 11.9 -> 10.0 us (5.0 TB/s),
 // 8192 x 8192 41.8 -> 30.5 (6.6 TB/s), 131072 x 128 16.7 -> 10.8, 64 x 14336 4.9 -> 3.4 (the cost of a launch).
-template <int DTYPE, int TEAM, int NV, bool TRITON>
+// PART: a vector wholly beyond the row of a wavefront reads as zero, but is not worth its arithmetic (1024 x 16392 with scale_ub,
+// Triton arithmetic: 17.5 -> 12.9 us; 2047 x 64, three of four wavefronts without a vector: 4.3 -> 3.8).  A kernel of its own:
+// the branches between the vectors keep their conversions apart (40 ns).
+template <int DTYPE, int TEAM, int NV, bool TRITON, bool PART>
 __global__ __launch_bounds__(TEAM > 256 ? TEAM : 256) void quantize_rows_vec_kernel(
     const void* __restrict__ x, int64_t rows, int K, int64_t in_stride, uint8_t* __restrict__ out,
     int64_t out_stride, float* __restrict__ scale, const float* __restrict__ scale_ub, JaggedRows jag) {
@@ -196,8 +199,12 @@ __global__ __launch_bounds__(TEAM > 256 ? TEAM : 256) void quantize_rows_vec_ker
     if (valid)
       for (int64_t k = K + lane; k < out_stride; k += TEAM) out[row * out_stride + k] = 0;
   };
+  Vec8<DTYPE> cache[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) cache[i] = load_vec8<DTYPE>(src, at(i, live, (uint32_t)in_stride * ELEM_BYTES, 8 * ELEM_BYTES));
   // A wavefront without a live row (where rows are as wide as a workgroup, the whole workgroup): zero codes, whatever scale_ub
-  // makes of the scale (0 / 0 is no zero), and nothing read or reduced.
+  // makes of the scale (0 / 0 is no zero), and nothing reduced.  (Behind the loads, which read no memory there: 40 ns less for
+  // every other row.)
   if (jag.zero_start != nullptr && __ballot(live) == 0) {
     float inv, sc;
     scales_from_amax<DTYPE, TRITON>(0.f, scale_ub, jag.triton_eps, inv, sc);
@@ -207,26 +214,23 @@ __global__ __launch_bounds__(TEAM > 256 ? TEAM : 256) void quantize_rows_vec_ker
     pad();
     return;
   }
-  // Whether the wavefront owns any part of vector i: one wholly beyond the row reads as zero, but is not worth its arithmetic
-  // (1024 x 16392 with scale_ub, Triton arithmetic: 17.5 -> 12.9 us; 2047 x 64, three of four wavefronts without a vector:
-  // 4.3 -> 3.8).
-  auto used = [&](int i) { return (uint32_t)(i * TEAM + (TEAM > kWave ? wave * kWave : 0)) < nvec; };
-  Vec8<DTYPE> cache[NV];
-#pragma unroll
-  for (int i = 0; i < NV; ++i) cache[i] = load_vec8<DTYPE>(src, at(i, live, (uint32_t)in_stride * ELEM_BYTES, 8 * ELEM_BYTES));
   uint32_t m = 0;
 #pragma unroll
   for (int i = 0; i < NV; ++i) m = absmax_bits<DTYPE>(m, cache[i]);   // vectors beyond the row and dead rows read as zero
   m = team_max<TEAM>(finish_absmax_bits<DTYPE>(m), smem);
 
+  // Whether the wavefront owns any part of vector i (PART: some wavefront does not).
+  auto used = [&](int i) { return !PART || (uint32_t)(i * TEAM + (TEAM > kWave ? wave * kWave : 0)) < nvec; };
   float inv, sc, rcp;
   const float amax = Traits<DTYPE>::abs_bits_to_f32(m);
   scales_from_amax<DTYPE, TRITON>(amax, scale_ub, jag.triton_eps, inv, sc);
   if (lane == 0 && valid) scale[row] = sc;
   if (row_is_plain<DTYPE, TRITON>(amax, scale_ub, jag.triton_eps, inv, rcp)) {
 #pragma unroll
-    for (int i = 0; i < NV; ++i)
-      if (used(i)) buffer_store8_through(dst, at(i, valid, (uint32_t)out_stride, 8), quantize_vec8<DTYPE, TRITON, kModePlain>(cache[i], inv, rcp));
+    for (int i = 0; i < NV; ++i) {
+      if (!used(i)) break;
+      buffer_store8_through(dst, at(i, valid, (uint32_t)out_stride, 8), quantize_vec8<DTYPE, TRITON, kModePlain>(cache[i], inv, rcp));
+    }
   } else {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -409,8 +413,13 @@ hipError_t launch_quantize_t(const void* x, int64_t rows, int64_t K, int64_t in_
   const int64_t nvec = K / 8;
   auto team = [&](auto t, auto n) {
     constexpr int TEAM = decltype(t)::value, NV = decltype(n)::value, TEAMS = TEAM > 256 ? 1 : 256 / TEAM;
-    quantize_rows_vec_kernel<DTYPE, TEAM, NV, TRITON><<<TEAM <= kWave ? dim3((unsigned)((rows + TEAMS - 1) / TEAMS)) : row_grid(rows), TEAM > 256 ? TEAM : 256, 0, s>>>(
-        x, rows, k, in_stride, out, out_stride, scale, scale_ub, jag);
+    const dim3 grid = TEAM <= kWave ? dim3((unsigned)((rows + TEAMS - 1) / TEAMS)) : row_grid(rows);
+    if (TEAM >= kWave && nvec <= NV * TEAM - kWave)
+      quantize_rows_vec_kernel<DTYPE, TEAM, NV, TRITON, TEAM >= kWave><<<grid, TEAM > 256 ? TEAM : 256, 0, s>>>(
+          x, rows, k, in_stride, out, out_stride, scale, scale_ub, jag);
+    else
+      quantize_rows_vec_kernel<DTYPE, TEAM, NV, TRITON, false><<<grid, TEAM > 256 ? TEAM : 256, 0, s>>>(
+          x, rows, k, in_stride, out, out_stride, scale, scale_ub, jag);
     return hipGetLastError();
   };
   // From 2048 rows on the chip is full with a wavefront or less per row: as many lanes as give each one to four vectors,
