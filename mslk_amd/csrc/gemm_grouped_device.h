@@ -382,7 +382,8 @@ hipError_t launch_device_shape(const DeviceGroups& p, hipStream_t s) {
 
 // 128 x 128 or 256 x 256 tiles for groups of rows (sizes known on the host or not).  Two 128 x 128 workgroups share a CU, so
 // one hides the other's first round trip and its epilogue; a 256 x 256 tile reads half as many operand bytes per product, and
-// a ragged one costs what its rows cost.  The small tiles win where they all run at once (8 experts x 1536 x 2048 over 4096
+// a ragged one costs what its rows cost.  The figures here are of sizes that fall like 1 / rank^1.1 and of weights that are not
+// in the caches; equal sizes differ where tiles fill (launch_device_layout below).  The small tiles win where they all run at once (8 experts x 1536 x 2048 over 4096
 // rows, 432 tiles: 19.8 against 27.5 us; 1 x 8192 x 5120 over 1024, 512 tiles: 47.0 / 54.4; but 2 x 4096 x 4096 over 2048, 544
 // tiles: 52.4 / 43.1; 8 x 4096 x 2048 over 2048, 640 tiles: 37.9 / 27.0) and up to 128 rows per group, where the weight
 // stream is the bound and half the rows of a 256-row tile are padding (64 x 2048 x 2048, by rows per group: 64 60.2 / 75.7,
