@@ -18,11 +18,25 @@
 namespace mslk_amd {
 namespace {
 
+// XCD x works on its own contiguous slice of the tile list (the launcher has cut the list by estimated cost).  Tile of the group
+// whose descriptor is tab.g[gi].
+MSLK_AMD_DEVINL void listed_tile(const GroupTable& tab, int gi, int row, int col, RowTile& w) {
+  const GroupDesc& d = tab.g[gi];
+  w.a = d.xq + (int64_t)row * d.K;
+  w.b = d.wq + (int64_t)col * d.K;
+  w.xs = d.xs + row;
+  w.ws = d.ws + col;
+  w.y = d.y + (int64_t)row * d.N + col;
+  w.m_rem = d.M - row;
+  w.n_rem = d.N - col;
+  w.N = d.N;
+  w.K = d.K;
+}
+
 template <int BM, int BN>
 __global__ __launch_bounds__(256) void grouped_tiled_kernel(GroupTable tab) {
   using TS = TileShape<BM, BN>;
   __shared__ __attribute__((aligned(1024))) char lds[TS::LDS_BYTES];
-  // XCD x works on its own contiguous slice of the tile list (the launcher has cut the list by estimated cost).
   const int xcd = blockIdx.x % kXcds;
   const int t = tab.xcd_begin[xcd] + blockIdx.x / kXcds;
   if (t >= tab.xcd_begin[xcd + 1]) return;
@@ -30,22 +44,53 @@ __global__ __launch_bounds__(256) void grouped_tiled_kernel(GroupTable tab) {
   const int lane = threadIdx.x & 63;
   const int begin = lane < tab.count ? tab.g[lane].tile_begin : 0x7FFFFFFF;
   const int gi = __builtin_amdgcn_readfirstlane(__popcll(__ballot(t >= begin)) - 1);
-  const GroupDesc& d = tab.g[gi];
-  const int tiles_m = (d.M + BM - 1) / BM, tiles_n = (d.N + BN - 1) / BN;
   int tm, tn;
-  const int panel_rows = local_tile(t - d.tile_begin, tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
+  const int panel_rows = local_tile(t - tab.g[gi].tile_begin, (tab.g[gi].M + BM - 1) / BM, (tab.g[gi].N + BN - 1) / BN, tm, tn);
+  RowTile w;
+  listed_tile(tab, gi, tm * BM, tn * BN, w);
   // ROWSKIP: the ragged last row tile of a group costs what its rows cost.  A tile alone in its panel is the only reader
   // of its weight block at that time: it fetches the weights with non-temporal loads.
   if (panel_rows == 1) {
     GemmTile<TS, 0, false, true, TS::LA / 2, false, true> tile;
-    tile.run(lds, d.xq + (int64_t)m0 * d.K, d.wq + (int64_t)n0 * d.K, d.xs + m0, d.ws + n0, nullptr,
-             d.y + (int64_t)m0 * d.N + n0, d.M - m0, d.N - n0, d.N, d.K);
+    tile.run(lds, w.a, w.b, w.xs, w.ws, nullptr, w.y, w.m_rem, w.n_rem, w.N, w.K);
   } else {
     GemmTile<TS, 0, false, true> tile;
-    tile.run(lds, d.xq + (int64_t)m0 * d.K, d.wq + (int64_t)n0 * d.K, d.xs + m0, d.ws + n0, nullptr,
-             d.y + (int64_t)m0 * d.N + n0, d.M - m0, d.N - n0, d.N, d.K);
+    tile.run(lds, w.a, w.b, w.xs, w.ws, nullptr, w.y, w.m_rem, w.n_rem, w.N, w.K);
   }
+}
+
+// 256 x 256 tiles: one workgroup per CU walks the slice of its XCD.
+__global__ __launch_bounds__(256) void grouped_listed_kernel(GroupTable tab) {
+  using TS = RowTileShape;
+  constexpr int BM = TS::kBM, BN = TS::kBN;
+  __shared__ __attribute__((aligned(1024))) char lds[TS::LDS_BYTES];
+  const int xcd = blockIdx.x % kXcds, begin = tab.xcd_begin[xcd], end = tab.xcd_begin[xcd + 1], stride = gridDim.x / kXcds;
+  const int lane = threadIdx.x & 63;
+  const int first = lane < tab.count ? tab.g[lane].tile_begin : 0x7FFFFFFF;   // of group `lane`
+  int slot = blockIdx.x / kXcds, i = 64;
+  TileBatch b;
+  walk_row_tiles(lds, [&](RowTile& w) {
+    if (i == 64) {
+      const int t = begin + slot + lane * stride;
+      int gi = 0;   // the last group that begins at or before t
+#pragma unroll
+      for (int step = 32; step > 0; step >>= 1) gi += __shfl(first, gi + step, 64) <= t ? step : 0;
+      const GroupDesc& d = tab.g[gi];
+      int tm, tn;
+      b.stream = local_tile(t < end ? t - d.tile_begin : 0, (d.M + BM - 1) / BM, (d.N + BN - 1) / BN, tm, tn) == 1;
+      b.row = tm * BM;
+      b.col = tn * BN;
+      b.group = gi;
+      b.count = __popcll(__ballot(t < end));
+      slot += 64 * stride;
+      i = 0;
+    }
+    if (i >= b.count) return false;
+    listed_tile(tab, __builtin_amdgcn_readlane(b.group, i), __builtin_amdgcn_readlane(b.row, i), __builtin_amdgcn_readlane(b.col, i), w);
+    w.stream = __builtin_amdgcn_readlane(b.stream, i);
+    ++i;
+    return true;
+  });
 }
 
 }  // namespace
@@ -180,6 +225,14 @@ static hipError_t launch_grouped_shape(const GroupTable& in, hipStream_t s) {
   int longest = 0;
   for (int i = 0; i < kXcds; ++i)
     if (t.xcd_begin[i + 1] - t.xcd_begin[i] > longest) longest = t.xcd_begin[i + 1] - t.xcd_begin[i];
+  if constexpr (BM == RowTileShape::kBM) {
+    bool chain = true;
+    for (int i = 0; i < n; ++i) chain = chain && chain_takes(t.g[i].N, t.g[i].K, t.g[i].xq, t.g[i].wq, t.g[i].ws, t.g[i].y);
+    if (chain) {
+      grouped_listed_kernel<<<(longest < wgs_per_xcd ? longest : wgs_per_xcd) * kXcds, 256, 0, s>>>(t);
+      return hipGetLastError();
+    }
+  }
   grouped_tiled_kernel<BM, BN><<<longest * kXcds, 256, 0, s>>>(t);
   return hipGetLastError();
 }

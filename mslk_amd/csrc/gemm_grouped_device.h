@@ -150,6 +150,133 @@ MSLK_AMD_DEVINL bool k_slice_tile(const DeviceGroups& p, int wg, int per, int& g
   return true;
 }
 
+// Groups of rows (or of columns) by sizes or offsets: the tile list of a launch, and the group a tile of it belongs to.
+// The G extents are read 64 at a time, one per lane, and turned into tile ranges by a wave-level prefix sum, so the
+// lookup costs one memory round trip for up to 128 groups (the first two chunks are fetched together and stay in
+// registers) instead of G dependent ones.  A workgroup of 256 x 256 tiles holds its CU's whole LDS, so nothing else runs
+// under its lookup (two of 128 x 128 share a CU): with more round trips for the groups beyond 64 and sums through LDS shuffles (a hundred cycles per step) 128 experts x
+// 2048 x 768 took 65.5 us over 8192 rows and 120.0 over 32768 (now 56.3 and 114.8), 64 x 4096 x 1024 over 16384 128.4
+// (120.1), 16 x 8192 x 5120 over 8192 324 (323).
+// The total tile count is formed first: XCD x (workgroup id mod 8) then takes a contiguous slice of the tile list, so
+// that the row tiles of a group that share a weight panel run on one XCD and find it in its L2 (without the slices the
+// device-extent layouts fetched 1.6 times what the host-extent kernel fetches for the same 16 experts).
+template <int LAYOUT, int BM, int BN>
+struct BlockGroups {
+  // Every quantity fits 32 bits (the host checks the dimensions and the grid): sizes beyond the tensor mark the group bad.
+  struct Extent { int64_t size; int begin, end; };
+  struct Chunk { int start, len, tiles, incl; };
+  Chunk c0, c1;
+  int carry_len2;        // of the first 128 groups, for the chunks beyond them
+  bool seen_bad2;
+  int64_t total_tiles;   // of the launch
+  int64_t per_xcd;       // of an XCD's slice
+
+  MSLK_AMD_DEVINL static Extent fetch(const DeviceGroups& p, int base) {
+    Extent x{0, 0, 0};
+    const int gi = base + (threadIdx.x & 63);
+    if (gi < p.G) {
+      if constexpr (LAYOUT == kGroupsSizesM) {
+        x.size = static_cast<const int64_t*>(p.layout)[gi];
+      } else {
+        x.begin = gi ? static_cast<const int32_t*>(p.layout)[gi - 1] : 0;
+        x.end = static_cast<const int32_t*>(p.layout)[gi];
+      }
+    }
+    return x;
+  }
+  // `seen_bad` carries "an earlier group was inconsistent" from chunk to chunk: such a group and every group after it
+  // own no tiles, so the tile count, the XCD slices and the lookup all stop at the first bad group and every tile
+  // of the groups in front of it gets a workgroup (the grid is sized for consistent extents).
+  MSLK_AMD_DEVINL static Chunk chunk_of(const DeviceGroups& p, const Extent& x, int base, int& carry_len, bool& seen_bad) {
+    const int fixed_tiles = LAYOUT == kGroupsOffsetsN ? (p.M + BM - 1) / BM : (p.N + BN - 1) / BN;
+    const int blk = LAYOUT == kGroupsOffsetsN ? BN : BM;
+    const int64_t total = LAYOUT == kGroupsOffsetsN ? p.N : p.M;
+    const int lane = threadIdx.x & 63;
+    Chunk c;
+    const bool in = base + lane < p.G;
+    bool bad;
+    if constexpr (LAYOUT == kGroupsSizesM) {
+      bad = x.size < 0 || x.size > total;
+      c.len = bad ? 0 : (int)x.size;
+      const int end = saturating_sum(carry_len, wave_prefix_sum<true>(c.len));
+      c.start = end - c.len;
+      carry_len = __builtin_amdgcn_readlane(end, 63);
+      bad = bad || (in && (end > total || end == 0x7FFFFFFF));
+    } else {
+      const int64_t len64 = (int64_t)x.end - x.begin;
+      bad = len64 < 0 || x.begin < 0 || x.end > total;
+      c.start = x.begin;
+      c.len = bad ? 0 : (int)len64;
+    }
+    const unsigned long long bad_lanes = __ballot(bad);
+    const bool after_bad = seen_bad || (bad_lanes != 0 && lane >= __ffsll((long long)bad_lanes) - 1);
+    seen_bad = seen_bad || bad_lanes != 0;
+    c.tiles = (in && !after_bad) ? ((c.len + blk - 1) / blk) * fixed_tiles : 0;
+    c.incl = wave_prefix_sum<false>(c.tiles);
+    return c;
+  }
+  MSLK_AMD_DEVINL static int tiles_of(const Chunk& c) { return __builtin_amdgcn_readlane(c.incl, 63); }
+
+  MSLK_AMD_DEVINL void scan(const DeviceGroups& p) {
+    const Extent x0 = fetch(p, 0), x1 = fetch(p, 64);
+    int carry_len = 0;
+    bool seen_bad = false;
+    c0 = chunk_of(p, x0, 0, carry_len, seen_bad);
+    c1 = chunk_of(p, x1, 64, carry_len, seen_bad);   // no groups there: no tiles
+    carry_len2 = carry_len;
+    seen_bad2 = seen_bad;
+    total_tiles = (int64_t)tiles_of(c0) + tiles_of(c1);
+    for (int base = 128; base < p.G && !seen_bad; base += 64)
+      total_tiles += tiles_of(chunk_of(p, fetch(p, base), base, carry_len, seen_bad));
+    per_xcd = (total_tiles + kXcds - 1) / kXcds;
+  }
+  // Group, extent and place inside the group of tile `tile` < total_tiles of the list.
+  MSLK_AMD_DEVINL bool find(const DeviceGroups& p, int64_t tile, GroupSpan& sp) const {
+    int64_t carry_tiles = 0;
+    auto find_in = [&](const Chunk& c, int base) {
+      const int64_t excl = carry_tiles + c.incl - c.tiles;
+      const unsigned long long hit = __ballot(c.tiles > 0 && tile >= excl && tile < excl + c.tiles);
+      if (hit == 0) {
+        carry_tiles += tiles_of(c);
+        return false;
+      }
+      const int src = __ffsll((long long)hit) - 1;
+      // the results are the same in every lane: out of scalar registers, so that the tile's addresses live there
+      sp.gi = base + src;
+      sp.o0 = __builtin_amdgcn_readlane(c.start, src);
+      sp.len = __builtin_amdgcn_readlane(c.len, src);
+      sp.t = (int)(uniform64(tile - carry_tiles) - __builtin_amdgcn_readlane(c.incl - c.tiles, src));
+      return true;
+    };
+    if (find_in(c0, 0) || find_in(c1, 64)) return true;
+    int carry_len = carry_len2;
+    bool seen_bad = seen_bad2;
+    for (int base = 128; base < p.G && !seen_bad; base += 64)
+      if (find_in(chunk_of(p, fetch(p, base), base, carry_len, seen_bad), base)) return true;
+    return false;
+  }
+  // The same for a tile per lane (all lanes of the wavefront call it; `live`: the lane has a tile).
+  MSLK_AMD_DEVINL void find_lanes(const DeviceGroups& p, int tile, bool live, int& gi, int& start, int& len, int& t) const {
+    int carry_tiles = 0;
+    auto find_in = [&](const Chunk& c, int base) {
+      const int rel = tile - carry_tiles, n = tiles_of(c);
+      int pos = 0;   // groups of the chunk whose tiles end at or before `rel`
+#pragma unroll
+      for (int step = 32; step > 0; step >>= 1) pos += __shfl(c.incl, pos + step - 1, 64) <= rel ? step : 0;
+      const int s = __shfl(c.start, pos, 64), l = __shfl(c.len, pos, 64), before = __shfl(c.incl - c.tiles, pos, 64);
+      if (rel >= 0 && rel < n) { gi = base + pos; start = s; len = l; t = rel - before; }
+      carry_tiles += n;
+    };
+    gi = start = len = t = 0;
+    find_in(c0, 0);
+    if (p.G > 64) find_in(c1, 64);
+    int carry_len = carry_len2;
+    bool seen_bad = seen_bad2;
+    for (int base = 128; base < p.G && !seen_bad && __ballot(live && tile >= carry_tiles) != 0; base += 64)
+      find_in(chunk_of(p, fetch(p, base), base, carry_len, seen_bad), base);
+  }
+};
+
 template <int LAYOUT, int BM, int BN>
 MSLK_AMD_DEVINL bool find_group(const DeviceGroups& p, int t, GroupSpan& sp) {
   const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
@@ -176,98 +303,12 @@ MSLK_AMD_DEVINL bool find_group(const DeviceGroups& p, int t, GroupSpan& sp) {
       return true;
     }
   } else {
-    // The G extents are read 64 at a time, one per lane, and turned into tile ranges by a wave-level prefix sum, so the
-    // lookup costs one memory round trip for up to 128 groups (the first two chunks are fetched together and stay in
-    // registers) instead of G dependent ones.  A workgroup of 256 x 256 tiles holds its CU's whole LDS, so nothing else runs
-    // under its lookup (two of 128 x 128 share a CU): with more round trips for the groups beyond 64 and sums through LDS shuffles (a hundred cycles per step) 128 experts x
-    // 2048 x 768 took 65.5 us over 8192 rows and 120.0 over 32768 (now 56.3 and 114.8), 64 x 4096 x 1024 over 16384 128.4
-    // (120.1), 16 x 8192 x 5120 over 8192 324 (323).
-    // The total tile count is formed first: XCD x (workgroup id mod 8) then takes a contiguous slice of the tile list, so
-    // that the row tiles of a group that share a weight panel run on one XCD and find it in its L2 (without the slices the
-    // device-extent layouts fetched 1.6 times what the host-extent kernel fetches for the same 16 experts).
-    const int fixed_tiles = LAYOUT == kGroupsOffsetsN ? tiles_m : tiles_n;
-    const int blk = LAYOUT == kGroupsOffsetsN ? BN : BM;
-    const int64_t total = LAYOUT == kGroupsOffsetsN ? p.N : p.M;
-    const int lane = threadIdx.x & 63;
-    // Every quantity fits 32 bits (the host checks the dimensions and the grid): sizes beyond the tensor mark the group bad.
-    struct Extent { int64_t size; int begin, end; };
-    struct Chunk { int start, len, tiles, incl; unsigned long long bad; };
-    auto fetch = [&](int base) {
-      Extent x{0, 0, 0};
-      const int gi = base + lane;
-      if (gi < p.G) {
-        if constexpr (LAYOUT == kGroupsSizesM) {
-          x.size = static_cast<const int64_t*>(p.layout)[gi];
-        } else {
-          x.begin = gi ? static_cast<const int32_t*>(p.layout)[gi - 1] : 0;
-          x.end = static_cast<const int32_t*>(p.layout)[gi];
-        }
-      }
-      return x;
-    };
-    // `seen_bad` carries "an earlier group was inconsistent" from chunk to chunk: such a group and every group after it
-    // own no tiles, so the tile count, the XCD slices and the lookup all stop at the first bad group and every tile
-    // of the groups in front of it gets a workgroup (the grid is sized for consistent extents).
-    auto chunk_of = [&](const Extent& x, int base, int& carry_len, bool& seen_bad) {
-      Chunk c;
-      const bool in = base + lane < p.G;
-      bool bad;
-      if constexpr (LAYOUT == kGroupsSizesM) {
-        bad = x.size < 0 || x.size > total;
-        c.len = bad ? 0 : (int)x.size;
-        const int end = saturating_sum(carry_len, wave_prefix_sum<true>(c.len));
-        c.start = end - c.len;
-        carry_len = __builtin_amdgcn_readlane(end, 63);
-        bad = bad || (in && (end > total || end == 0x7FFFFFFF));
-      } else {
-        const int64_t len64 = (int64_t)x.end - x.begin;
-        bad = len64 < 0 || x.begin < 0 || x.end > total;
-        c.start = x.begin;
-        c.len = bad ? 0 : (int)len64;
-      }
-      c.bad = __ballot(bad);
-      const bool after_bad = seen_bad || (c.bad != 0 && lane >= __ffsll((long long)c.bad) - 1);
-      seen_bad = seen_bad || c.bad != 0;
-      c.tiles = (in && !after_bad) ? ((c.len + blk - 1) / blk) * fixed_tiles : 0;
-      c.incl = wave_prefix_sum<false>(c.tiles);
-      return c;
-    };
-    auto tiles_of = [&](const Chunk& c) { return __builtin_amdgcn_readlane(c.incl, 63); };
-    const Extent x0 = fetch(0), x1 = fetch(64);
-    int carry_len = 0;
-    bool seen_bad = false;
-    const Chunk c0 = chunk_of(x0, 0, carry_len, seen_bad);
-    const Chunk c1 = chunk_of(x1, 64, carry_len, seen_bad);   // no groups there: no tiles
-    const int carry_len2 = carry_len;
-    const bool seen_bad2 = seen_bad;
-    int64_t total_tiles = (int64_t)tiles_of(c0) + tiles_of(c1);
-    for (int base = 128; base < p.G && !seen_bad; base += 64) total_tiles += tiles_of(chunk_of(fetch(base), base, carry_len, seen_bad));
-    const int64_t per_xcd = (total_tiles + kXcds - 1) / kXcds;
+    BlockGroups<LAYOUT, BM, BN> groups;
+    groups.scan(p);
     const int64_t slot = t / kXcds;                       // `t` arrives as the workgroup id
-    const int64_t tile = (int64_t)(t % kXcds) * per_xcd + slot;
-    if (slot >= per_xcd || tile >= total_tiles) return false;
-    int64_t carry_tiles = 0;
-    auto find_in = [&](const Chunk& c, int base) {
-      const int64_t excl = carry_tiles + c.incl - c.tiles;
-      const unsigned long long hit = __ballot(c.tiles > 0 && tile >= excl && tile < excl + c.tiles);
-      if (hit == 0) {
-        carry_tiles += tiles_of(c);
-        return false;
-      }
-      const int src = __ffsll((long long)hit) - 1;
-      // the results are the same in every lane: out of scalar registers, so that the tile's addresses live there
-      sp.gi = base + src;
-      sp.o0 = __builtin_amdgcn_readlane(c.start, src);
-      sp.len = __builtin_amdgcn_readlane(c.len, src);
-      sp.t = (int)(uniform64(tile - carry_tiles) - __builtin_amdgcn_readlane(c.incl - c.tiles, src));
-      return true;
-    };
-    if (find_in(c0, 0) || find_in(c1, 64)) return true;
-    carry_len = carry_len2;
-    seen_bad = seen_bad2;
-    for (int base = 128; base < p.G && !seen_bad; base += 64)
-      if (find_in(chunk_of(fetch(base), base, carry_len, seen_bad), base)) return true;
-    return false;
+    const int64_t tile = (int64_t)(t % kXcds) * groups.per_xcd + slot;
+    if (slot >= groups.per_xcd || tile >= groups.total_tiles) return false;
+    return groups.find(p, tile, sp);
   }
 }
 
@@ -289,6 +330,118 @@ MSLK_AMD_DEVINL void slow_tile(const uint8_t* a, const uint8_t* b, const float* 
     if constexpr (BIAS == 2) v += bf16_bits_to_f32(static_cast<const uint16_t*>(bias)[n]);
     y[(int64_t)m * ldc + n] = (uint16_t)f32_to_bf16_bits(v);
   }
+}
+
+// 256 x 256 tiles of row groups: one workgroup per CU walks its share of the tile list, tile after tile in one chain of K steps
+// (GemmTile::chain_tile).
+using RowTileShape = TileShape<256, 256>;
+struct RowTile {
+  const uint8_t *a, *b;
+  const float *xs, *ws;
+  uint16_t* y;
+  int m_rem, n_rem;   // valid rows / columns from the tile's first
+  int N, K;           // row pitch of Y, bytes of an operand row
+  int stream;         // the only reader of its weight block at that time: weights fetched with non-temporal loads
+};
+
+// The tiles of one workgroup, found 64 at a time, one per lane: row and column, group and what is left of it.
+struct TileBatch {
+  int row, m_rem, col, group, stream, count;
+};
+
+// What the chain takes: 16-byte pieces of the rows of all operands, of the column scales and of Y, and three K steps.
+inline bool chain_takes(int64_t N, int64_t K, const void* xq, const void* wq, const void* ws, const void* y) {
+  const uintptr_t all = reinterpret_cast<uintptr_t>(xq) | reinterpret_cast<uintptr_t>(wq) | reinterpret_cast<uintptr_t>(ws) | reinterpret_cast<uintptr_t>(y);
+  return K > 2 * kBK && K % 16 == 0 && N % 8 == 0 && all % 16 == 0;
+}
+
+// `next(tile)` gives the tiles one after the other.
+template <typename Next>
+MSLK_AMD_DEVINL void walk_row_tiles(char* lds, Next&& next) {
+  using TS = RowTileShape;
+  using Plain = GemmTile<TS, 0, false, true, TS::LA / 2, false, false, true>;
+  using Streamed = GemmTile<TS, 0, false, true, TS::LA / 2, false, true, true>;
+  RowTile t, n;
+  if (!next(t)) return;
+  auto operands = [](const RowTile& w) { return TileOperands{w.a, w.b, w.m_rem, w.n_rem, w.K, (uint32_t)w.K}; };
+  Plain tile;
+  Streamed streamed;
+  TileChain<TS> chain(lds);
+  tile.chain_start(chain, operands(t));
+  for (;;) {
+    const bool more = next(n);
+    if (!more) n = t;   // its loads are issued once more, for nobody
+    const TileOperands o = operands(n);
+    // One K loop and epilogue per number of m fragments with valid rows and kind of weight loads: a common end for all would
+    // have the sums moved between registers.
+    auto run = [&](auto& build, auto fragments, auto all) {
+      constexpr int FMV = decltype(fragments)::value;
+      v4f acc[TS::FN][TS::FM];
+      TileScales<TS> scales;
+      build.template chain_tile<FMV>(chain, t.K, o, acc, scales, t.xs, t.ws, t.m_rem, t.n_rem);
+      build.template epilogue_direct<decltype(all)::value != 0, FMV>(acc, scales, t.y, t.m_rem, t.n_rem, t.N);
+    };
+    auto run_rows = [&](auto& build) {
+      constexpr int Q = TS::kBM / 4, FM = TS::FM;
+      if (t.m_rem >= TS::kBM && t.n_rem >= TS::kBN) run(build, Int<FM>(), Int<1>());
+      else if (t.m_rem > 3 * Q) run(build, Int<FM>(), Int<0>());
+      else if (t.m_rem > 2 * Q) run(build, Int<3 * FM / 4>(), Int<0>());
+      else if (t.m_rem > Q) run(build, Int<FM / 2>(), Int<0>());
+      else run(build, Int<FM / 4>(), Int<0>());
+    };
+    if (t.stream) {
+      streamed.adopt(tile);
+      run_rows(streamed);
+      tile.adopt(streamed);
+    } else {
+      run_rows(tile);
+    }
+    if (!more) break;
+    t = n;
+  }
+  wait_vmcnt0();   // no copy into LDS may outlive the workgroup
+}
+
+template <int LAYOUT>
+__global__ __launch_bounds__(256) void grouped_rows_kernel(DeviceGroups p) {
+  using TS = RowTileShape;
+  constexpr int BM = TS::kBM, BN = TS::kBN;
+  __shared__ __attribute__((aligned(1024))) char lds[TS::LDS_BYTES];
+  BlockGroups<LAYOUT, BM, BN> groups;
+  groups.scan(p);
+  const int stride = gridDim.x / kXcds, xcd = blockIdx.x % kXcds, per_xcd = (int)groups.per_xcd, total = (int)groups.total_tiles;
+  int slot = blockIdx.x / kXcds, i = 64;
+  TileBatch b;
+  walk_row_tiles(lds, [&](RowTile& w) {
+    if (i == 64) {
+      const int mine = slot + (int)(threadIdx.x & 63) * stride;   // (at most 2^31 tiles in all)
+      const bool live = mine < per_xcd && mine < total - xcd * per_xcd;
+      int start, len, t, tm, tn;
+      groups.find_lanes(p, live ? xcd * per_xcd + mine : 0, live, b.group, start, len, t);
+      b.stream = local_tile(t, len > 0 ? (len + BM - 1) / BM : 1, (p.N + BN - 1) / BN, tm, tn) == 1;
+      b.row = start + tm * BM;
+      b.m_rem = len - tm * BM;
+      b.col = tn * BN;
+      b.count = __popcll(__ballot(live));
+      slot += 64 * stride;
+      i = 0;
+    }
+    if (i >= b.count) return false;
+    const int64_t row = __builtin_amdgcn_readlane(b.row, i), col = __builtin_amdgcn_readlane(b.col, i);
+    const int64_t group = __builtin_amdgcn_readlane(b.group, i);
+    w.m_rem = __builtin_amdgcn_readlane(b.m_rem, i);
+    w.stream = __builtin_amdgcn_readlane(b.stream, i);
+    w.n_rem = p.N - (int)col;
+    w.a = p.xq + row * p.K;
+    w.b = p.wq + (group * p.N + col) * p.K;
+    w.xs = p.xs + row;
+    w.ws = p.ws + group * p.N + col;
+    w.y = p.y + row * p.N + col;
+    w.N = p.N;
+    w.K = p.K;
+    ++i;
+    return true;
+  });
 }
 
 template <int LAYOUT, int BM, int BN, int BIAS>
@@ -411,8 +564,14 @@ hipError_t launch_device_layout(const DeviceGroups& p, hipStream_t s) {
     const int64_t full_tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
     const bool short_k = p.K < 768 && full_tiles128 <= 2 * device_compute_units();
     if (launchable && (p.unaligned || short_k || small_row_groups(M, G, tiles128))) return launch_device_shape<LAYOUT, 128, 128, BIAS>(p, s);
+    const int64_t most_tiles = ((M + 255) / 256 + G) * ((N + 255) / 256);   // every group may end in a partial tile
+    if (M > 0 && most_tiles <= 2147483647 && chain_takes(N, p.K, p.xq, p.wq, p.ws, p.y)) {
+      const int64_t cus = device_compute_units(), wgs = (most_tiles + kXcds - 1) / kXcds * kXcds;
+      grouped_rows_kernel<LAYOUT><<<(unsigned)(wgs < cus ? wgs : cus), 256, 0, s>>>(p);
+      return hipGetLastError();
+    }
     return launch_device_shape<LAYOUT, 256, 256, BIAS>(p, s);
-  }
+  } else {
   // Tile shape from the average group: 256 x 256 once such tiles give every CU work.
   const int64_t Mg = p.M, Ng = LAYOUT == kGroupsOffsetsN ? (p.N + G - 1) / G : p.N;
   const int64_t big = G * ((Mg + 255) / 256) * ((Ng + 255) / 256);
@@ -420,6 +579,7 @@ hipError_t launch_device_layout(const DeviceGroups& p, hipStream_t s) {
   const bool use_big = big >= 192 && pad * 4 <= Mg * Ng * 5;   // at most 25 % padding
   if (use_big) return launch_device_shape<LAYOUT, 256, 256, BIAS>(p, s);
   return launch_device_shape<LAYOUT, 128, 128, BIAS>(p, s);
+  }
 }
 
 }  // namespace

@@ -62,6 +62,27 @@ struct TileShape {
   static constexpr int LB = BN / 8 / NW;
 };
 
+// Of GemmTile::chain_tile(): the buffers of the step at hand by role (TS: two XQ and three WQ buffers), ...
+template <typename TS>
+struct TileChain {
+  char *a_cur, *a_nxt, *b_cur, *b_nxt, *b_far;
+  MSLK_AMD_DEVINL explicit TileChain(char* lds) : a_cur(lds), a_nxt(lds + TS::A_BYTES), b_cur(lds + 2 * TS::A_BYTES),
+                                                  b_nxt(b_cur + TS::B_BYTES), b_far(b_nxt + TS::B_BYTES) {}
+  MSLK_AMD_DEVINL void advance() {
+    { char* t = a_cur; a_cur = a_nxt; a_nxt = t; }
+    { char* t = b_cur; b_cur = b_nxt; b_nxt = b_far; b_far = t; }
+  }
+};
+// ... the operands of one tile (first row of each, valid rows >= 1, bytes of a row to consume, bytes between rows) ...
+struct TileOperands {
+  const uint8_t *a, *b;
+  int rows_a, rows_b, K;
+  uint32_t ld;
+};
+// ... and the scales of a lane's sums.
+template <typename TS>
+struct TileScales { float ws[TS::FN][4], xs[TS::FM]; };
+
 MSLK_AMD_DEVINL int lds_swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 
 MSLK_AMD_DEVINL void wait_vmcnt0() { __builtin_amdgcn_s_waitcnt(0x0F70); }
@@ -96,6 +117,13 @@ typedef const __attribute__((address_space(1))) void* gbl_ptr_t;
 MSLK_AMD_DEVINL void store16_stream(uint16_t* dst, uint4 val) {
   const v4i v = {(int)val.x, (int)val.y, (int)val.z, (int)val.w};
   asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 1" : : "v"(dst), "v"(v) : "memory");
+}
+
+// The same left to the L2, which puts the two halves of a 128-byte line together (epilogue_direct writes 64 bytes of a row at a
+// time; past the L2 a grouped launch that stores much took up to 30 % longer: 64 x 512 rows x 2048 x 768 81 against 62 us).
+MSLK_AMD_DEVINL void store16(void* dst, uint4 val) {
+  const v4i v = {(int)val.x, (int)val.y, (int)val.z, (int)val.w};
+  asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1" : : "v"(dst), "v"(v) : "memory");
 }
 
 // Global -> LDS copy of 16 bytes per lane (1 KiB per wave, contiguous in LDS from `lds_wave_base`), addressed as
@@ -142,9 +170,13 @@ MSLK_AMD_DEVINL void dma16(const uint8_t* base, uint32_t off, char* lds_wave_bas
 // (mslk_amd_debug_gemm_phases) writes them out beside its own entry and exit times; no other kernel carries them.
 // W_STREAM: the weight tile is fetched with non-temporal loads (dma16<true>): for tiles whose weight block at most two row
 // tiles share.
+// DIRECT: the rows of a weight tile are dealt to the n fragments so that a lane holds eight consecutive columns of its row in
+// two neighbouring fragments, and the epilogue (epilogue_direct) stores them as they are, without a transpose through LDS:
+// fragment t takes rows 32 (t / 2) + 4 (t % 2) + 8 (i / 4) + i % 4 for i = 0 ... 15.  Row-major weights only.
 template <typename TS, int BIAS, bool PS = false, bool ROWSKIP = false, int XQ_EARLY = TS::LA / 2, bool STAMPS = false,
-          bool W_STREAM = false>
+          bool W_STREAM = false, bool DIRECT = false>
 struct GemmTile {
+  static_assert(!(DIRECT && PS), "the blocked layout fixes the rows of a fragment");
   // Per-lane state that is constant over the K loop.
   uint32_t a_off[TS::LA];   // byte offset of this lane's 16-byte chunk relative to a_base, k = 0
   uint32_t b_off[TS::LB];
@@ -152,6 +184,8 @@ struct GemmTile {
   uint64_t stamp_first_operands = 0, stamp_k_loop_end = 0;   // STAMPS only
   int a_rows = TS::kBM;     // valid rows of the XQ tile (wave-uniform)
   const uint8_t* a_base;    // XQ + m0 * K   (wave-uniform)
+  const uint8_t* a_base_hi; // the same for the XQ loads from number XQ_EARLY on (another tile's while chain_tile() changes over)
+  int a_rows_hi;
   const uint8_t* b_base;    // WQ + n0 * K
 
   // xq/wq point at row m0 / n0 of the operands; rows_a / rows_b = valid rows from there (>= 1).
@@ -163,14 +197,23 @@ struct GemmTile {
     // the tile pointers are the same in every lane; say so, so that the DMA loads get their base in scalar registers
     a_base = uniform_ptr(xq_tile);
     b_base = uniform_ptr(wq_tile);
-    a_rows = rows_a;
+    a_base_hi = a_base;
+    a_rows = a_rows_hi = rows_a;
+    offsets_a<0, TS::LA>(lane, wave, rows_a, ld);
+    offsets_b(lane, wave, rows_b, ld);
+  }
+  // Lane offsets of the XQ loads [LO, HI) / of the WQ loads of a tile.
+  template <int LO, int HI>
+  MSLK_AMD_DEVINL void offsets_a(int lane, int wave, int rows_a, uint32_t ld) {
 #pragma unroll
-    for (int i = 0; i < TS::LA; ++i) {
+    for (int i = LO; i < HI; ++i) {
       const int row = (wave * TS::LA + i) * 8 + (lane >> 3);
       const int chunk = (lane & 7) ^ lds_swz(row);
       const int rc = row < rows_a ? row : rows_a - 1;   // clamp: edge tiles re-read the last row
       a_off[i] = (uint32_t)rc * ld + chunk * 16;
     }
+  }
+  MSLK_AMD_DEVINL void offsets_b(int lane, int wave, int rows_b, uint32_t ld) {
 #pragma unroll
     for (int i = 0; i < TS::LB; ++i) {
       if constexpr (PS) {
@@ -181,7 +224,7 @@ struct GemmTile {
         b_off[i] = (uint32_t)nb * 16u * ld + (q & 1) * 1024 + lane * 16;
       } else {
         const int row = (wave * TS::LB + i) * 8 + (lane >> 3);
-        const int chunk = (lane & 7) ^ lds_swz(row);
+        const int chunk = (lane & 7) ^ swz_b(row);
         const int rc = row < rows_b ? row : rows_b - 1;
         b_off[i] = (uint32_t)rc * ld + chunk * 16;
       }
@@ -194,7 +237,7 @@ struct GemmTile {
   // DMA load number i (0 .. LA-1 for the XQ tile, 0 .. LB-1 for the WQ tile) of the K step at byte k0.
   // `abuf` / `bbuf` are the LDS buffers that receive the XQ / WQ tile of the K step at byte k0.
   MSLK_AMD_DEVINL void issue_a(char* abuf, int k0, int i) {
-    dma16(a_base + k0, a_off[i], abuf + (wave_id() * TS::LA + i) * 1024);
+    dma16((i < XQ_EARLY ? a_base : a_base_hi) + k0, a_off[i], abuf + (wave_id() * TS::LA + i) * 1024);
   }
   MSLK_AMD_DEVINL void issue_b(char* bbuf, int k0, int i) {
     // pre-shuffled: the K step at byte k0 starts 16 rows x k0 bytes into the row group
@@ -207,7 +250,7 @@ struct GemmTile {
   // Ragged tiles: a wave whose share of the XQ tile (8 * LA consecutive rows) starts beyond the valid rows fetches
   // nothing -- nobody multiplies those rows (one wave-uniform branch for the wave's loads of a step).
   MSLK_AMD_DEVINL void issue_a_live(char* abuf, int k0, int lo = 0, int hi = TS::LA) {
-    if (wave_id() * TS::LA * 8 < a_rows) {
+    if (wave_id() * TS::LA * 8 < (lo < XQ_EARLY ? a_rows : a_rows_hi)) {   // (a chain asks for both parts apart)
 #pragma unroll
       for (int i = 0; i < TS::LA; ++i)
         if (i >= lo && i < hi) issue_a(abuf, k0, i);
@@ -233,12 +276,22 @@ struct GemmTile {
 #pragma unroll
     for (int i = 0; i < TS::LB; ++i) {
       const int row = (wave * TS::LB + i) * 8 + (lane >> 3);
-      const int chunk = (lane & 7) ^ lds_swz(row);
+      const int chunk = (lane & 7) ^ swz_b(row);
       char* dst = bbuf + (wave * TS::LB + i) * 1024;
       const bool valid = PS ? ((wave * TS::LB + i) & 1) * 64 < k_valid : chunk * 16 < k_valid;
       if (valid) dma16<W_STREAM>(b_base + (PS ? k0 * 16 : k0), b_off[i], dst);
       else *reinterpret_cast<uint4*>(dst + lane * 16) = make_uint4(0, 0, 0, 0);
     }
+  }
+
+  // Chunk permutation of the WQ tile.  DIRECT: the 16 rows of a fragment differ in bits 0, 1, 3 and 4.  A 16-byte read is served
+  // 16 lanes at a time, but not 16 consecutive ones: rows with equal bits 3 and 4 at one chunk together with the other rows at
+  // the chunk two further (lanes 0 - 3, 12 - 15, 20 - 27 first).  With bits 3 and 4 simply side by side above bit 1 two rows of such a set shared their
+  // banks and a K step took 8 % longer.
+  MSLK_AMD_DEVINL static int swz_b(int row) {
+    if constexpr (!DIRECT) return lds_swz(row);
+    const int r3 = (row >> 3) & 1, r4 = (row >> 4) & 1;
+    return ((row >> 1) & 1) | (r4 << 1) | ((r3 ^ r4) << 2);
   }
 
   // LDS byte offsets of this lane's two 16-byte halves of an MFMA operand fragment, relative to the
@@ -264,12 +317,19 @@ struct GemmTile {
   MSLK_AMD_DEVINL static v8i load_frag_a(const char* tile, int t, FragOff fo) {
     return load_frag<(ILV ? TS::WM : 1) * 16 * kBK>(tile, t, fo);
   }
-  // WQ fragment t of the wave: as load_frag, or lane-linear out of the two 1 KiB blocks of row group t.
+  // WQ fragment t of the wave: as load_frag (DIRECT: with its own rows), or lane-linear out of the two 1 KiB blocks of row group t.
   MSLK_AMD_DEVINL static v8i load_frag_b(const char* tile, int t, FragOff fo) {
     if constexpr (PS) {
       const char* blk = tile + t * 2048 + (threadIdx.x & 63) * 16;
       const v4i lo = *reinterpret_cast<const v4i*>(blk);
       const v4i hi = *reinterpret_cast<const v4i*>(blk + 1024);
+      return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    } else if constexpr (DIRECT) {
+      const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+      const int row = (i >> 2) * 8 + (i & 3), s = swz_b(row);   // the further rows of a tile do not change the permutation
+      const char* at = tile + (t >> 1) * 32 * kBK + (t & 1) * 4 * kBK + row * kBK;
+      const v4i lo = *reinterpret_cast<const v4i*>(at + (((2 * g) ^ s) << 4));
+      const v4i hi = *reinterpret_cast<const v4i*>(at + (((2 * g + 1) ^ s) << 4));
       return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     } else {
       return load_frag(tile, t, fo);
@@ -333,23 +393,28 @@ struct GemmTile {
   //     into `a_dst` != `a_nxt`, and PENDING, the number of this wave's youngest loads that may still be in
   //     flight at the barrier, covers RING - 2 steps.
   // FMV < FM: a ragged tile, only the first FMV m fragments of every wave hold valid rows -- see step_rows().
-  template <int NA_HEAD, bool DMA_B, bool NEXT, int PENDING, int FMV = TS::FM, int NA_TAIL = 0>
+  // FIRST: the sums start here (acc is only written).
+  template <int NA_HEAD, bool DMA_B, bool NEXT, int PENDING, int FMV = TS::FM, int NA_TAIL = 0, bool FIRST = false>
   MSLK_AMD_DEVINL void step(const char* b_cur, char* a_dst, const char* a_nxt, const char* b_nxt, char* b_far, int k_a,
                             int k_b, v4f (&acc)[TS::FN][TS::FM], v8i (&xf)[TS::FM], v8i& wf0, char* a_tail_dst = nullptr,
                             int k_a_tail = 0) {
     static_assert(NA_HEAD >= 0 && NA_TAIL >= 0 && NA_HEAD <= TS::LA && NA_TAIL <= TS::LA && (NA_TAIL == 0 || NEXT), "XQ loads of a step");
     if constexpr (FMV < TS::FM) {
-      step_rows<NA_HEAD, DMA_B, NEXT, PENDING, FMV, NA_TAIL>(b_cur, a_dst, a_nxt, b_nxt, b_far, k_a, k_b, acc, xf, wf0, a_tail_dst, k_a_tail);
+      step_rows<NA_HEAD, DMA_B, NEXT, PENDING, FMV, NA_TAIL, FIRST>(b_cur, a_dst, a_nxt, b_nxt, b_far, k_a, k_b, acc, xf, wf0, a_tail_dst, k_a_tail);
       return;
     }
     v8i wf_last;
-    step_head<NA_HEAD, DMA_B>(b_cur, a_dst, b_far, k_a, k_b, acc, xf, wf0, wf_last);
-    step_tail<NEXT, PENDING, NA_TAIL>(a_nxt, b_nxt, acc, xf, wf0, wf_last, a_tail_dst, k_a_tail);
+    step_head<NA_HEAD, DMA_B, FIRST>(b_cur, a_dst, b_far, k_a, k_b, acc, xf, wf0, wf_last);
+    step_tail<NEXT, PENDING, NA_TAIL, FIRST>(a_nxt, b_nxt, acc, xf, wf0, wf_last, a_tail_dst, k_a_tail);
   }
 
   // The part of a full-tile K step in front of its barrier: every n fragment but the last, with the step's DMA loads.
   // Leaves the last WQ fragment of the step in `wf_last`.
-  template <int NA_HEAD, bool DMA_B>
+  template <bool FIRST>
+  MSLK_AMD_DEVINL static void multiply(const v8i& wf, const v8i& xf, v4f& acc) {
+    acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, xf, FIRST ? v4f{0.f, 0.f, 0.f, 0.f} : acc, 0, 0, 0, 0, 0, 0);
+  }
+  template <int NA_HEAD, bool DMA_B, bool FIRST = false>
   MSLK_AMD_DEVINL void step_head(const char* b_cur, char* a_dst, char* b_far, int k_a, int k_b, v4f (&acc)[TS::FN][TS::FM],
                                  v8i (&xf)[TS::FM], const v8i& wf0, v8i& wf_last) {
     constexpr int HALF = TS::FN / 2;
@@ -377,7 +442,7 @@ struct GemmTile {
       v8i wf_next;
 #pragma unroll
       for (int tm = 0; tm < TS::FM; ++tm) {
-        acc[tn][tm] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, xf[tm], acc[tn][tm], 0, 0, 0, 0, 0, 0);
+        multiply<FIRST>(wf, xf[tm], acc[tn][tm]);
         if (tm == 0) wf_next = load_frag_b(b_tile, tn + 1, fo);
         if constexpr (SPREAD) {
           // Large tiles (at most one load per MFMA): the loads of a step are spread over ALL groups in front of the
@@ -403,7 +468,7 @@ struct GemmTile {
 
   // The rest of the step: the barrier (NEXT), then the last n fragment, whose XQ fragments are replaced by those of the
   // next step as they retire; A_TAIL: the XQ tile at byte k_a goes into `a_free`, one load behind each MFMA.
-  template <bool NEXT, int PENDING, int NA_TAIL = 0>
+  template <bool NEXT, int PENDING, int NA_TAIL = 0, bool FIRST = false>
   MSLK_AMD_DEVINL void step_tail(const char* a_nxt, const char* b_nxt, v4f (&acc)[TS::FN][TS::FM], v8i (&xf)[TS::FM], v8i& wf0,
                                  const v8i& wf_last, char* a_free = nullptr, int k_a = 0) {
     const FragOff fo = frag_off();
@@ -414,7 +479,7 @@ struct GemmTile {
     const char* a_next = a_tile_of<false>(a_nxt);
 #pragma unroll
     for (int tm = 0; tm < TS::FM; ++tm) {
-      acc[TS::FN - 1][tm] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf_last, xf[tm], acc[TS::FN - 1][tm], 0, 0, 0, 0, 0, 0);
+      multiply<FIRST>(wf_last, xf[tm], acc[TS::FN - 1][tm]);
       if constexpr (NA_TAIL > 0) {   // the first NA_TAIL loads of the XQ tile, spread over the MFMAs
 #pragma unroll
         for (int q = (tm * NA_TAIL + TS::FM - 1) / TS::FM; q < ((tm + 1) * NA_TAIL + TS::FM - 1) / TS::FM; ++q) issue_a(a_free, k_a, q);
@@ -431,7 +496,7 @@ struct GemmTile {
   // the WQ loads follow the first MFMA group as one block and the XQ loads (left out by waves whose rows are all beyond
   // the valid ones) the first MFMA behind the barrier.  Such a step is short: it waits for memory rather than for the
   // matrix cores, so the fine interleave of step() would buy nothing.
-  template <int NA_HEAD, bool DMA_B, bool NEXT, int PENDING, int FMV, int NA_TAIL>
+  template <int NA_HEAD, bool DMA_B, bool NEXT, int PENDING, int FMV, int NA_TAIL, bool FIRST = false>
   MSLK_AMD_DEVINL void step_rows(const char* b_cur, char* a_dst, const char* a_nxt, const char* b_nxt, char* b_far, int k_a,
                                  int k_b, v4f (&acc)[TS::FN][TS::FM], v8i (&xf)[TS::FM], v8i& wf0, char* a_tail_dst, int k_a_tail) {
     static_assert(TS::FN >= 3 && FMV >= 1 && FMV < TS::FM, "ragged step");
@@ -442,8 +507,7 @@ struct GemmTile {
     for (int tn = 0; tn < TS::FN - 1; ++tn) {
       const v8i wf_next = load_frag_b(b_tile, tn + 1, fo);
 #pragma unroll
-      for (int tm = 0; tm < FMV; ++tm)
-        acc[tn][tm] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, xf[tm], acc[tn][tm], 0, 0, 0, 0, 0, 0);
+      for (int tm = 0; tm < FMV; ++tm) multiply<FIRST>(wf, xf[tm], acc[tn][tm]);
       if (tn == 0) {
         if constexpr (NA_HEAD > 0) issue_a_live(a_dst, k_a, TS::LA - NA_HEAD, TS::LA);   // older than the WQ loads of the step
         if constexpr (DMA_B) issue_b_all(b_far, k_b);
@@ -458,7 +522,7 @@ struct GemmTile {
     const char* a_next = a_tile_of<true>(a_nxt);
 #pragma unroll
     for (int tm = 0; tm < FMV; ++tm) {
-      acc[TS::FN - 1][tm] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, xf[tm], acc[TS::FN - 1][tm], 0, 0, 0, 0, 0, 0);
+      multiply<FIRST>(wf, xf[tm], acc[TS::FN - 1][tm]);
       if constexpr (NA_TAIL > 0) {
         if (tm == 0) issue_a_live(a_tail_dst, k_a_tail, 0, NA_TAIL);
       }
@@ -709,6 +773,187 @@ struct GemmTile {
       step<0, false, false, 0, FMV>(b_tail, a_tail, a_tail, b_tail, b_tail, 0, 0, acc, xf, wf0);
     }
     __syncthreads();  // the stages are dead from here on: the epilogue reuses LDS as a transpose buffer
+  }
+
+  // ---- Tiles one after the other without a gap (two-plus-three buffers, DIRECT, K > 2 kBK, K % 16 == 0) ----
+  // The K steps of consecutive tiles form one chain: the last two steps of a tile issue the first loads of the next one in the
+  // places where the steps before them issue the loads of their own tile, so a tile starts with its first operands in LDS.  The
+  // epilogue touches no LDS and runs while the next tile's loads land.
+  // A K that is no multiple of the step ends in a step over the last kBK bytes of the rows: what the step before has
+  // consumed already is cleared in the fragments of both operands.
+  using Chain = TileChain<TS>;
+  using Scales = TileScales<TS>;
+
+  // Takes over the addresses of a tile of another build (weights streamed or not).
+  template <typename Other>
+  MSLK_AMD_DEVINL void adopt(const Other& o) {
+#pragma unroll
+    for (int i = 0; i < TS::LA; ++i) a_off[i] = o.a_off[i];
+#pragma unroll
+    for (int i = 0; i < TS::LB; ++i) b_off[i] = o.b_off[i];
+    a_base = o.a_base; a_base_hi = o.a_base_hi; b_base = o.b_base;
+    a_rows = o.a_rows; a_rows_hi = o.a_rows_hi;
+  }
+
+  // The state a tile of the chain starts from: XQ and WQ of step 0 in LDS, WQ and the first XQ_EARLY loads of XQ of step 1 in flight.
+  MSLK_AMD_DEVINL void chain_start(const Chain& c, const TileOperands& o) {
+    init(o.a, o.b, o.rows_a < TS::kBM ? o.rows_a : TS::kBM, o.rows_b < TS::kBN ? o.rows_b : TS::kBN, o.ld);
+    issue_a_all(c.a_cur, 0);
+    issue_b_all(c.b_cur, 0);
+    issue_b_all(c.b_nxt, kBK);
+#pragma unroll
+    for (int i = 0; i < XQ_EARLY; ++i) issue_a(c.a_nxt, kBK, i);
+    wait_and_barrier<TS::LB + XQ_EARLY>();
+  }
+
+  // K loop of one tile, then the state above for tile `n`.  `scales` are loaded under the last step (ILV as in the epilogue).
+  template <int FMV>
+  MSLK_AMD_DEVINL void chain_tile(Chain& c, int K, const TileOperands& n, v4f (&acc)[TS::FN][TS::FM], Scales& scales,
+                                  const float* xs, const float* ws, int m_rem, int n_rem) {
+    static_assert(DIRECT && TS::RING == 0 && ROWSKIP, "chained tiles");
+    constexpr int XT = XQ_EARLY, XH = TS::LA - XT;
+    const int KT = (K + kBK - 1) / kBK, k_last = K - kBK;
+    v8i xf[TS::FM], wf0;
+    load_first_frags<FMV>(c.a_cur, c.b_cur, xf, wf0);
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    const int wave = wave_id(), rows_a = n.rows_a < TS::kBM ? n.rows_a : TS::kBM;
+    step<XH, true, true, TS::LB, FMV, XT, true>(c.b_cur, c.a_nxt, c.a_nxt, c.b_nxt, c.b_far, kBK, 2 * kBK < k_last ? 2 * kBK : k_last, acc,
+                                                xf, wf0, c.a_cur, 2 * kBK < k_last ? 2 * kBK : k_last);
+    c.advance();
+    int kt = 1;
+    do {
+      const int k1 = (kt + 1) * kBK < k_last ? (kt + 1) * kBK : k_last;
+      int k2 = (kt + 2) * kBK < k_last ? (kt + 2) * kBK : k_last;
+      if (kt == KT - 2) {   // WQ and the early XQ loads are those of the next tile
+        k2 = 0;
+        a_base = uniform_ptr(n.a);
+        b_base = uniform_ptr(n.b);
+        a_rows = rows_a;
+        offsets_a<0, XT>(lane, wave, rows_a, n.ld);
+        offsets_b(lane, wave, n.rows_b < TS::kBN ? n.rows_b : TS::kBN, n.ld);
+      }
+      step<XH, true, true, TS::LB, FMV, XT>(c.b_cur, c.a_nxt, c.a_nxt, c.b_nxt, c.b_far, k1, k2, acc, xf, wf0, c.a_cur, k2);
+      c.advance();
+    } while (++kt < KT - 1);
+    // last step: the rest of the next tile's first XQ tile in front of the barrier, its second step's loads behind it
+    a_base_hi = a_base;
+    a_rows_hi = a_rows;
+    offsets_a<XT, TS::LA>(lane, wave, rows_a, n.ld);
+    load_scales<(FMV < TS::FM)>(scales, xs, ws, m_rem, n_rem);
+    const int drop = (KT * kBK - K) >> 4;   // chunks of this step that the one before has consumed
+    const int g = lane >> 4;
+    const int keep0 = 2 * g >= drop ? -1 : 0, keep1 = 2 * g + 1 >= drop ? -1 : 0;
+    auto kept = [&](v8i f) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        f[e] &= keep0;
+        f[4 + e] &= keep1;
+      }
+      return f;
+    };
+    const FragOff fo = frag_off();
+    const char* b_tile = b_tile_of(c.b_cur);
+#pragma unroll
+    for (int tm = 0; tm < FMV; ++tm) xf[tm] = kept(xf[tm]);
+    v8i wf = kept(wf0);
+#pragma unroll
+    for (int tn = 0; tn < TS::FN - 1; ++tn) {
+      v8i wf_next;
+#pragma unroll
+      for (int tm = 0; tm < FMV; ++tm) {
+        acc[tn][tm] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, xf[tm], acc[tn][tm], 0, 0, 0, 0, 0, 0);
+        if (tm == 0) wf_next = load_frag_b(b_tile, tn + 1, fo);
+        if (tm == FMV - 1) {
+          if constexpr (FMV < TS::FM) {
+            if (tn == 0) issue_a_live(c.a_nxt, 0, XT, TS::LA);
+          } else {
+            if (tn < XH) issue_a(c.a_nxt, 0, XT + tn);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      wf = kept(wf_next);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    static_assert(XH <= TS::FN - 1, "one XQ load per fragment");
+    wait_and_barrier<0>();
+    constexpr int NL = TS::LB + XT;
+#pragma unroll
+    for (int tm = 0; tm < FMV; ++tm) {
+      acc[TS::FN - 1][tm] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, xf[tm], acc[TS::FN - 1][tm], 0, 0, 0, 0, 0, 0);
+#pragma unroll
+      for (int q = tm * NL / FMV; q < (tm + 1) * NL / FMV; ++q) {
+        if (q < TS::LB) issue_b(c.b_far, kBK, q);
+        else issue_a(c.a_cur, kBK, q - TS::LB);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    c.advance();
+  }
+
+  // DIRECT: row of fragment row tm that this lane stores, and its first column of the fragment pair 2 t, 2 t + 1
+  template <bool ILV>
+  MSLK_AMD_DEVINL static int direct_row(int tm) {
+    const int wm = wave_id() / TS::WN;
+    return ILV ? (tm * TS::WM + wm) * 16 : wm * (TS::kBM / TS::WM) + tm * 16;
+  }
+  template <bool ILV>
+  MSLK_AMD_DEVINL void load_scales(Scales& sc, const float* xs, const float* ws, int m_rem, int n_rem) {
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    const int j = lane & 15, n_base = (wave_id() % TS::WN) * (TS::kBN / TS::WN) + 8 * (lane >> 4);
+#pragma unroll
+    for (int t = 0; t < TS::FN / 2; ++t) {   // eight columns are valid or beyond the end together
+      const int n = n_base + t * 32 < n_rem ? n_base + t * 32 : 0;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const float4 w4 = *reinterpret_cast<const float4*>(ws + n + 4 * h);
+        float (&o)[4] = sc.ws[2 * t + h];
+        o[0] = w4.x; o[1] = w4.y; o[2] = w4.z; o[3] = w4.w;
+      }
+    }
+#pragma unroll
+    for (int tm = 0; tm < TS::FM; ++tm) {
+      const int m = direct_row<ILV>(tm) + j;
+      sc.xs[tm] = xs[m < m_rem ? m : m_rem - 1];
+    }
+  }
+
+  // Scale, convert and store the tile; y at its first row and column, N elements between rows.  ALL: every row and column of
+  // the tile is valid.  N % 8 == 0, y and the column scales aligned to 16 bytes.
+  // FMV < FM: only that many m fragments of a wave have valid rows, dealt to the wave rows round-robin.
+  template <bool ALL, int FMV>
+  MSLK_AMD_DEVINL void epilogue_direct(v4f (&acc)[TS::FN][TS::FM], const Scales& sc, uint16_t* y, int m_rem, int n_rem, int N) {
+    constexpr bool ILV = FMV < TS::FM;
+    static_assert(TS::FM * TS::FN * 4 >= 256 && BIAS == 0, "tiles whose sums fill the accumulator registers");
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    const int j = lane & 15, n_base = (wave_id() % TS::WN) * (TS::kBN / TS::WN) + 8 * (lane >> 4);
+    const uint32_t lane_off = ((uint32_t)j * (uint32_t)N + (uint32_t)n_base) * 2u;   // bytes; 16 N < 2^31
+#pragma unroll
+    for (int tm = 0; tm < FMV; ++tm) {
+      const int row0 = direct_row<ILV>(tm);
+      if (!ALL && row0 >= m_rem) continue;   // no valid row in this fragment (wave-uniform)
+      char* const row = reinterpret_cast<char*>(y + (int64_t)row0 * N);
+#pragma unroll
+      for (int t = 0; t < TS::FN / 2; ++t) {
+        uint32_t w[4];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          float v[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            v[r] = (acc[2 * t + h][tm][r] * sc.ws[2 * t + h][r]) * sc.xs[tm];   // the order of the reference's epilogue (fp8_rowwise_common.h:66)
+          }
+          w[2 * h] = pack_out_x2<false>(v[0], v[1]);
+          w[2 * h + 1] = pack_out_x2<false>(v[2], v[3]);
+        }
+        if (ALL || (row0 + j < m_rem && n_base + t * 32 < n_rem))
+          store16(row + lane_off + t * 64, make_uint4(w[0], w[1], w[2], w[3]));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
   }
 
   // Epilogue.  A lane's accumulators of one 16-row m fragment are 4 consecutive n in each of the
