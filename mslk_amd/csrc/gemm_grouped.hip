@@ -59,30 +59,40 @@ __global__ __launch_bounds__(256) void grouped_tiled_kernel(GroupTable tab) {
   }
 }
 
-// 256 x 256 tiles: one workgroup per CU walks the slice of its XCD.
-__global__ __launch_bounds__(256) void grouped_listed_kernel(GroupTable tab) {
+// 256 x 256 tiles: `wgs` workgroups per XCD walk the full passes of its slice; up to as many more take what is left.
+__global__ __launch_bounds__(256) void grouped_listed_kernel(GroupTable tab, int wgs) {
   using TS = RowTileShape;
   constexpr int BM = TS::kBM, BN = TS::kBN;
   __shared__ __attribute__((aligned(1024))) char lds[TS::LDS_BYTES];
-  const int xcd = blockIdx.x % kXcds, begin = tab.xcd_begin[xcd], end = tab.xcd_begin[xcd + 1], stride = gridDim.x / kXcds;
+  const int xcd = blockIdx.x % kXcds, begin = tab.xcd_begin[xcd], tiles = tab.xcd_begin[xcd + 1] - begin;
   const int lane = threadIdx.x & 63;
   const int first = lane < tab.count ? tab.g[lane].tile_begin : 0x7FFFFFFF;   // of group `lane`
-  int slot = blockIdx.x / kXcds, i = 64;
+  const SliceShares shares(tiles, wgs);
+  int slot = blockIdx.x / kXcds, end = shares.walked, piece = 0;
+  const bool rest = slot >= wgs;
+  if (rest) {
+    piece = (slot - wgs) % shares.pieces;
+    slot = shares.walked + (slot - wgs) / shares.pieces;
+    end = slot < tiles ? slot + 1 : slot;
+  }
   TileBatch b;
-  walk_row_tiles(lds, [&](RowTile& w) {
+  int i = 64;
+  auto next = [&](RowTile& w) {
     if (i == 64) {
-      const int t = begin + slot + lane * stride;
+      const int mine = slot + lane * wgs;
+      const bool live = mine < end;
+      const int t = live ? begin + mine : 0;
       int gi = 0;   // the last group that begins at or before t
 #pragma unroll
       for (int step = 32; step > 0; step >>= 1) gi += __shfl(first, gi + step, 64) <= t ? step : 0;
       const GroupDesc& d = tab.g[gi];
       int tm, tn;
-      b.stream = local_tile(t < end ? t - d.tile_begin : 0, (d.M + BM - 1) / BM, (d.N + BN - 1) / BN, tm, tn) == 1;
+      b.stream = local_tile(t - d.tile_begin, (d.M + BM - 1) / BM, (d.N + BN - 1) / BN, tm, tn) == 1;
       b.row = tm * BM;
       b.col = tn * BN;
       b.group = gi;
-      b.count = __popcll(__ballot(t < end));
-      slot += 64 * stride;
+      b.count = __popcll(__ballot(live));
+      slot += 64 * wgs;
       i = 0;
     }
     if (i >= b.count) return false;
@@ -90,7 +100,13 @@ __global__ __launch_bounds__(256) void grouped_listed_kernel(GroupTable tab) {
     w.stream = __builtin_amdgcn_readlane(b.stream, i);
     ++i;
     return true;
-  });
+  };
+  if (rest && shares.pieces > 1) {
+    RowTile t;
+    if (next(t)) run_quarter_tile(lds, t, piece);
+  } else {
+    walk_row_tiles(lds, next);
+  }
 }
 
 }  // namespace
@@ -229,7 +245,8 @@ static hipError_t launch_grouped_shape(const GroupTable& in, hipStream_t s) {
     bool chain = true;
     for (int i = 0; i < n; ++i) chain = chain && chain_takes(t.g[i].N, t.g[i].K, t.g[i].xq, t.g[i].wq, t.g[i].ws, t.g[i].y);
     if (chain) {
-      grouped_listed_kernel<<<(longest < wgs_per_xcd ? longest : wgs_per_xcd) * kXcds, 256, 0, s>>>(t);
+      if (longest <= wgs_per_xcd) grouped_listed_kernel<<<longest * kXcds, 256, 0, s>>>(t, longest);
+      else grouped_listed_kernel<<<2 * wgs_per_xcd * kXcds, 256, 0, s>>>(t, wgs_per_xcd);
       return hipGetLastError();
     }
   }

@@ -344,6 +344,22 @@ struct RowTile {
   int stream;         // the only reader of its weight block at that time: weights fetched with non-temporal loads
 };
 
+// Division of the `tiles` tiles of an XCD among its `wgs` workgroups.  The first `wgs` workgroups walk the full passes, entry i of
+// the slice going to workgroup i % wgs.  What is left over for a last pass, as long as it is at most three quarters of one, is
+// given to further workgroups, one tile each, which the hardware starts where one of the first ones ends: tiles cost what their
+// rows cost, and the workgroups that were given cheap ones take what is left.  At most a quarter of a pass is cut into quarters of tiles besides.
+// (16 experts x 5120 x 4096 over 8192 rows, 780 tiles: a fourth pass with 12 of 256 workgroups busy, 198 -> 156 us.)
+struct SliceShares {
+  int walked;        // entries of the slice that the first workgroups walk
+  int pieces;        // of a left-over tile: 1 or 4
+  MSLK_AMD_DEVINL SliceShares(int tiles, int wgs) {
+    const int left = tiles % wgs;
+    const bool apart = tiles > wgs && left * 4 <= wgs * 3;
+    walked = apart ? tiles - left : tiles;
+    pieces = left * 4 <= wgs ? 4 : 1;
+  }
+};
+
 // The tiles of one workgroup, found 64 at a time, one per lane: row and column, group and what is left of it.
 struct TileBatch {
   int row, m_rem, col, group, stream, count;
@@ -353,6 +369,16 @@ struct TileBatch {
 inline bool chain_takes(int64_t N, int64_t K, const void* xq, const void* wq, const void* ws, const void* y) {
   const uintptr_t all = reinterpret_cast<uintptr_t>(xq) | reinterpret_cast<uintptr_t>(wq) | reinterpret_cast<uintptr_t>(ws) | reinterpret_cast<uintptr_t>(y);
   return K > 2 * kBK && K % 16 == 0 && N % 8 == 0 && all % 16 == 0;
+}
+
+// One of four pieces of a tile, by a workgroup of its own.
+MSLK_AMD_DEVINL void run_quarter_tile(char* lds, const RowTile& t, int piece) {
+  using TS = TileShape<128, 128, 2, 2, 5>;
+  const int row = (piece & 1) * 128, col = (piece >> 1) * 128;
+  if (row >= t.m_rem || col >= t.n_rem) return;
+  GemmTile<TS, 0> tile;
+  tile.run(lds, t.a + (int64_t)row * t.K, t.b + (int64_t)col * t.K, t.xs + row, t.ws + col, nullptr, t.y + (int64_t)row * t.N + col,
+           t.m_rem - row, t.n_rem - col, t.N, t.K);
 }
 
 // `next(tile)` gives the tiles one after the other.
@@ -402,20 +428,30 @@ MSLK_AMD_DEVINL void walk_row_tiles(char* lds, Next&& next) {
   wait_vmcnt0();   // no copy into LDS may outlive the workgroup
 }
 
+// `wgs`: workgroups per XCD that walk the full passes; up to as many more of them take what is left.
 template <int LAYOUT>
-__global__ __launch_bounds__(256) void grouped_rows_kernel(DeviceGroups p) {
+__global__ __launch_bounds__(256) void grouped_rows_kernel(DeviceGroups p, int wgs) {
   using TS = RowTileShape;
   constexpr int BM = TS::kBM, BN = TS::kBN;
   __shared__ __attribute__((aligned(1024))) char lds[TS::LDS_BYTES];
   BlockGroups<LAYOUT, BM, BN> groups;
   groups.scan(p);
-  const int stride = gridDim.x / kXcds, xcd = blockIdx.x % kXcds, per_xcd = (int)groups.per_xcd, total = (int)groups.total_tiles;
-  int slot = blockIdx.x / kXcds, i = 64;
+  const int xcd = blockIdx.x % kXcds, per_xcd = (int)groups.per_xcd, left = (int)groups.total_tiles - xcd * per_xcd;
+  const int tiles = left < per_xcd ? left : per_xcd;
+  const SliceShares shares(tiles, wgs);
+  int slot = blockIdx.x / kXcds, end = shares.walked, piece = 0;
+  const bool rest = slot >= wgs;
+  if (rest) {
+    piece = (slot - wgs) % shares.pieces;
+    slot = shares.walked + (slot - wgs) / shares.pieces;
+    end = slot < tiles ? slot + 1 : slot;
+  }
   TileBatch b;
-  walk_row_tiles(lds, [&](RowTile& w) {
+  int i = 64;
+  auto next = [&](RowTile& w) {
     if (i == 64) {
-      const int mine = slot + (int)(threadIdx.x & 63) * stride;   // (at most 2^31 tiles in all)
-      const bool live = mine < per_xcd && mine < total - xcd * per_xcd;
+      const int mine = slot + (int)(threadIdx.x & 63) * wgs;   // (at most 2^31 tiles in all)
+      const bool live = mine < end;
       int start, len, t, tm, tn;
       groups.find_lanes(p, live ? xcd * per_xcd + mine : 0, live, b.group, start, len, t);
       b.stream = local_tile(t, len > 0 ? (len + BM - 1) / BM : 1, (p.N + BN - 1) / BN, tm, tn) == 1;
@@ -423,7 +459,7 @@ __global__ __launch_bounds__(256) void grouped_rows_kernel(DeviceGroups p) {
       b.m_rem = len - tm * BM;
       b.col = tn * BN;
       b.count = __popcll(__ballot(live));
-      slot += 64 * stride;
+      slot += 64 * wgs;
       i = 0;
     }
     if (i >= b.count) return false;
@@ -441,7 +477,13 @@ __global__ __launch_bounds__(256) void grouped_rows_kernel(DeviceGroups p) {
     w.K = p.K;
     ++i;
     return true;
-  });
+  };
+  if (rest && shares.pieces > 1) {
+    RowTile t;
+    if (next(t)) run_quarter_tile(lds, t, piece);
+  } else {
+    walk_row_tiles(lds, next);
+  }
 }
 
 template <int LAYOUT, int BM, int BN, int BIAS>
@@ -567,7 +609,8 @@ hipError_t launch_device_layout(const DeviceGroups& p, hipStream_t s) {
     const int64_t most_tiles = ((M + 255) / 256 + G) * ((N + 255) / 256);   // every group may end in a partial tile
     if (M > 0 && most_tiles <= 2147483647 && chain_takes(N, p.K, p.xq, p.wq, p.ws, p.y)) {
       const int64_t cus = device_compute_units(), wgs = (most_tiles + kXcds - 1) / kXcds * kXcds;
-      grouped_rows_kernel<LAYOUT><<<(unsigned)(wgs < cus ? wgs : cus), 256, 0, s>>>(p);
+      if (wgs <= cus) grouped_rows_kernel<LAYOUT><<<(unsigned)wgs, 256, 0, s>>>(p, (int)wgs / kXcds);
+      else grouped_rows_kernel<LAYOUT><<<(unsigned)(2 * cus), 256, 0, s>>>(p, (int)cus / kXcds);
       return hipGetLastError();
     }
     return launch_device_shape<LAYOUT, 256, 256, BIAS>(p, s);

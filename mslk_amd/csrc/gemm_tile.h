@@ -778,7 +778,9 @@ struct GemmTile {
   // ---- Tiles one after the other without a gap (two-plus-three buffers, DIRECT, K > 2 kBK, K % 16 == 0) ----
   // The K steps of consecutive tiles form one chain: the last two steps of a tile issue the first loads of the next one in the
   // places where the steps before them issue the loads of their own tile, so a tile starts with its first operands in LDS.  The
-  // epilogue touches no LDS and runs while the next tile's loads land.
+  // epilogue touches no LDS and runs while the next tile's loads land.  What this replaces: of the 15 us that a tile of six K steps took
+  // (128 experts x 2048 x 768), 1 us went into finding the tile, 2 - 2.5 into the wait for its first operands, 4 into the epilogue
+  // and 0.5 into starting the workgroup; now 12 us, of them 2.8 for the epilogue (vector arithmetic: 3.5 instructions for each of 256 sums).
   // A K that is no multiple of the step ends in a step over the last kBK bytes of the rows: what the step before has
   // consumed already is cleared in the fragments of both operands.
   using Chain = TileChain<TS>;
