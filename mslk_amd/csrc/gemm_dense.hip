@@ -225,6 +225,13 @@ hipError_t launch_dense_tiled(const GemmProblem& p, hipStream_t s) {
   // M = 768, N = 6144, K = 7168: 47.5 -> 40.6; M = 768, N = K = 8192: 54.6 -> 49.0).
   if (small_tiles > cus && big_tiles <= cus / 2) {
     const int64_t tiles19 = (int64_t)((p.M + 191) / 192) * ((p.N + 127) / 128);
+    // 128 x 160 tiles (wave tile 64 x 80, ring of four) where these fit one per CU as well: a sixth less work per tile than 192 x 128
+    // and no more to move (36 KiB a step), and a tile of less than half the work where the 192-row ones do not fit.  With the
+    // quantizer in front, three layers in turn: M = 140 at 19000 x 8192 56.6 -> 50.2 us, 250 at 16640 x 8192 64.5 -> 57.6, 200 at
+    // 18000 x 4096 28.0 -> 24.3, 1024 at 5000 x 8192 48.2 -> 44.6, 512 at 10000 x 4096 27.9 -> 26.6, 385 at 10240 x 4096 26.4 -> 25.3,
+    // 512 at 9216 x 2048 17.8 -> 17.3; 500 at 10240 x 8192 44.0 -> 41.5; the same at
+    // 768 x 6400 x 8192 and 1152 x 4096 x 8192; of 34 shapes none slower by more than the runs of one side differ.
+    if ((int64_t)((p.M + 127) / 128) * ((p.N + 159) / 160) <= cus) return launch_dense_small_tile(kTile128x160, p, s);
     if (tiles19 <= cus) return launch_dense_small_tile(kTile192x128, p, s);
   }
   {

@@ -17,6 +17,7 @@ hipError_t launch_dense_small_tile(int shape, const GemmProblem& p, hipStream_t 
     case kTile128x128Ring: return launch_tiled_shape<TileShape<128, 128, 2, 2, 5>, false, 1>(p, s);
     case kTile128x128: return launch_tiled_shape<TileShape<128, 128>, false>(p, s);
     case kTile192x128: return launch_tiled_shape<TileShape<192, 128, 2, 2, 3>, false>(p, s);
+    case kTile128x160: return launch_tiled_shape<TileShape<128, 160, 2, 2, 4>, false>(p, s);
     default: return hipErrorInvalidValue;
   }
 }

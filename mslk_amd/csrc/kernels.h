@@ -88,6 +88,7 @@ enum DenseSmallTile : int {
   kTile128x128Ring,   // five ring buffers, one workgroup per CU
   kTile128x128,       // two-plus-three buffers, two workgroups per CU
   kTile192x128,
+  kTile128x160,       // four ring buffers, one workgroup per CU
 };
 hipError_t launch_dense_small_tile(int shape, const GemmProblem& p, hipStream_t s);
 // Its branch for pre-shuffled weights (a translation unit of its own); cus: device_compute_units().

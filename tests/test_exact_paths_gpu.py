@@ -372,3 +372,24 @@ def test_weight_streaming_kernel_exact_on_k_loops_that_do_not_divide_among_its_w
     torch.cuda.synchronize()
     _same_bits(y, _want(xi, wi, xs, ws, bias), f"{M}x{N}x{K}")
 
+
+
+@pytest.mark.parametrize("bias_dtype,fp16_out", [(None, False), (torch.float32, False), (torch.bfloat16, True)])
+@pytest.mark.parametrize("M,N,K", [
+    (512, 10240, 384),    # 256 full tiles, fewer K steps than ring buffers
+    (385, 10240, 1040),   # one row in the last row tile, a K tail
+    (500, 10112, 512),    # a last column tile of 32 columns
+    (640, 8136, 528),     # five row tiles; the last column tile ends inside the second wave's columns
+    (500, 10093, 768),    # rows of Y that are 2-byte aligned
+])
+def test_tiles_of_160_columns_exact(M, N, K, bias_dtype, fp16_out):
+    """Stores in which not every lane takes part, and a wave's columns that begin and end inside a line."""
+    from mslk_amd import _lib
+    assert _lib.lib().mslk_amd_debug_dispatch_name(M, N, K, 0, 0, 0, 1).decode().startswith("dense_tiled<128,160")
+    g = torch.Generator().manual_seed(M + 3 * N + K)
+    xi, wi, xs, ws = _ints(M, K, g), _ints(N, K, g), _pow2(M, g), _pow2(N, g)
+    bias = None if bias_dtype is None else torch.randint(-4, 5, (N,), generator=g).float()
+    op = torch.ops.mslk.f8f8f16_rowwise if fp16_out else torch.ops.mslk.f8f8bf16_rowwise
+    y = op(xi.to(F8).to(DEV), wi.to(F8).to(DEV), xs.to(DEV), ws.to(DEV), bias=None if bias is None else bias.to(bias_dtype).to(DEV))
+    torch.cuda.synchronize()
+    _same_bits(y, _want(xi, wi, xs, ws, bias, fp16_out), f"{M}x{N}x{K} bias={bias_dtype} fp16={fp16_out}")
