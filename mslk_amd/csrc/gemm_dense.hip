@@ -229,8 +229,7 @@ hipError_t launch_dense_tiled(const GemmProblem& p, hipStream_t s) {
     // and no more to move (36 KiB a step), and a tile of less than half the work where the 192-row ones do not fit.  With the
     // quantizer in front, three layers in turn: M = 140 at 19000 x 8192 56.6 -> 50.2 us, 250 at 16640 x 8192 64.5 -> 57.6, 200 at
     // 18000 x 4096 28.0 -> 24.3, 1024 at 5000 x 8192 48.2 -> 44.6, 512 at 10000 x 4096 27.9 -> 26.6, 385 at 10240 x 4096 26.4 -> 25.3,
-    // 512 at 9216 x 2048 17.8 -> 17.3; 500 at 10240 x 8192 44.0 -> 41.5; the same at
-    // 768 x 6400 x 8192 and 1152 x 4096 x 8192; of 34 shapes none slower by more than the runs of one side differ.
+    // 512 at 9216 x 2048 17.8 -> 17.3, 500 at 10240 x 8192 44.0 -> 41.5; the same at 768 x 6400 x 8192 and 1152 x 4096 x 8192; of 34 shapes none slower by more than the runs of one side differ.
     if ((int64_t)((p.M + 127) / 128) * ((p.N + 159) / 160) <= cus) return launch_dense_small_tile(kTile128x160, p, s);
     if (tiles19 <= cus) return launch_dense_small_tile(kTile192x128, p, s);
   }
