@@ -323,6 +323,15 @@ const char* mslk_amd_debug_dispatch_name(int64_t M, int64_t N, int64_t K, int bi
                                          int with_workspace);
 
 /*
+ * The same for the grouped entry points on aligned operands: layout 0 is mslk_amd_f8f8bf16_rowwise_grouped_stacked, the
+ * MSLK_AMD_GROUPS_* codes are mslk_amd_f8f8bf16_rowwise_grouped_mm ("grouped_rows<256,256> workgroups=512", ...); the second
+ * is mslk_amd_f8f8bf16_rowwise_grouped, whose host-side schedule also says how many tiles the XCD with the most of them has
+ * ("grouped_listed<256,256> longest=96 workgroups=512"), for at most 256 groups.
+ */
+const char* mslk_amd_debug_grouped_dispatch_name(int layout, int G, int64_t M, int64_t N, int64_t K);
+const char* mslk_amd_debug_grouped_list_dispatch_name(int G, const int64_t* M, const int64_t* N, const int64_t* K);
+
+/*
  * Ceiling probes for the benchmark's roofline columns; no counterpart in the reference (its bench divides by fixed
  * peak figures, bench/gemm/gemm_bench.py:61-68) and not part of the product path.
  *   mslk_amd_debug_stream_read: `workgroups` x 256 lanes read `bytes` from `src` once and write nothing.  mode 0: 16-byte

@@ -463,6 +463,43 @@ const char* mslk_amd_debug_dispatch_name(int64_t M, int64_t N, int64_t K, int bi
   return result;
 }
 
+const char* mslk_amd_debug_grouped_dispatch_name(int layout, int G, int64_t M, int64_t N, int64_t K) {
+  void* const fake = reinterpret_cast<void*>(uintptr_t(1) << 20);
+  const float* const scale = static_cast<const float*>(fake);
+  thread_local char result[600];
+  dispatch_probe_begin();
+  int rc;
+  if (layout == 0)
+    rc = mslk_amd_f8f8bf16_rowwise_grouped_stacked(fake, fake, scale, scale, static_cast<const int64_t*>(fake), G, M, N, K, fake, nullptr);
+  else
+    rc = mslk_amd_f8f8bf16_rowwise_grouped_mm(fake, fake, scale, scale, layout == MSLK_AMD_GROUPS_UNIFORM ? nullptr : static_cast<const int32_t*>(fake),
+                                              layout, G, M, N, K, fake, nullptr);
+  const char* text = dispatch_probe_end();
+  if (rc != 0) snprintf(result, sizeof(result), "error: %s", g_err);
+  else snprintf(result, sizeof(result), "%s", text[0] ? text : "nothing to launch");
+  return result;
+}
+
+const char* mslk_amd_debug_grouped_list_dispatch_name(int G, const int64_t* M, const int64_t* N, const int64_t* K) {
+  void* const fake = reinterpret_cast<void*>(uintptr_t(1) << 20);
+  thread_local char result[600];
+  constexpr int kMost = 256;
+  if (G > kMost) return "error: more than 256 groups";
+  const void* operands[kMost];
+  const float* scales[kMost];
+  void* outputs[kMost];
+  for (int g = 0; g < G; ++g) {
+    operands[g] = outputs[g] = fake;
+    scales[g] = static_cast<const float*>(fake);
+  }
+  dispatch_probe_begin();
+  const int rc = mslk_amd_f8f8bf16_rowwise_grouped(G, operands, operands, scales, scales, outputs, M, N, K, nullptr);
+  const char* text = dispatch_probe_end();
+  if (rc != 0) snprintf(result, sizeof(result), "error: %s", g_err);
+  else snprintf(result, sizeof(result), "%s", text[0] ? text : "nothing to launch");
+  return result;
+}
+
 int mslk_amd_debug_stream_read(const void* src, int64_t bytes, int mode, int workgroups, void* sink, void* stream) {
   if (mode < 0 || mode > 2) return fail("debug_stream_read: mode must be 0 (register loads), 1 (LDS DMA loads) or 2 (non-temporal LDS DMA loads)");
   if (bytes < 0 || bytes % (mode == 0 ? 16 : 1024) != 0) return fail("debug_stream_read: bytes must be a non-negative multiple of %d", mode == 0 ? 16 : 1024);

@@ -245,11 +245,13 @@ static hipError_t launch_grouped_shape(const GroupTable& in, hipStream_t s) {
     bool chain = true;
     for (int i = 0; i < n; ++i) chain = chain && chain_takes(t.g[i].N, t.g[i].K, t.g[i].xq, t.g[i].wq, t.g[i].ws, t.g[i].y);
     if (chain) {
+      if (dispatch_probe_record("grouped_listed<%d,%d> longest=%d workgroups=%d", BM, BN, longest, (longest <= wgs_per_xcd ? longest : 2 * wgs_per_xcd) * kXcds)) return hipSuccess;
       if (longest <= wgs_per_xcd) grouped_listed_kernel<<<longest * kXcds, 256, 0, s>>>(t, longest);
       else grouped_listed_kernel<<<2 * wgs_per_xcd * kXcds, 256, 0, s>>>(t, wgs_per_xcd);
       return hipGetLastError();
     }
   }
+  if (dispatch_probe_record("grouped_tiled<%d,%d> longest=%d workgroups=%d", BM, BN, longest, longest * kXcds)) return hipSuccess;
   grouped_tiled_kernel<BM, BN><<<longest * kXcds, 256, 0, s>>>(t);
   return hipGetLastError();
 }

@@ -571,6 +571,7 @@ hipError_t launch_device_shape(const DeviceGroups& p, hipStream_t s) {
   }
   if (grid <= 0) return hipSuccess;
   if (grid > 2147483647) return hipErrorInvalidValue;
+  if (dispatch_probe_record("grouped_device<%d,%d>%s workgroups=%lld", BM, BN, p.unaligned ? " unaligned" : "", (long long)grid)) return hipSuccess;
   grouped_device_kernel<LAYOUT, BM, BN, BIAS><<<(unsigned)grid, 256, 0, s>>>(p);
   return hipGetLastError();
 }
@@ -609,6 +610,7 @@ hipError_t launch_device_layout(const DeviceGroups& p, hipStream_t s) {
     const int64_t most_tiles = ((M + 255) / 256 + G) * ((N + 255) / 256);   // every group may end in a partial tile
     if (M > 0 && most_tiles <= 2147483647 && chain_takes(N, p.K, p.xq, p.wq, p.ws, p.y)) {
       const int64_t cus = device_compute_units(), wgs = (most_tiles + kXcds - 1) / kXcds * kXcds;
+      if (dispatch_probe_record("grouped_rows<%d,%d> workgroups=%lld", RowTileShape::kBM, RowTileShape::kBN, (long long)(wgs <= cus ? wgs : 2 * cus))) return hipSuccess;
       if (wgs <= cus) grouped_rows_kernel<LAYOUT><<<(unsigned)wgs, 256, 0, s>>>(p, (int)wgs / kXcds);
       else grouped_rows_kernel<LAYOUT><<<(unsigned)(2 * cus), 256, 0, s>>>(p, (int)cus / kXcds);
       return hipGetLastError();

@@ -56,3 +56,19 @@ def assert_gemm_close(y_gpu: torch.Tensor, ref: torch.Tensor, what: str = "", rm
     bad, worst = O.gemm_elementwise_violations(y_gpu.float(), ref, rms)
     assert bad == 0, f"{what}: {bad} elements beyond rtol {O.ELEM_RTOL} / atol {O.ELEM_ATOL_RMS} rms (worst {worst:.2f} x the bound)"
     return max_rel, normwise
+
+
+def grouped_kernel(layout: int, groups: int, M: int, N: int, K: int) -> str:
+    """The kernel that a grouped entry point picks (0: sizes in device memory, 1 ... 4: the layouts of grouped_mm)."""
+    from mslk_amd import _lib
+    return _lib.lib().mslk_amd_debug_grouped_dispatch_name(layout, groups, M, N, K).decode()
+
+
+def grouped_list_kernel(sizes, N: int, K) -> str:
+    """The same for a list of groups; K is one number or one per group."""
+    import ctypes
+    from mslk_amd import _lib
+    G = len(sizes)
+    i64 = lambda v: (ctypes.c_int64 * G)(*v)
+    return _lib.lib().mslk_amd_debug_grouped_list_dispatch_name(
+        G, i64(sizes), i64([N] * G), i64([K] * G if isinstance(K, int) else K)).decode()

@@ -9,6 +9,7 @@ import torch
 
 import mslk_amd
 from mslk_amd import _lib, gemm
+from tests.helpers import grouped_kernel, grouped_list_kernel
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 F8 = torch.float8_e4m3fn
@@ -227,6 +228,39 @@ def test_dispatch_of_the_dense_entry_points_is_pinned(args, want):
     from mslk_amd import _lib
     got = _lib.lib().mslk_amd_debug_dispatch_name(*args).decode()
     assert got == want
+
+
+# Layout code (0: sizes; 1 ... 4: as grouped_mm), groups, M, N, K -> the kernel of the grouped entry points
+GROUPED_DISPATCH_TABLE = [
+    ((0, 16, 8192, 5120, 4096), "grouped_rows<256,256> workgroups=512"),
+    ((1, 128, 32768, 2048, 768), "grouped_rows<256,256> workgroups=512"),
+    ((0, 16, 256, 5120, 4096), "grouped_device<128,128> workgroups=720"),          # 16 rows per group
+    ((1, 8, 8192, 1024, 512), "grouped_device<128,128> workgroups=576"),           # short K, all full tiles at once
+    ((1, 2, 3000, 8192, 256), "grouped_device<256,256> workgroups=448"),           # two K steps: not for the chain
+    ((0, 2, 3000, 8196, 512), "grouped_device<256,256> workgroups=464"),           # rows of Y that are 8-byte aligned
+    ((0, 8, 4096, 4096, 1000), "grouped_device<128,128> unaligned workgroups=1280"),
+    ((3, 8, 4096, 2048, 16384), "grouped_device<256,256> workgroups=1024"),        # K slices
+    ((4, 16, 512, 4096, 4096), "grouped_device<256,256> workgroups=512"),          # uniform
+    ((0, 0, 16, 16, 16), "nothing to launch"),
+]
+
+
+@pytest.mark.parametrize("args,want", GROUPED_DISPATCH_TABLE)
+def test_dispatch_of_the_grouped_entry_points_is_pinned(args, want):
+    assert grouped_kernel(*args) == want
+
+
+GROUPED_LIST_DISPATCH_TABLE = [
+    ([512] * 16, 8192, 5120, "grouped_listed<256,256> longest=128 workgroups=512"),
+    ([16] * 16, 5120, 4096, "grouped_tiled<128,128> longest=80 workgroups=640"),
+    ([2304], 8192, 256, "grouped_tiled<256,256> longest=37 workgroups=296"),       # two K steps: not for the chain
+    ([0, 0], 8192, 512, "nothing to launch"),
+]
+
+
+@pytest.mark.parametrize("sizes,N,K,want", GROUPED_LIST_DISPATCH_TABLE)
+def test_dispatch_of_lists_of_groups_is_pinned(sizes, N, K, want):
+    assert grouped_list_kernel(sizes, N, K) == want
 
 
 def test_dispatch_dry_run_reports_argument_errors_and_leaves_no_state():
