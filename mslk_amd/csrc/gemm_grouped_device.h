@@ -365,7 +365,8 @@ struct TileBatch {
   int row, m_rem, col, group, stream, count;
 };
 
-// What the chain takes: 16-byte pieces of the rows of all operands, of the column scales and of Y, and three K steps.
+// What the chain takes: 16-byte pieces of the rows of all operands, of the column scales and of Y, and three K steps.  (Of operands that
+// are not marked unaligned: its offsets inside a tile have 32 bits.)
 inline bool chain_takes(int64_t N, int64_t K, const void* xq, const void* wq, const void* ws, const void* y) {
   const uintptr_t all = reinterpret_cast<uintptr_t>(xq) | reinterpret_cast<uintptr_t>(wq) | reinterpret_cast<uintptr_t>(ws) | reinterpret_cast<uintptr_t>(y);
   return K > 2 * kBK && K % 16 == 0 && N % 8 == 0 && all % 16 == 0;
@@ -608,7 +609,7 @@ hipError_t launch_device_layout(const DeviceGroups& p, hipStream_t s) {
     const bool short_k = p.K < 768 && full_tiles128 <= 2 * device_compute_units();
     if (launchable && (p.unaligned || short_k || small_row_groups(M, G, tiles128))) return launch_device_shape<LAYOUT, 128, 128, BIAS>(p, s);
     const int64_t most_tiles = ((M + 255) / 256 + G) * ((N + 255) / 256);   // every group may end in a partial tile
-    if (M > 0 && most_tiles <= 2147483647 && chain_takes(N, p.K, p.xq, p.wq, p.ws, p.y)) {
+    if (!p.unaligned && M > 0 && most_tiles <= 2147483647 && chain_takes(N, p.K, p.xq, p.wq, p.ws, p.y)) {
       const int64_t cus = device_compute_units(), wgs = (most_tiles + kXcds - 1) / kXcds * kXcds;
       if (dispatch_probe_record("grouped_rows<%d,%d> workgroups=%lld", RowTileShape::kBM, RowTileShape::kBN, (long long)(wgs <= cus ? wgs : 2 * cus))) return hipSuccess;
       if (wgs <= cus) grouped_rows_kernel<LAYOUT><<<(unsigned)wgs, 256, 0, s>>>(p, (int)wgs / kXcds);

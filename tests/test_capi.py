@@ -239,6 +239,9 @@ GROUPED_DISPATCH_TABLE = [
     ((1, 2, 3000, 8192, 256), "grouped_device<256,256> workgroups=448"),           # two K steps: not for the chain
     ((0, 2, 3000, 8196, 512), "grouped_device<256,256> workgroups=464"),           # rows of Y that are 8-byte aligned
     ((0, 8, 4096, 4096, 1000), "grouped_device<128,128> unaligned workgroups=1280"),
+    # offsets inside a tile beyond 32 bits, with more 128 x 128 tiles than a launch takes: the scalar tile all the same
+    ((0, 1, 8192, 2**26 + 8, 512), "grouped_device<256,256> unaligned workgroups=8650792"),
+    ((1, 1, 2**21, 2**17, 2**24), "grouped_device<256,256> unaligned workgroups=4194816"),
     ((3, 8, 4096, 2048, 16384), "grouped_device<256,256> workgroups=1024"),        # K slices
     ((4, 16, 512, 4096, 4096), "grouped_device<256,256> workgroups=512"),          # uniform
     ((0, 0, 16, 16, 16), "nothing to launch"),
