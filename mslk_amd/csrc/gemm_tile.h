@@ -119,13 +119,6 @@ MSLK_AMD_DEVINL void store16_stream(uint16_t* dst, uint4 val) {
   asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 1" : : "v"(dst), "v"(v) : "memory");
 }
 
-// The same left to the L2, which puts the two halves of a 128-byte line together (epilogue_direct writes 64 bytes of a row at a
-// time; past the L2 a grouped launch that stores much took up to 30 % longer: 64 x 512 rows x 2048 x 768 81 against 62 us).
-MSLK_AMD_DEVINL void store16(void* dst, uint4 val) {
-  const v4i v = {(int)val.x, (int)val.y, (int)val.z, (int)val.w};
-  asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1" : : "v"(dst), "v"(v) : "memory");
-}
-
 // Global -> LDS copy of 16 bytes per lane (1 KiB per wave, contiguous in LDS from `lds_wave_base`), addressed as
 // wave-uniform base + 32-bit lane offset.  Written as an instruction instead of the compiler's builtin for two reasons:
 //   * while a load the compiler knows of as "writes LDS through the vector memory path" is in flight, every wait it
@@ -925,34 +918,52 @@ struct GemmTile {
   // Scale, convert and store the tile; y at its first row and column, N elements between rows.  ALL: every row and column of
   // the tile is valid.  N % 8 == 0, y and the column scales aligned to 16 bytes.
   // FMV < FM: only that many m fragments of a wave have valid rows, dealt to the wave rows round-robin.
+  // A lane's eight columns are 16 of 64 bytes that one fragment pair gives each of 16 rows.  Two pairs make a 128-byte line: the lanes
+  // of rows 0 - 7 and 8 - 15 exchange one of their two pieces (row_ror:8), so that one store writes whole lines of eight rows and the
+  // next those of the other eight, past the L2.  Half lines were slow past the L2 (64 x 512 rows x 2048 x 768: 81 against 62 us), and left to the L2
+  // they displaced operands: eight groups of 1500 rows and 56 of 40 as a list, x 4096 x 4096, 365 us (333 now), 64 groups of 16384
+  // rows x 2816 x 2880 220 (203), 64 x 150 rows x 4096 x 2048 124 (115); 64 x 300 rows x 4096 x 768 102 (95), of cold weights.
   template <bool ALL, int FMV>
   MSLK_AMD_DEVINL void epilogue_direct(v4f (&acc)[TS::FN][TS::FM], const Scales& sc, uint16_t* y, int m_rem, int n_rem, int N) {
     constexpr bool ILV = FMV < TS::FM;
     static_assert(TS::FM * TS::FN * 4 >= 256 && BIAS == 0, "tiles whose sums fill the accumulator registers");
+    static_assert(TS::FN % 4 == 0, "whole lines");
     int lane = threadIdx.x & 63;
     asm volatile("" : "+v"(lane));
-    const int j = lane & 15, n_base = (wave_id() % TS::WN) * (TS::kBN / TS::WN) + 8 * (lane >> 4);
+    const int j = lane & 7, n_base = (wave_id() % TS::WN) * (TS::kBN / TS::WN) + 8 * (lane >> 4) + 32 * ((lane >> 3) & 1);
     const uint32_t lane_off = ((uint32_t)j * (uint32_t)N + (uint32_t)n_base) * 2u;   // bytes; 16 N < 2^31
+    const uint32_t lane_off8 = lane_off + 16u * (uint32_t)N;                         // eight rows further
 #pragma unroll
     for (int tm = 0; tm < FMV; ++tm) {
       const int row0 = direct_row<ILV>(tm);
       if (!ALL && row0 >= m_rem) continue;   // no valid row in this fragment (wave-uniform)
       char* const row = reinterpret_cast<char*>(y + (int64_t)row0 * N);
 #pragma unroll
-      for (int t = 0; t < TS::FN / 2; ++t) {
-        uint32_t w[4];
+      for (int t = 0; t < TS::FN / 2; t += 2) {
+        uint32_t w[2][4];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int h = 0; h < 4; ++h) {
           float v[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             v[r] = (acc[2 * t + h][tm][r] * sc.ws[2 * t + h][r]) * sc.xs[tm];   // the order of the reference's epilogue (fp8_rowwise_common.h:66)
           }
-          w[2 * h] = pack_out_x2<false>(v[0], v[1]);
-          w[2 * h + 1] = pack_out_x2<false>(v[2], v[3]);
+          w[h >> 1][2 * (h & 1)] = pack_out_x2<false>(v[0], v[1]);
+          w[h >> 1][2 * (h & 1) + 1] = pack_out_x2<false>(v[2], v[3]);
+          if (h == 1) __builtin_amdgcn_sched_barrier(0);
         }
-        if (ALL || (row0 + j < m_rem && n_base + t * 32 < n_rem))
-          store16(row + lane_off + t * 64, make_uint4(w[0], w[1], w[2], w[3]));
+        // rows 0 - 7 in `lo`, 8 - 15 in `hi`: the first pair's columns in lanes 0 - 7 of every 16, the second's in lanes 8 - 15
+        uint32_t lo[4], hi[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          lo[e] = __builtin_amdgcn_update_dpp(w[0][e], w[1][e], 0x128, 0xF, 0xC, false);
+          hi[e] = __builtin_amdgcn_update_dpp(w[1][e], w[0][e], 0x128, 0xF, 0x3, false);
+        }
+        const bool col = ALL || n_base + t * 32 < n_rem;
+        if (ALL || (col && row0 + j < m_rem))
+          store16_stream(reinterpret_cast<uint16_t*>(row + lane_off + t * 64), make_uint4(lo[0], lo[1], lo[2], lo[3]));
+        if (ALL || (col && row0 + j + 8 < m_rem))
+          store16_stream(reinterpret_cast<uint16_t*>(row + lane_off8 + t * 64), make_uint4(hi[0], hi[1], hi[2], hi[3]));
         __builtin_amdgcn_sched_barrier(0);
       }
     }

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import mslk_amd  # noqa: F401
+from tests.helpers import grouped_kernel
 
 pytestmark = pytest.mark.gpu
 DEV, F8 = "cuda:0", torch.float8_e4m3fn
@@ -43,6 +44,23 @@ def test_tiles_in_a_chain(sizes, N, K):
         return   # lists take no shorter rows
     lists = [list(xq.split(sizes)), list(wq.unbind(0)), list(xs.split(sizes)), list(ws.unbind(0))]
     assert torch.equal(torch.ops.mslk.f8f8bf16_rowwise_grouped_cat(*lists).cpu(), want)
+
+
+@pytest.mark.parametrize("N", [8200, 8232, 8168, 8192 + 56])
+@pytest.mark.parametrize("sizes", [[263, 264, 265, 271, 272, 273, 7, 8, 9], [1031, 1032, 1033, 15, 16, 17]])
+def test_stores_of_ragged_tiles(sizes, N):
+    """Eight rows and 64 columns go out together: rows that end next to a multiple of eight, columns inside a group of 64; and nothing
+    beyond them is written."""
+    K = 400
+    xq, wq, xs, ws, want = _operands(sizes, N, K)
+    rows = sum(sizes)
+    assert grouped_kernel(0, len(sizes), rows, N, K).startswith("grouped_rows<256,256>")
+    buffer = torch.full((rows + 64, N), 777.0, dtype=torch.bfloat16, device=DEV)
+    off = torch.tensor(sizes).cumsum(0).to(torch.int32).to(DEV)
+    torch.ops.mslk.f8f8bf16_rowwise_grouped_mm(xq, wq, xs, ws, off, buffer[32:32 + rows])
+    out = buffer.cpu()
+    assert torch.equal(out[32:32 + rows], want)
+    assert (out[:32] == 777.0).all() and (out[32 + rows:] == 777.0).all()
 
 
 def test_codes_beyond_a_row_do_not_count():
