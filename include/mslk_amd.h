@@ -332,6 +332,13 @@ const char* mslk_amd_debug_grouped_dispatch_name(int layout, int G, int64_t M, i
 const char* mslk_amd_debug_grouped_list_dispatch_name(int G, const int64_t* M, const int64_t* N, const int64_t* K);
 
 /*
+ * How the 256 x 256 tiles of row groups are divided inside an XCD: the entry of its slice of `tiles` tiles that workgroup `worker`
+ * (of 2 * wgs) works on in `pass`, -1 for none, and which piece of how many of that tile (*piece, *pieces).  Host code; returns -2
+ * for arguments out of range.
+ */
+int mslk_amd_debug_row_walk(int tiles, int wgs, int worker, int pass, int* piece, int* pieces);
+
+/*
  * Ceiling probes for the benchmark's roofline columns; no counterpart in the reference (its bench divides by fixed
  * peak figures, bench/gemm/gemm_bench.py:61-68) and not part of the product path.
  *   mslk_amd_debug_stream_read: `workgroups` x 256 lanes read `bytes` from `src` once and write nothing.  mode 0: 16-byte

@@ -500,6 +500,11 @@ const char* mslk_amd_debug_grouped_list_dispatch_name(int G, const int64_t* M, c
   return result;
 }
 
+int mslk_amd_debug_row_walk(int tiles, int wgs, int worker, int pass, int* piece, int* pieces) {
+  if (tiles < 0 || tiles > (1 << 28) || wgs <= 0 || wgs > 1024 || worker < 0 || worker >= 2 * wgs || pass < 0 || pass > (1 << 20) || !piece || !pieces) return -2;
+  return debug_row_walk(tiles, wgs, worker, pass, piece, pieces);
+}
+
 int mslk_amd_debug_stream_read(const void* src, int64_t bytes, int mode, int workgroups, void* sink, void* stream) {
   if (mode < 0 || mode > 2) return fail("debug_stream_read: mode must be 0 (register loads), 1 (LDS DMA loads) or 2 (non-temporal LDS DMA loads)");
   if (bytes < 0 || bytes % (mode == 0 ? 16 : 1024) != 0) return fail("debug_stream_read: bytes must be a non-negative multiple of %d", mode == 0 ? 16 : 1024);

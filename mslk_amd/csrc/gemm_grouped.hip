@@ -68,19 +68,14 @@ __global__ __launch_bounds__(256) void grouped_listed_kernel(GroupTable tab, int
   const int lane = threadIdx.x & 63;
   const int first = lane < tab.count ? tab.g[lane].tile_begin : 0x7FFFFFFF;   // of group `lane`
   const SliceShares shares(tiles, wgs);
-  int slot = blockIdx.x / kXcds, end = shares.walked, piece = 0;
-  const bool rest = slot >= wgs;
-  if (rest) {
-    piece = (slot - wgs) % shares.pieces;
-    slot = shares.walked + (slot - wgs) / shares.pieces;
-    end = slot < tiles ? slot + 1 : slot;
-  }
+  const int worker = blockIdx.x / kXcds;
+  const bool rest = worker >= wgs;
   TileBatch b;
-  int i = 64;
+  int i = 64, pass = 0;
   auto next = [&](RowTile& w) {
     if (i == 64) {
-      const int mine = slot + lane * wgs;
-      const bool live = mine < end;
+      const int mine = rest ? shares.left_entry(worker) : shares.walked_entry(worker, pass + lane);
+      const bool live = rest ? lane == 0 && pass == 0 && mine < tiles : mine < shares.walked;
       const int t = live ? begin + mine : 0;
       int gi = 0;   // the last group that begins at or before t
 #pragma unroll
@@ -92,7 +87,7 @@ __global__ __launch_bounds__(256) void grouped_listed_kernel(GroupTable tab, int
       b.col = tn * BN;
       b.group = gi;
       b.count = __popcll(__ballot(live));
-      slot += 64 * wgs;
+      pass += 64;
       i = 0;
     }
     if (i >= b.count) return false;
@@ -103,7 +98,7 @@ __global__ __launch_bounds__(256) void grouped_listed_kernel(GroupTable tab, int
   };
   if (rest && shares.pieces > 1) {
     RowTile t;
-    if (next(t)) run_quarter_tile(lds, t, piece);
+    if (next(t)) run_quarter_tile(lds, t, shares.left_piece(worker));
   } else {
     walk_row_tiles(lds, next);
   }
@@ -284,6 +279,15 @@ hipError_t launch_grouped_tiled(const GroupTable& in, hipStream_t s) {
 static bool device_groups_aligned(const DeviceGroups& p) {
   return p.K % 16 == 0 && (int64_t)256 * p.K < (int64_t(1) << 32) && p.N < (1 << 26) &&
          reinterpret_cast<uintptr_t>(p.xq) % 16 == 0 && reinterpret_cast<uintptr_t>(p.wq) % 16 == 0;
+}
+
+int debug_row_walk(int tiles, int wgs, int worker, int pass, int* piece, int* pieces) {
+  const SliceShares shares(tiles, wgs);
+  const bool rest = worker >= wgs;
+  *piece = rest ? shares.left_piece(worker) : 0;
+  *pieces = rest ? shares.pieces : 1;
+  if (rest) return pass == 0 && shares.left_entry(worker) < tiles ? shares.left_entry(worker) : -1;
+  return shares.walked_entry(worker, pass) < shares.walked ? shares.walked_entry(worker, pass) : -1;
 }
 
 hipError_t launch_device_groups(const DeviceGroups& in, int layout, hipStream_t s) {

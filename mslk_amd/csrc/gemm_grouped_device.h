@@ -344,20 +344,34 @@ struct RowTile {
   int stream;         // the only reader of its weight block at that time: weights fetched with non-temporal loads
 };
 
-// Division of the `tiles` tiles of an XCD among its `wgs` workgroups.  The first `wgs` workgroups walk the full passes, entry i of
-// the slice going to workgroup i % wgs.  What is left over for a last pass, as long as it is at most three quarters of one, is
+// Division of the `tiles` tiles of an XCD among its `wgs` workgroups.  The first `wgs` workgroups walk the full passes, one entry of
+// the slice each per pass.  What is left over for a last pass, as long as it is at most three quarters of one, is
 // given to further workgroups, one tile each, which the hardware starts where one of the first ones ends: tiles cost what their
 // rows cost, and the workgroups that were given cheap ones take what is left.  At most a quarter of a pass is cut into quarters of tiles besides.
 // (16 experts x 5120 x 4096 over 8192 rows, 780 tiles: a fourth pass with 12 of 256 workgroups busy, 198 -> 156 us.)
+// Neighbouring entries are the row tiles of a panel (local_tile), the last of which may be ragged.  From pass to pass a workgroup
+// moves on by wgs + turn entries, and wgs + turn has no divisor in common with any number of row tiles in a panel: every workgroup gets
+// its share of the ragged ones.  With entry i for workgroup i % wgs half of the 32 workgroups of an XCD were given all full tiles
+// of groups of 300 rows, and the launch took as long as full tiles do (64 x 300 rows x 4096 x 768: 121 -> 105 us; 128 x 257 x 2048 x 768
+// 122 -> 98; 16 x 257 x 8192 x 2048 107 -> 97).
 struct SliceShares {
+  int wgs, turn;
   int walked;        // entries of the slice that the first workgroups walk
   int pieces;        // of a left-over tile: 1 or 4
-  MSLK_AMD_DEVINL SliceShares(int tiles, int wgs) {
+  __host__ __device__ SliceShares(int tiles, int workgroups) : wgs(workgroups) {
+    static_assert(kGroupM <= 4, "one to four row tiles in a panel");
     const int left = tiles % wgs;
     const bool apart = tiles > wgs && left * 4 <= wgs * 3;
     walked = apart ? tiles - left : tiles;
     pieces = left * 4 <= wgs ? 4 : 1;
+    const int r = wgs % 6;
+    turn = r == 2 ? 3 : r == 3 ? 2 : r == 1 || r == 5 ? 0 : 1;   // wgs + turn is 1 or 5 modulo 6
   }
+  // Entry of the slice that workgroup `worker` < wgs walks in `pass`: its own if it is below `walked`.
+  __host__ __device__ int walked_entry(int worker, int pass) const { return pass * wgs + (worker + pass * turn) % wgs; }
+  // Left-over entry, and piece of it, of workgroup `worker` >= wgs: one of the slice if it is below `tiles`.
+  __host__ __device__ int left_entry(int worker) const { return walked + (worker - wgs) / pieces; }
+  __host__ __device__ int left_piece(int worker) const { return (worker - wgs) % pieces; }
 };
 
 // The tiles of one workgroup, found 64 at a time, one per lane: row and column, group and what is left of it.
@@ -440,19 +454,15 @@ __global__ __launch_bounds__(256) void grouped_rows_kernel(DeviceGroups p, int w
   const int xcd = blockIdx.x % kXcds, per_xcd = (int)groups.per_xcd, left = (int)groups.total_tiles - xcd * per_xcd;
   const int tiles = left < per_xcd ? left : per_xcd;
   const SliceShares shares(tiles, wgs);
-  int slot = blockIdx.x / kXcds, end = shares.walked, piece = 0;
-  const bool rest = slot >= wgs;
-  if (rest) {
-    piece = (slot - wgs) % shares.pieces;
-    slot = shares.walked + (slot - wgs) / shares.pieces;
-    end = slot < tiles ? slot + 1 : slot;
-  }
+  const int worker = blockIdx.x / kXcds;
+  const bool rest = worker >= wgs;
   TileBatch b;
-  int i = 64;
+  int i = 64, pass = 0;
   auto next = [&](RowTile& w) {
     if (i == 64) {
-      const int mine = slot + (int)(threadIdx.x & 63) * wgs;   // (at most 2^31 tiles in all)
-      const bool live = mine < end;
+      const int lane = threadIdx.x & 63;
+      const int mine = rest ? shares.left_entry(worker) : shares.walked_entry(worker, pass + lane);   // (at most 2^31 tiles in all)
+      const bool live = rest ? lane == 0 && pass == 0 && mine < tiles : mine < shares.walked;
       int start, len, t, tm, tn;
       groups.find_lanes(p, live ? xcd * per_xcd + mine : 0, live, b.group, start, len, t);
       b.stream = local_tile(t, len > 0 ? (len + BM - 1) / BM : 1, (p.N + BN - 1) / BN, tm, tn) == 1;
@@ -460,7 +470,7 @@ __global__ __launch_bounds__(256) void grouped_rows_kernel(DeviceGroups p, int w
       b.m_rem = len - tm * BM;
       b.col = tn * BN;
       b.count = __popcll(__ballot(live));
-      slot += 64 * wgs;
+      pass += 64;
       i = 0;
     }
     if (i >= b.count) return false;
@@ -481,7 +491,7 @@ __global__ __launch_bounds__(256) void grouped_rows_kernel(DeviceGroups p, int w
   };
   if (rest && shares.pieces > 1) {
     RowTile t;
-    if (next(t)) run_quarter_tile(lds, t, piece);
+    if (next(t)) run_quarter_tile(lds, t, shares.left_piece(worker));
   } else {
     walk_row_tiles(lds, next);
   }

@@ -75,6 +75,9 @@ hipError_t launch_debug_gemm_phases(const GemmProblem& p, uint64_t* stamps, hipS
 void dispatch_probe_begin();
 const char* dispatch_probe_end();                       // "a + b" when the dispatch would issue several launches
 bool dispatch_probe_record(const char* fmt, ...);       // false when no dry run is active on this thread
+// Entry of an XCD's slice of `tiles` tiles that workgroup `worker` of 2 * `wgs` works on in `pass` (-1: none), and which of how many
+// pieces of it: the division of the row chain's tiles, computed on the host for the tests (mslk_amd_debug_row_walk).
+int debug_row_walk(int tiles, int wgs, int worker, int pass, int* piece, int* pieces);
 // Compute units of the current device, rounded down to a multiple of the XCD count (256 on a whole MI355X, also
 // when no device can be queried); the tile-shape thresholds and the persistent grid both use it.
 int device_compute_units();
