@@ -20,7 +20,7 @@ namespace {
 
 // XCD x works on its own contiguous slice of the tile list (the launcher has cut the list by estimated cost).  Tile of the group
 // whose descriptor is tab.g[gi].
-MSLK_AMD_DEVINL void listed_tile(const GroupTable& tab, int gi, int row, int col, RowTile& w) {
+MSLK_AMD_DEVINL void listed_tile(const GroupTable& tab, int gi, int row, int col, int stream, RowTile& w) {
   const GroupDesc& d = tab.g[gi];
   w.a = d.xq + (int64_t)row * d.K;
   w.b = d.wq + (int64_t)col * d.K;
@@ -31,6 +31,7 @@ MSLK_AMD_DEVINL void listed_tile(const GroupTable& tab, int gi, int row, int col
   w.n_rem = d.N - col;
   w.N = d.N;
   w.K = d.K;
+  w.stream = stream;
 }
 
 template <int BM, int BN>
@@ -47,10 +48,10 @@ __global__ __launch_bounds__(256) void grouped_tiled_kernel(GroupTable tab) {
   int tm, tn;
   const int panel_rows = local_tile(t - tab.g[gi].tile_begin, (tab.g[gi].M + BM - 1) / BM, (tab.g[gi].N + BN - 1) / BN, tm, tn);
   RowTile w;
-  listed_tile(tab, gi, tm * BM, tn * BN, w);
+  listed_tile(tab, gi, tm * BM, tn * BN, panel_rows == 1, w);
   // ROWSKIP: the ragged last row tile of a group costs what its rows cost.  A tile alone in its panel is the only reader
   // of its weight block at that time: it fetches the weights with non-temporal loads.
-  if (panel_rows == 1) {
+  if (w.stream) {
     GemmTile<TS, 0, false, true, TS::LA / 2, false, true> tile;
     tile.run(lds, w.a, w.b, w.xs, w.ws, nullptr, w.y, w.m_rem, w.n_rem, w.N, w.K);
   } else {
@@ -70,12 +71,28 @@ __global__ __launch_bounds__(256) void grouped_listed_kernel(GroupTable tab, int
   const SliceShares shares(tiles, wgs);
   const int worker = blockIdx.x / kXcds;
   const bool rest = worker >= wgs;
+  // The first tile, often the only one, is found for itself; the others, 64 at a time, under its first loads.
+  const int entry = rest ? shares.left_entry(worker) : shares.walked_entry(worker, 0);
+  if (entry >= (rest ? tiles : shares.walked)) return;
+  RowTile t;
+  {
+    const int gi = __builtin_amdgcn_readfirstlane(__popcll(__ballot(begin + entry >= first)) - 1);
+    const GroupDesc& d = tab.g[gi];
+    int tm, tn;
+    const int stream = local_tile(begin + entry - d.tile_begin, (d.M + BM - 1) / BM, (d.N + BN - 1) / BN, tm, tn) == 1;
+    listed_tile(tab, gi, tm * BM, tn * BN, stream, t);
+  }
+  if (rest && shares.pieces > 1) {
+    run_quarter_tile(lds, t, shares.left_piece(worker));
+    return;
+  }
   TileBatch b;
-  int i = 64, pass = 0;
-  auto next = [&](RowTile& w) {
+  int i = 64, pass = 1;
+  walk_row_tiles(lds, t, [&](RowTile& w) {
+    if (rest || tiles <= wgs) return false;
     if (i == 64) {
-      const int mine = rest ? shares.left_entry(worker) : shares.walked_entry(worker, pass + lane);
-      const bool live = rest ? lane == 0 && pass == 0 && mine < tiles : mine < shares.walked;
+      const int mine = shares.walked_entry(worker, pass + lane);
+      const bool live = mine < shares.walked;
       const int t = live ? begin + mine : 0;
       int gi = 0;   // the last group that begins at or before t
 #pragma unroll
@@ -91,17 +108,11 @@ __global__ __launch_bounds__(256) void grouped_listed_kernel(GroupTable tab, int
       i = 0;
     }
     if (i >= b.count) return false;
-    listed_tile(tab, __builtin_amdgcn_readlane(b.group, i), __builtin_amdgcn_readlane(b.row, i), __builtin_amdgcn_readlane(b.col, i), w);
-    w.stream = __builtin_amdgcn_readlane(b.stream, i);
+    listed_tile(tab, __builtin_amdgcn_readlane(b.group, i), __builtin_amdgcn_readlane(b.row, i), __builtin_amdgcn_readlane(b.col, i),
+                __builtin_amdgcn_readlane(b.stream, i), w);
     ++i;
     return true;
-  };
-  if (rest && shares.pieces > 1) {
-    RowTile t;
-    if (next(t)) run_quarter_tile(lds, t, shares.left_piece(worker));
-  } else {
-    walk_row_tiles(lds, next);
-  }
+  });
 }
 
 }  // namespace
@@ -237,12 +248,11 @@ static hipError_t launch_grouped_shape(const GroupTable& in, hipStream_t s) {
   for (int i = 0; i < kXcds; ++i)
     if (t.xcd_begin[i + 1] - t.xcd_begin[i] > longest) longest = t.xcd_begin[i + 1] - t.xcd_begin[i];
   if constexpr (BM == RowTileShape::kBM) {
-    bool chain = true;
+    bool chain = longest > wgs_per_xcd;   // (as for sizes on the device: without a second tile the chain gains nothing)
     for (int i = 0; i < n; ++i) chain = chain && chain_takes(t.g[i].N, t.g[i].K, t.g[i].xq, t.g[i].wq, t.g[i].ws, t.g[i].y);
     if (chain) {
-      if (dispatch_probe_record("grouped_listed<%d,%d> longest=%d workgroups=%d", BM, BN, longest, (longest <= wgs_per_xcd ? longest : 2 * wgs_per_xcd) * kXcds)) return hipSuccess;
-      if (longest <= wgs_per_xcd) grouped_listed_kernel<<<longest * kXcds, 256, 0, s>>>(t, longest);
-      else grouped_listed_kernel<<<2 * wgs_per_xcd * kXcds, 256, 0, s>>>(t, wgs_per_xcd);
+      if (dispatch_probe_record("grouped_listed<%d,%d> longest=%d workgroups=%d", BM, BN, longest, 2 * wgs_per_xcd * kXcds)) return hipSuccess;
+      grouped_listed_kernel<<<2 * wgs_per_xcd * kXcds, 256, 0, s>>>(t, wgs_per_xcd);
       return hipGetLastError();
     }
   }

@@ -396,22 +396,25 @@ MSLK_AMD_DEVINL void run_quarter_tile(char* lds, const RowTile& t, int piece) {
            t.m_rem - row, t.n_rem - col, t.N, t.K);
 }
 
-// `next(tile)` gives the tiles one after the other.
+// Tile `t` and then those that `next(tile)` gives, one after the other.
 template <typename Next>
-MSLK_AMD_DEVINL void walk_row_tiles(char* lds, Next&& next) {
+MSLK_AMD_DEVINL void walk_row_tiles(char* lds, RowTile t, Next&& next) {
   using TS = RowTileShape;
   using Plain = GemmTile<TS, 0, false, true, TS::LA / 2, false, false, true>;
   using Streamed = GemmTile<TS, 0, false, true, TS::LA / 2, false, true, true>;
-  RowTile t, n;
-  if (!next(t)) return;
+  RowTile n;
   auto operands = [](const RowTile& w) { return TileOperands{w.a, w.b, w.m_rem, w.n_rem, w.K, (uint32_t)w.K}; };
   Plain tile;
   Streamed streamed;
   TileChain<TS> chain(lds);
   tile.chain_start(chain, operands(t));
+  bool more = next(n);   // under the first loads
+  tile.chain_started();
   for (;;) {
-    const bool more = next(n);
-    if (!more) n = t;   // its loads are issued once more, for nobody
+    if (!more) {   // the last two steps issue loads all the same: of one row of each operand, which the caches hold
+      n = t;
+      n.m_rem = n.n_rem = 1;
+    }
     const TileOperands o = operands(n);
     // One K loop and epilogue per number of m fragments with valid rows and kind of weight loads: a common end for all would
     // have the sums moved between registers.
@@ -439,6 +442,7 @@ MSLK_AMD_DEVINL void walk_row_tiles(char* lds, Next&& next) {
     }
     if (!more) break;
     t = n;
+    more = next(n);
   }
   wait_vmcnt0();   // no copy into LDS may outlive the workgroup
 }
@@ -456,13 +460,39 @@ __global__ __launch_bounds__(256) void grouped_rows_kernel(DeviceGroups p, int w
   const SliceShares shares(tiles, wgs);
   const int worker = blockIdx.x / kXcds;
   const bool rest = worker >= wgs;
+  auto tile_at = [&](int64_t group, int64_t row, int m_rem, int64_t col, int stream, RowTile& w) {
+    w.m_rem = m_rem;
+    w.stream = stream;
+    w.n_rem = p.N - (int)col;
+    w.a = p.xq + row * p.K;
+    w.b = p.wq + (group * p.N + col) * p.K;
+    w.xs = p.xs + row;
+    w.ws = p.ws + group * p.N + col;
+    w.y = p.y + row * p.N + col;
+    w.N = p.N;
+    w.K = p.K;
+  };
+  // The first tile, often the only one, is found for itself; the others, 64 at a time, under its first loads.
+  const int entry = rest ? shares.left_entry(worker) : shares.walked_entry(worker, 0);
+  GroupSpan sp;
+  if (entry >= (rest ? tiles : shares.walked) || !groups.find(p, (int64_t)xcd * per_xcd + entry, sp)) return;
+  RowTile t;
+  {
+    int tm, tn;
+    const int stream = local_tile(sp.t, (sp.len + BM - 1) / BM, (p.N + BN - 1) / BN, tm, tn) == 1;
+    tile_at(sp.gi, sp.o0 + tm * BM, sp.len - tm * BM, tn * BN, stream, t);
+  }
+  if (rest && shares.pieces > 1) {
+    run_quarter_tile(lds, t, shares.left_piece(worker));
+    return;
+  }
   TileBatch b;
-  int i = 64, pass = 0;
-  auto next = [&](RowTile& w) {
+  int i = 64, pass = 1;
+  walk_row_tiles(lds, t, [&](RowTile& w) {
+    if (rest || tiles <= wgs) return false;
     if (i == 64) {
-      const int lane = threadIdx.x & 63;
-      const int mine = rest ? shares.left_entry(worker) : shares.walked_entry(worker, pass + lane);   // (at most 2^31 tiles in all)
-      const bool live = rest ? lane == 0 && pass == 0 && mine < tiles : mine < shares.walked;
+      const int mine = shares.walked_entry(worker, pass + (int)(threadIdx.x & 63));   // (at most 2^31 tiles in all)
+      const bool live = mine < shares.walked;
       int start, len, t, tm, tn;
       groups.find_lanes(p, live ? xcd * per_xcd + mine : 0, live, b.group, start, len, t);
       b.stream = local_tile(t, len > 0 ? (len + BM - 1) / BM : 1, (p.N + BN - 1) / BN, tm, tn) == 1;
@@ -474,27 +504,11 @@ __global__ __launch_bounds__(256) void grouped_rows_kernel(DeviceGroups p, int w
       i = 0;
     }
     if (i >= b.count) return false;
-    const int64_t row = __builtin_amdgcn_readlane(b.row, i), col = __builtin_amdgcn_readlane(b.col, i);
-    const int64_t group = __builtin_amdgcn_readlane(b.group, i);
-    w.m_rem = __builtin_amdgcn_readlane(b.m_rem, i);
-    w.stream = __builtin_amdgcn_readlane(b.stream, i);
-    w.n_rem = p.N - (int)col;
-    w.a = p.xq + row * p.K;
-    w.b = p.wq + (group * p.N + col) * p.K;
-    w.xs = p.xs + row;
-    w.ws = p.ws + group * p.N + col;
-    w.y = p.y + row * p.N + col;
-    w.N = p.N;
-    w.K = p.K;
+    tile_at(__builtin_amdgcn_readlane(b.group, i), __builtin_amdgcn_readlane(b.row, i), __builtin_amdgcn_readlane(b.m_rem, i),
+            __builtin_amdgcn_readlane(b.col, i), __builtin_amdgcn_readlane(b.stream, i), w);
     ++i;
     return true;
-  };
-  if (rest && shares.pieces > 1) {
-    RowTile t;
-    if (next(t)) run_quarter_tile(lds, t, shares.left_piece(worker));
-  } else {
-    walk_row_tiles(lds, next);
-  }
+  });
 }
 
 template <int LAYOUT, int BM, int BN, int BIAS>
@@ -618,12 +632,14 @@ hipError_t launch_device_layout(const DeviceGroups& p, hipStream_t s) {
     const int64_t full_tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
     const bool short_k = p.K < 768 && full_tiles128 <= 2 * device_compute_units();
     if (launchable && (p.unaligned || short_k || small_row_groups(M, G, tiles128))) return launch_device_shape<LAYOUT, 128, 128, BIAS>(p, s);
-    const int64_t most_tiles = ((M + 255) / 256 + G) * ((N + 255) / 256);   // every group may end in a partial tile
-    if (!p.unaligned && M > 0 && most_tiles <= 2147483647 && chain_takes(N, p.K, p.xq, p.wq, p.ws, p.y)) {
-      const int64_t cus = device_compute_units(), wgs = (most_tiles + kXcds - 1) / kXcds * kXcds;
-      if (dispatch_probe_record("grouped_rows<%d,%d> workgroups=%lld", RowTileShape::kBM, RowTileShape::kBN, (long long)(wgs <= cus ? wgs : 2 * cus))) return hipSuccess;
-      if (wgs <= cus) grouped_rows_kernel<LAYOUT><<<(unsigned)wgs, 256, 0, s>>>(p, (int)wgs / kXcds);
-      else grouped_rows_kernel<LAYOUT><<<(unsigned)(2 * cus), 256, 0, s>>>(p, (int)cus / kXcds);
+    // The chain where there may be more tiles than CUs.  Without a second tile it has nothing to put a tile's end under, and its workgroups
+    // of left-over tiles cost a launch each (K = 384 ... 2048 x 4096: one group of 4096 rows 8 - 17 % more than tiles one per
+    // workgroup, two of 1024 16 %).
+    const int64_t cus = device_compute_units();
+    const int64_t most_tiles = (M + 255 * G) / 256 * ((N + 255) / 256);   // every group may end in a tile of one row
+    if (!p.unaligned && M > 0 && most_tiles > cus && most_tiles <= 2147483647 && chain_takes(N, p.K, p.xq, p.wq, p.ws, p.y)) {
+      if (dispatch_probe_record("grouped_rows<%d,%d> workgroups=%lld", RowTileShape::kBM, RowTileShape::kBN, (long long)(2 * cus))) return hipSuccess;
+      grouped_rows_kernel<LAYOUT><<<(unsigned)(2 * cus), 256, 0, s>>>(p, (int)cus / kXcds);
       return hipGetLastError();
     }
     return launch_device_shape<LAYOUT, 256, 256, BIAS>(p, s);

@@ -790,7 +790,8 @@ struct GemmTile {
     a_rows = o.a_rows; a_rows_hi = o.a_rows_hi;
   }
 
-  // The state a tile of the chain starts from: XQ and WQ of step 0 in LDS, WQ and the first XQ_EARLY loads of XQ of step 1 in flight.
+  // The state a tile of the chain starts from, once chain_started() returns: XQ and WQ of step 0 in LDS, WQ and the first XQ_EARLY
+  // loads of XQ of step 1 in flight.
   MSLK_AMD_DEVINL void chain_start(const Chain& c, const TileOperands& o) {
     init(o.a, o.b, o.rows_a < TS::kBM ? o.rows_a : TS::kBM, o.rows_b < TS::kBN ? o.rows_b : TS::kBN, o.ld);
     issue_a_all(c.a_cur, 0);
@@ -798,8 +799,8 @@ struct GemmTile {
     issue_b_all(c.b_nxt, kBK);
 #pragma unroll
     for (int i = 0; i < XQ_EARLY; ++i) issue_a(c.a_nxt, kBK, i);
-    wait_and_barrier<TS::LB + XQ_EARLY>();
   }
+  MSLK_AMD_DEVINL static void chain_started() { wait_and_barrier<TS::LB + XQ_EARLY>(); }
 
   // K loop of one tile, then the state above for tile `n`.  `scales` are loaded under the last step (ILV as in the epilogue).
   template <int FMV>

@@ -239,6 +239,9 @@ GROUPED_DISPATCH_TABLE = [
     ((1, 2, 3000, 8192, 256), "grouped_device<256,256> workgroups=448"),           # two K steps: not for the chain
     ((0, 2, 3000, 8196, 512), "grouped_device<256,256> workgroups=464"),           # rows of Y that are 8-byte aligned
     ((0, 8, 4096, 4096, 1000), "grouped_device<128,128> unaligned workgroups=1280"),
+    ((1, 1, 4096, 4096, 768), "grouped_device<256,256> workgroups=272"),           # at most one tile per CU: no chain
+    ((0, 2, 2048, 4096, 1024), "grouped_device<256,256> workgroups=160"),
+    ((0, 1, 4097, 4096, 768), "grouped_rows<256,256> workgroups=512"),             # 272 tiles
     # offsets inside a tile beyond 32 bits, with more 128 x 128 tiles than a launch takes: the scalar tile all the same
     ((0, 1, 8192, 2**26 + 8, 512), "grouped_device<256,256> unaligned workgroups=8650792"),
     ((1, 1, 2**21, 2**17, 2**24), "grouped_device<256,256> unaligned workgroups=4194816"),
@@ -257,6 +260,7 @@ GROUPED_LIST_DISPATCH_TABLE = [
     ([512] * 16, 8192, 5120, "grouped_listed<256,256> longest=128 workgroups=512"),
     ([16] * 16, 5120, 4096, "grouped_tiled<128,128> longest=80 workgroups=640"),
     ([2304], 8192, 256, "grouped_tiled<256,256> longest=37 workgroups=296"),       # two K steps: not for the chain
+    ([1024] * 4, 4096, 512, "grouped_tiled<256,256> longest=32 workgroups=256"),   # at most one tile per CU: no chain
     ([0, 0], 8192, 512, "nothing to launch"),
 ]
 
