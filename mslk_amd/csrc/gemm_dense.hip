@@ -225,12 +225,22 @@ hipError_t launch_dense_tiled(const GemmProblem& p, hipStream_t s) {
   // M = 768, N = 6144, K = 7168: 47.5 -> 40.6; M = 768, N = K = 8192: 54.6 -> 49.0).
   if (small_tiles > cus && big_tiles <= cus / 2) {
     const int64_t tiles19 = (int64_t)((p.M + 191) / 192) * ((p.N + 127) / 128);
-    // 128 x 160 tiles (wave tile 64 x 80, ring of four) where these fit one per CU as well: a sixth less work per tile than 192 x 128
-    // and no more to move (36 KiB a step), and a tile of less than half the work where the 192-row ones do not fit.  With the
-    // quantizer in front, three layers in turn: M = 140 at 19000 x 8192 56.6 -> 50.2 us, 250 at 16640 x 8192 64.5 -> 57.6, 200 at
-    // 18000 x 4096 28.0 -> 24.3, 1024 at 5000 x 8192 48.2 -> 44.6, 512 at 10000 x 4096 27.9 -> 26.6, 385 at 10240 x 4096 26.4 -> 25.3,
-    // 512 at 9216 x 2048 17.8 -> 17.3, 500 at 10240 x 8192 44.0 -> 41.5; the same at 768 x 6400 x 8192 and 1152 x 4096 x 8192; of 34 shapes none slower by more than the runs of one side differ.
-    if ((int64_t)((p.M + 127) / 128) * ((p.N + 159) / 160) <= cus) return launch_dense_small_tile(kTile128x160, p, s);
+    // 128 x 160 tiles (wave tile 64 x 80, ring of four) where these fit one per CU as well: a sixth less work per K step than 192 x 128
+    // and no more to move (36 KiB a step).  Where the 192-row ones do not fit: one tile per CU with a ring of its own instead of two
+    // passes, from K = 1024 on (three layers in turn, 250 x 16640 9.6 -> 9.1 us, 200 x 18000 10.2 -> 9.1; at K = 256 5.7 / 6.1 and 6.0 / 6.3).  Product alone, cold
+    // weights, 192 x 128 / 128 x 160: K = 4096 500 x 10240 26.0 / 26.3 us (21.8 / 20.9 with weights in the Infinity Cache), 696 x 6144
+    // 15.2 / 13.6, 1152 x 4096 15.6 / 14.6, 1024 x 5000 26.3 / 25.0.
+    // A tile's end is slower than with 192 x 128 ones (40 of 64 lanes store): full tiles lose below K = 2048 (768 x 6144, 1536 x 3072,
+    // 1152 x 4096: K = 512 4.1 / 4.5 us, 1536 6.3 / 6.5), or 4096 where the last of them has most of its columns beyond the end or
+    // nearly none (N % 160 >= 128: 640 x 7168 9.1 / 9.4 at K = 2048, 12.7 / 13.2 at 3072, even at 4096).  But a tile with bounds
+    // tests is slower still, and where 192 x 128 ones end in such tiles with many valid rows or columns and these do not, they win for
+    // any K (956 x 5120 at K = 1536: 7.3 / 6.6; 896 x 5614 9.3 / 8.6).  Of 525 combinations of 75 shapes and K = 512 ... 4096 14 are more
+    // than 2 % slower than without these tiles, 7 % at most (2416 x 2048 x 512: 4.3 / 4.6); 3 % at most is left on the table.  (With weights
+    // in the Infinity Cache full tiles lose 3 - 5 % at K = 2048 and win or tie from 3072 on.)
+    const int64_t tiles160 = (int64_t)((p.M + 127) / 128) * ((p.N + 159) / 160);
+    const bool edges = p.N % 128 ? p.N % 160 <= 128 : p.M % 192 > 64 && p.M % 128 != 0;
+    const int from_k = tiles19 > cus ? 1024 : edges ? 0 : p.N % 160 >= 128 ? 4096 : 2048;
+    if (tiles160 <= cus && p.K >= from_k) return launch_dense_small_tile(kTile128x160, p, s);
     if (tiles19 <= cus) return launch_dense_small_tile(kTile192x128, p, s);
   }
   {
