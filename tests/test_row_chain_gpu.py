@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import mslk_amd  # noqa: F401
-from tests.helpers import grouped_kernel
+from tests.helpers import grouped_kernel, grouped_list_kernel
 
 pytestmark = pytest.mark.gpu
 DEV, F8 = "cuda:0", torch.float8_e4m3fn
@@ -64,22 +64,109 @@ def test_stores_of_ragged_tiles(sizes, N):
 
 
 def test_codes_beyond_a_row_do_not_count():
-    """The last step of K = 400 reads bytes the step before has consumed, and NaN codes among them count once."""
-    sizes, N, K = [600, 700], 2048, 400
-    xq, wq, xs, ws, _ = _operands(sizes, N, K)
-    xq.view(torch.uint8)[5, 300] = 0x7F
-    wq.view(torch.uint8)[1, 77, 390] = 0x7F
-    out = torch.ops.mslk.f8f8bf16_rowwise_grouped_stacked(xq, wq, xs, ws, torch.tensor(sizes).to(DEV)).float()
-    nan = torch.isnan(out)
-    want = torch.zeros_like(nan)
-    want[5, :] = True
-    want[600:, 77] = True
-    assert torch.equal(nan, want)
+    """The last step of K = 400 reads bytes the step before has consumed: they count once, and codes of the rows around do not."""
+    sizes, N, K = [2300, 2400], 8192, 400   # 76 tiles for the 32 CUs of an XCD: two walked each, twelve left over
+    assert grouped_kernel(0, len(sizes), sum(sizes), N, K).startswith("grouped_rows<256,256>")
+    xq, wq, xs, ws, finite = _operands(sizes, N, K)
+    x8, w8 = xq.view(torch.uint8), wq.view(torch.uint8)
+    rows = [5, 255, 2299, 2300, 4698]               # among them the last one of a tile and of a group, and the first of a group
+    cols = {0: [77, 256, 8191], 1: [0, 300, 8190]}
+    places = [272, 383, 384, 399, 0]                # consumed by the step before: from 272 on; by the last one alone: from 384 on
+    for row, k in zip(rows, places):
+        x8[row, k] = 0x7F
+    for g, k in ((0, 300), (1, 390)):
+        for col in cols[g]:
+            w8[g, col, k] = 0x7F
+    want = finite.clone()
+    want[rows] = float("nan")
+    want[:2300, cols[0]] = float("nan")
+    want[2300:, cols[1]] = float("nan")
+    out = torch.ops.mslk.f8f8bf16_rowwise_grouped_stacked(xq, wq, xs, ws, torch.tensor(sizes).to(DEV)).cpu()
+    assert torch.equal(torch.isnan(out), torch.isnan(want))
+    assert torch.equal(out.nan_to_num(0.0), want.nan_to_num(0.0))
 
 
 def test_lists_of_different_k():
-    """A list may hold groups of different K: the chain changes over from one row pitch to another."""
-    parts = [_operands([rows], 4096, K) for rows, K in ((700, 512), (300, 1024), (513, 528), (900, 640), (256, 1536))]
+    """A list may hold groups of different K: the chain changes over from one row pitch to another, and between rows that are a whole number
+    of steps and rows that are not.  At most 32 tiles per panel and 33 entries from one tile of a workgroup to its next (but where its
+    entries go round the end of a pass): the two are of different groups, and no two groups have the same K."""
+    rows = [(700, 300, 513, 900, 256, 1000)[i % 6] for i in range(44)]
+    ks = [512 + 16 * ((i * 13) % 44) for i in range(44)]
+    N = 2048
+    assert len(set(ks)) == len(ks) and any(k % 128 == 0 for k in ks)
+    kernel = grouped_list_kernel(rows, N, ks)
+    assert kernel.startswith("grouped_listed<256,256>") and _longest(kernel) >= 96, kernel   # three tiles per workgroup
+    parts = [_operands([m], N, k) for m, k in zip(rows, ks)]
     out = torch.ops.mslk.f8f8bf16_rowwise_grouped([p[0] for p in parts], [p[1][0] for p in parts], [p[2] for p in parts], [p[3][0] for p in parts])
     for y, p in zip(out, parts):
         assert torch.equal(y.cpu(), p[4])
+
+
+def _longest(kernel):
+    return int(kernel.split("longest=")[1].split()[0])
+
+
+def test_left_over_tiles_of_lists_in_quarters():
+    sizes, N, K = [2304], 8192, 528
+    kernel = grouped_list_kernel(sizes, N, K)
+    assert kernel.startswith("grouped_listed<256,256>")
+    left = _longest(kernel) - 32
+    assert 1 <= left <= 8, kernel   # at most a quarter of the 32 CUs of an XCD
+    xq, wq, xs, ws, want = _operands(sizes, N, K)
+    out = torch.ops.mslk.f8f8bf16_rowwise_grouped([xq], [wq[0]], [xs], [ws[0]])
+    assert torch.equal(out[0].cpu(), want)
+
+
+@pytest.mark.parametrize("form,sizes,N,K", [
+    ("sizes", [8000, 300, 8596], 65536, 272),
+    ("offsets", [129 + i % 128 for i in range(130)], 32768, 272),   # more groups than two lookups hold
+    ("list", [8000, 300, 8596], 65536, 512),
+])
+def test_more_tiles_than_one_lookup_finds(form, sizes, N, K):
+    """A workgroup finds 64 of its tiles at a time: more than 64 * 256 of them."""
+    total, G = sum(sizes), len(sizes)
+    assert sum((m + 255) // 256 for m in sizes) * (N // 256) > 64 * 256
+    kernel = grouped_list_kernel(sizes, N, K) if form == "list" else grouped_kernel(1 if form == "offsets" else 0, G, total, N, K)
+    assert kernel.startswith("grouped_listed<256,256>" if form == "list" else "grouped_rows<256,256>"), kernel
+    if form == "list":
+        assert _longest(kernel) > 64 * 32 + 32
+    g = torch.Generator(device=DEV).manual_seed(N + K + G)
+    codes = torch.arange(-8, 9, device=DEV).float().to(F8).view(torch.uint8)
+    draw = lambda *shape: codes[torch.randint(0, 17, shape, generator=g, device=DEV, dtype=torch.int32)].view(F8)
+    xq, wq = draw(total, K), torch.stack([draw(N, K).view(torch.uint8) for _ in sizes]).view(F8)
+    xs = torch.pow(2.0, torch.randint(-3, 4, (total,), generator=g, device=DEV).float())
+    ws = torch.pow(2.0, torch.randint(-3, 4, (G, N), generator=g, device=DEV).float())
+    m = torch.tensor(sizes, device=DEV)
+    if form == "sizes":
+        out = torch.ops.mslk.f8f8bf16_rowwise_grouped_stacked(xq, wq, xs, ws, m)
+    elif form == "offsets":
+        out = torch.empty(total, N, dtype=torch.bfloat16, device=DEV)
+        torch.ops.mslk.f8f8bf16_rowwise_grouped_mm(xq, wq, xs, ws, m.cumsum(0).to(torch.int32), out)
+    else:
+        out = torch.cat(torch.ops.mslk.f8f8bf16_rowwise_grouped(list(xq.split(sizes)), list(wq.unbind(0)), list(xs.split(sizes)), list(ws.unbind(0))))
+    row = 0
+    for i, size in enumerate(sizes):   # sums below 2^24: exact in fp32
+        w = wq[i].float()
+        for r in range(row, row + size, 4096):
+            e = min(r + 4096, row + size)
+            want = ((xq[r:e].float() @ w.t()) * ws[i] * xs[r:e, None]).to(torch.bfloat16)
+            assert torch.equal(out[r:e], want), (i, r)
+        row += size
+
+
+@pytest.mark.parametrize("K", [2880, 1040, 400])
+def test_rows_do_not_depend_on_the_tiles_they_fall_into(K):
+    """Random codes of the whole range, whose sums round: the last step of the chain has its codes at the end of the matrix instruction's
+    k positions and zeros in front, the other tiles the reverse, and the sums are the same bit for bit."""
+    N, rows = 8192, 2304
+    g = torch.Generator().manual_seed(K)
+    draw = lambda *shape: (torch.randint(0, 127, shape, generator=g) + 128 * torch.randint(0, 2, shape, generator=g)).to(torch.uint8).view(F8).to(DEV)
+    xq, wq = draw(2 * rows, K), draw(2, N, K)
+    xs, ws = (torch.rand(n, generator=g).add(0.5).to(DEV) for n in ((2 * rows,), (2, N)))
+    stacked = lambda x, w, s, t, sizes: torch.ops.mslk.f8f8bf16_rowwise_grouped_stacked(x, w, s, t, torch.tensor(sizes).to(DEV))
+    assert grouped_kernel(0, 2, 2 * rows, N, K) == grouped_kernel(0, 1, rows, N, K) == "grouped_rows<256,256> workgroups=512"
+    walked = stacked(xq, wq, xs, ws, [rows, rows])[:rows]                    # 72 tiles for the 32 CUs of an XCD: two each, eight left over
+    quarters = stacked(xq[:rows], wq[:1], xs[:rows], ws[:1], [rows])         # 36: the last four in quarters
+    assert grouped_kernel(0, 1, 128, N, K).startswith("grouped_device<128,128>")
+    small = torch.cat([stacked(xq[r:r + 128], wq[:1], xs[r:r + 128], ws[:1], [128]) for r in range(0, rows, 128)])
+    assert torch.equal(walked, quarters) and torch.equal(walked, small)
