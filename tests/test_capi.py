@@ -269,6 +269,9 @@ GROUPED_LIST_DISPATCH_TABLE = [
     ([16] * 16, 5120, 4096, "grouped_tiled<128,128> longest=80 workgroups=640"),
     ([2304], 8192, 256, "grouped_tiled<256,256> longest=37 workgroups=296"),       # two K steps: not for the chain
     ([1024] * 4, 4096, 512, "grouped_tiled<256,256> longest=32 workgroups=256"),   # at most one tile per CU: no chain
+    ([6784], 2816, 5120, "grouped_tiled<256,256> longest=44 workgroups=352"),      # a pass and three eighths: no workgroup has a second tile
+    ([2304], 8192, 512, "grouped_listed<256,256> longest=37 workgroups=512"),      # a pass and a sixth: the rest in quarters
+    ([700] * 5, 8192, 640, "grouped_listed<256,256> longest=60 workgroups=512"),   # more than a pass and three quarters: two tiles each
     ([0, 0], 8192, 512, "nothing to launch"),
 ]
 
