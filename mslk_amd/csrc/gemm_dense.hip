@@ -226,20 +226,25 @@ hipError_t launch_dense_tiled(const GemmProblem& p, hipStream_t s) {
   if (small_tiles > cus && big_tiles <= cus / 2) {
     const int64_t tiles19 = (int64_t)((p.M + 191) / 192) * ((p.N + 127) / 128);
     // 128 x 160 tiles (wave tile 64 x 80, ring of four) where these fit one per CU as well: a sixth less work per K step than 192 x 128
-    // and no more to move (36 KiB a step).  Where the 192-row ones do not fit: one tile per CU with a ring of its own instead of two
-    // passes, from K = 1024 on (three layers in turn, 250 x 16640 9.6 -> 9.1 us, 200 x 18000 10.2 -> 9.1; at K = 256 5.7 / 6.1 and 6.0 / 6.3).  Product alone, cold
-    // weights, 192 x 128 / 128 x 160: K = 4096 500 x 10240 26.0 / 26.3 us (21.8 / 20.9 with weights in the Infinity Cache), 696 x 6144
-    // 15.2 / 13.6, 1152 x 4096 15.6 / 14.6, 1024 x 5000 26.3 / 25.0.
-    // A tile's end is slower than with 192 x 128 ones (40 of 64 lanes store): full tiles lose below K = 2048 (768 x 6144, 1536 x 3072,
-    // 1152 x 4096: K = 512 4.1 / 4.5 us, 1536 6.3 / 6.5), or 4096 where the last of them has most of its columns beyond the end or
-    // nearly none (N % 160 >= 128: 640 x 7168 9.1 / 9.4 at K = 2048, 12.7 / 13.2 at 3072, even at 4096).  But a tile with bounds
-    // tests is slower still, and where 192 x 128 ones end in such tiles with many valid rows or columns and these do not, they win for
-    // any K (956 x 5120 at K = 1536: 7.3 / 6.6; 896 x 5614 9.3 / 8.6).  Of 525 combinations of 75 shapes and K = 512 ... 4096 14 are more
-    // than 2 % slower than without these tiles, 7 % at most (2416 x 2048 x 512: 4.3 / 4.6); 3 % at most is left on the table.  (With weights
-    // in the Infinity Cache full tiles lose 3 - 5 % at K = 2048 and win or tie from 3072 on.)
+    // and no more to move (36 KiB a step), but a slower end (40 of 64 lanes store).  4455 products of 779 shapes (M = 129 ... 2700), cold weights,
+    // time of the 160-column tiles over the time without them, in the geometric mean:
+    //   192 x 128 tiles do not fit one per CU (two passes of 128 x 128 instead): K = 256 1.10, 384 1.02, 512 0.93, 768 0.85, 1024 0.84, 2048 0.77,
+    //     8192 0.77; rows of Y that are not 16-byte aligned (N % 8) 512 1.15, 768 1.01, 1024 0.96, 2048 0.82, 8192 0.76;
+    //   N % 8 != 0: K <= 512 1.05, <= 1024 1.03, <= 2048 0.98, <= 4096 0.95, beyond 0.93;
+    //   192 x 128 tiles end in a ragged column: 0.95 - 0.97 for every K (a tile with bounds tests is slower, and theirs has more rows);
+    //   full columns, M % 192 > 128 (such a tile again, with most rows valid): 0.96 at short K, 0.92 beyond 2048;
+    //   full columns and M % 128 == 0: K <= 512 1.09, <= 1024 1.05, <= 2048 1.04, <= 4096 1.02, beyond 1.01 (from 7168 on 0.99);
+    //   full columns, M % 192 < 64: 1.10, 1.07, 1.04, 1.00, 0.99; M % 192 == 0: 1.11, 1.06, 1.00, 0.96, 0.93; between 1.02, 1.02, 1.01, 0.98, 0.97.
+    // By the rule below 49 of 3340 products that 192 x 128 tiles fit are more than 5 % slower than on those, 12 % at most (2176 x 2055 x 2880:
+    // 22.7 / 25.4 us), and 12 more than 5 % slower than on 160-column ones, 9 % at most (302 x 11520 x 512).
     const int64_t tiles160 = (int64_t)((p.M + 127) / 128) * ((p.N + 159) / 160);
-    const bool edges = p.N % 128 ? p.N % 160 <= 128 : p.M % 192 > 64 && p.M % 128 != 0;
-    const int from_k = tiles19 > cus ? 1024 : edges ? 0 : p.N % 160 >= 128 ? 4096 : 2048;
+    const int last_rows = p.M % 192;
+    int from_k = 2048;
+    if (tiles19 > cus) from_k = p.N % 8 ? 1024 : 512;
+    else if (p.N % 8) from_k = 1024;
+    else if (p.N % 128 || last_rows > 128) from_k = 0;
+    else if (p.M % 128 == 0) from_k = 7168;
+    else if (last_rows > 0 && last_rows < 64) from_k = 3072;
     if (tiles160 <= cus && p.K >= from_k) return launch_dense_small_tile(kTile128x160, p, s);
     if (tiles19 <= cus) return launch_dense_small_tile(kTile192x128, p, s);
   }

@@ -201,14 +201,19 @@ DISPATCH_TABLE = [
     ((1536, 6144, 1024, 0, 0, 0, 1), "dense_tiled<256,256,waves=2x2,ring=0> tiles=144"),                     # short K keeps the fused epilogue of the 256 x 256 tiles
     ((768, 7168, 6144, 0, 0, 0, 1), "dense_tiled<192,128,waves=2x2,ring=3> tiles=224"),
     ((500, 10240, 8192, 0, 0, 0, 1), "dense_tiled<128,160,waves=2x2,ring=4> tiles=256"),                      # less work per tile than 192 x 128, still one per CU
-    ((1536, 3072, 2048, 0, 0, 0, 1), "dense_tiled<128,160,waves=2x2,ring=4> tiles=240"),                      # full tiles: from K = 2048 on
-    ((1536, 3072, 1536, 0, 0, 0, 1), "dense_tiled<192,128,waves=2x2,ring=3> tiles=192"),
-    ((640, 7168, 4096, 0, 0, 0, 1), "dense_tiled<128,160,waves=2x2,ring=4> tiles=225"),                       # the last column tile is nearly full: from 4096 on
-    ((640, 7168, 3072, 0, 0, 0, 1), "dense_tiled<192,128,waves=2x2,ring=3> tiles=224"),
+    ((1152, 4096, 2048, 0, 0, 0, 1), "dense_tiled<192,128,waves=2x2,ring=3> tiles=192"),                      # 128-row tiles full as well: not for the 160-column ones
+    ((640, 7168, 4096, 0, 0, 0, 1), "dense_tiled<192,128,waves=2x2,ring=3> tiles=224"),
+    ((768, 6400, 7168, 0, 0, 0, 1), "dense_tiled<128,160,waves=2x2,ring=4> tiles=240"),                       # ... but very long K
+    ((960, 4608, 2048, 0, 0, 0, 1), "dense_tiled<128,160,waves=2x2,ring=4> tiles=232"),                       # 192-row tiles full: from K = 2048 on
+    ((960, 4608, 1536, 0, 0, 0, 1), "dense_tiled<192,128,waves=2x2,ring=3> tiles=180"),
+    ((580, 7168, 3072, 0, 0, 0, 1), "dense_tiled<128,160,waves=2x2,ring=4> tiles=225"),                       # 4 of 192 rows in the last row tile: from 3072 on
+    ((580, 7168, 2048, 0, 0, 0, 1), "dense_tiled<192,128,waves=2x2,ring=3> tiles=224"),
     ((956, 5120, 512, 0, 0, 0, 1), "dense_tiled<128,160,waves=2x2,ring=4> tiles=256"),                        # 188 of 192 rows in the last row tile
-    ((896, 5614, 512, 0, 0, 0, 1), "dense_tiled<128,160,waves=2x2,ring=4> tiles=252"),                        # 110 of 128 columns in the last column tile
-    ((250, 16640, 1024, 0, 0, 0, 1), "dense_tiled<128,160,waves=2x2,ring=4> tiles=208"),                      # 192 x 128 tiles would need two passes
-    ((250, 16640, 512, 0, 0, 0, 1), "dense_tiled<128,128,waves=2x2,ring=0> tiles=260"),
+    ((896, 5616, 512, 0, 0, 0, 1), "dense_tiled<128,160,waves=2x2,ring=4> tiles=252"),                        # a ragged last column tile
+    ((896, 5614, 512, 0, 0, 0, 1), "dense_tiled<192,128,waves=2x2,ring=3> tiles=220"),                        # rows of Y off 16 bytes: from 1024 on
+    ((896, 5614, 1024, 0, 0, 0, 1), "dense_tiled<128,160,waves=2x2,ring=4> tiles=252"),
+    ((250, 16640, 512, 0, 0, 0, 1), "dense_tiled<128,160,waves=2x2,ring=4> tiles=208"),                       # 192 x 128 tiles would need two passes
+    ((250, 16640, 384, 0, 0, 0, 1), "dense_tiled<128,128,waves=2x2,ring=0> tiles=260"),
     ((128, 512, 14336, 0, 0, 0, 1), "splitk_partial<64,64,waves=4x1,ring=5> slices=8 + splitk_reduce"),       # few tiles, long K, workspace given
     ((128, 512, 14336, 0, 0, 0, 0), "dense_tiled<128,32,waves=4x1,ring=8> weights streamed tiles=16"),         # ... and not given
     ((128, 4096, 14336, 2, 1, 0, 1), "splitk_partial<64,64,waves=4x1,ring=5> slices=2 + splitk_reduce"),

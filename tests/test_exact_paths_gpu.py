@@ -376,15 +376,15 @@ def test_weight_streaming_kernel_exact_on_k_loops_that_do_not_divide_among_its_w
 
 @pytest.mark.parametrize("bias_dtype,fp16_out", [(None, False), (torch.float32, False), (torch.bfloat16, True)])
 @pytest.mark.parametrize("M,N,K,tile", [
-    (500, 10240, 384, "128,160"),    # fewer K steps than ring buffers
-    (512, 10240, 2048, "128,160"),   # 256 full tiles
-    (385, 10240, 2064, "128,160"),   # one row in the last row tile, a K tail
-    (500, 10112, 512, "128,160"),    # a last column tile of 32 columns
-    (640, 8120, 528, "128,160"),     # five row tiles; the last column tile ends inside the second wave's columns
-    (500, 10093, 768, "128,160"),    # rows of Y that are 2-byte aligned
+    (956, 5120, 384, "128,160"),     # fewer K steps than ring buffers
+    (512, 10080, 2048, "128,160"),   # 252 full tiles
+    (385, 10240, 3088, "128,160"),   # one row in the last row tile, a K tail
+    (956, 4992, 512, "128,160"),     # a last column tile of 32 columns
+    (640, 8136, 528, "128,160"),     # five row tiles; the last column tile ends inside the second wave's columns
+    (500, 10093, 1040, "128,160"),   # rows of Y that are 2-byte aligned
     (512, 10240, 384, "192,128"),    # the same edges on the tiles that short K takes
     (385, 10240, 1040, "192,128"),
-    (640, 8136, 528, "192,128"),
+    (640, 8137, 528, "192,128"),
 ])
 def test_tiles_of_160_columns_exact(M, N, K, tile, bias_dtype, fp16_out):
     """Stores in which not every lane takes part, and a wave's columns that begin and end inside a line."""
