@@ -251,8 +251,7 @@ static hipError_t launch_grouped_shape(const GroupTable& in, hipStream_t s) {
     // Without a second tile the chain gains nothing: at most one tile per CU, or up to a pass and three quarters of whole tiles, each with a workgroup
     // of its own.  (120 lists of the latter kind, K = 512 ... 8192, one per workgroup / in the chain: 0.90 - 1.11 of the time, 0.988 in the mean, 0.98 from
     // K = 4096 on; 1 x 6784 x 2816 x 5120 101 / 105 us, 8 x 5096 x 4096 x 640 26.6 / 28.8, 16 x 3104 x 7168 x 512 31.9 / 29.6.)
-    const SliceShares shares(longest, wgs_per_xcd);
-    bool chain = shares.walked > wgs_per_xcd || (longest > wgs_per_xcd && shares.pieces > 1);
+    bool chain = !SliceShares(longest, wgs_per_xcd).no_second_tile(longest);
     for (int i = 0; i < n; ++i) chain = chain && chain_takes(t.g[i].N, t.g[i].K, t.g[i].xq, t.g[i].wq, t.g[i].ws, t.g[i].y);
     if (chain) {
       if (dispatch_probe_record("grouped_listed<%d,%d> longest=%d workgroups=%d", BM, BN, longest, 2 * wgs_per_xcd * kXcds)) return hipSuccess;

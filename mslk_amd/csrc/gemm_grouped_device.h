@@ -348,12 +348,13 @@ struct RowTile {
 // the slice each per pass.  What is left over for a last pass, as long as it is at most three quarters of one, is
 // given to further workgroups, one tile each, which the hardware starts where one of the first ones ends: tiles cost what their
 // rows cost, and the workgroups that were given cheap ones take what is left.  At most a quarter of a pass is cut into quarters of tiles besides.
-// (16 experts x 5120 x 4096 over 8192 rows, 780 tiles: a fourth pass with 12 of 256 workgroups busy, 198 -> 156 us.)
+// (16 experts x 5120 x 4096 over 8192 skewed rows, 780 tiles: a fourth pass with 12 of 256 workgroups busy 184 us, left-over tiles whole 185, in
+// quarters 167; 64 groups, 16384 rows x 2816 x 2880 204 / 198 / 197.)
 // Neighbouring entries are the row tiles of a panel (local_tile), the last of which may be ragged.  From pass to pass a workgroup
 // moves on by wgs + turn entries, and wgs + turn has no divisor in common with any number of row tiles in a panel: every workgroup gets
 // its share of the ragged ones.  With entry i for workgroup i % wgs half of the 32 workgroups of an XCD were given all full tiles
-// of groups of 300 rows, and the launch took as long as full tiles do (64 x 300 rows x 4096 x 768: 121 -> 105 us; 128 x 257 x 2048 x 768
-// 122 -> 98; 16 x 257 x 8192 x 2048 107 -> 97).
+// of groups of 300 rows, and the launch took as long as full tiles do (64 x 300 rows x 4096 x 2048: 215 us, now 194; 128 x 257 x 2048 x 768
+// 112 / 92; 16 x 257 x 8192 x 2048 107 / 97; skewed sizes the same within 2 %).
 struct SliceShares {
   int wgs, turn;
   int walked;        // entries of the slice that the first workgroups walk
@@ -369,6 +370,8 @@ struct SliceShares {
   }
   // Entry of the slice that workgroup `worker` < wgs walks in `pass`: its own if it is below `walked`.
   __host__ __device__ int walked_entry(int worker, int pass) const { return pass * wgs + (worker + pass * turn) % wgs; }
+  // Every workgroup with work has one whole tile: the chain gains nothing.
+  __host__ __device__ bool no_second_tile(int tiles) const { return tiles <= wgs || (walked <= wgs && pieces == 1); }
   // Left-over entry, and piece of it, of workgroup `worker` >= wgs: one of the slice if it is below `tiles`.
   __host__ __device__ int left_entry(int worker) const { return walked + (worker - wgs) / pieces; }
   __host__ __device__ int left_piece(int worker) const { return (worker - wgs) % pieces; }
@@ -403,7 +406,7 @@ MSLK_AMD_DEVINL void walk_row_tiles(char* lds, RowTile t, Next&& next) {
   using Plain = GemmTile<TS, 0, false, true, TS::LA / 2, false, false, true>;
   using Streamed = GemmTile<TS, 0, false, true, TS::LA / 2, false, true, true>;
   RowTile n;
-  auto operands = [](const RowTile& w) { return TileOperands{w.a, w.b, w.m_rem, w.n_rem, w.K, (uint32_t)w.K}; };
+  auto operands = [](const RowTile& w) { return TileOperands{w.a, w.b, w.m_rem, w.n_rem, (uint32_t)w.K}; };
   Plain tile;
   Streamed streamed;
   TileChain<TS> chain(lds);

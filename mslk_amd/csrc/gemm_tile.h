@@ -73,10 +73,10 @@ struct TileChain {
     { char* t = b_cur; b_cur = b_nxt; b_nxt = b_far; b_far = t; }
   }
 };
-// ... the operands of one tile (first row of each, valid rows >= 1, bytes of a row to consume, bytes between rows) ...
+// ... the operands of one tile (first row of each, valid rows >= 1, bytes between rows) ...
 struct TileOperands {
   const uint8_t *a, *b;
-  int rows_a, rows_b, K;
+  int rows_a, rows_b;
   uint32_t ld;
 };
 // ... and the scales of a lane's sums.
@@ -279,8 +279,9 @@ struct GemmTile {
 
   // Chunk permutation of the WQ tile.  DIRECT: the 16 rows of a fragment differ in bits 0, 1, 3 and 4.  A 16-byte read is served
   // 16 lanes at a time, but not 16 consecutive ones: rows with equal bits 3 and 4 at one chunk together with the other rows at
-  // the chunk two further (lanes 0 - 3, 12 - 15, 20 - 27 first).  With bits 3 and 4 simply side by side above bit 1 two rows of such a set shared their
-  // banks and a K step took 8 % longer.
+  // the chunk two further (lanes 0 - 3, 12 - 15, 20 - 27 first).  With bits 3 and 4 simply side by side above bit 1 two rows of such a set share their
+  // banks: 4 x 4096 rows x 4096 x 4096 8.4 of 25.2 million LDS cycles are conflicts, none of 16.8 in this order (203 against 199 us there, the same
+  // time in launches that wait for memory).
   MSLK_AMD_DEVINL static int swz_b(int row) {
     if constexpr (!DIRECT) return lds_swz(row);
     const int r3 = (row >> 3) & 1, r4 = (row >> 4) & 1;
@@ -401,12 +402,14 @@ struct GemmTile {
     step_tail<NEXT, PENDING, NA_TAIL, FIRST>(a_nxt, b_nxt, acc, xf, wf0, wf_last, a_tail_dst, k_a_tail);
   }
 
-  // The part of a full-tile K step in front of its barrier: every n fragment but the last, with the step's DMA loads.
-  // Leaves the last WQ fragment of the step in `wf_last`.
+  // FIRST: the product alone instead of its sum with `acc`.
   template <bool FIRST>
   MSLK_AMD_DEVINL static void multiply(const v8i& wf, const v8i& xf, v4f& acc) {
     acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, xf, FIRST ? v4f{0.f, 0.f, 0.f, 0.f} : acc, 0, 0, 0, 0, 0, 0);
   }
+
+  // The part of a full-tile K step in front of its barrier: every n fragment but the last, with the step's DMA loads.
+  // Leaves the last WQ fragment of the step in `wf_last`.
   template <int NA_HEAD, bool DMA_B, bool FIRST = false>
   MSLK_AMD_DEVINL void step_head(const char* b_cur, char* a_dst, char* b_far, int k_a, int k_b, v4f (&acc)[TS::FN][TS::FM],
                                  v8i (&xf)[TS::FM], const v8i& wf0, v8i& wf_last) {
@@ -771,11 +774,12 @@ struct GemmTile {
   // ---- Tiles one after the other without a gap (two-plus-three buffers, DIRECT, K > 2 kBK, K % 16 == 0) ----
   // The K steps of consecutive tiles form one chain: the last two steps of a tile issue the first loads of the next one in the
   // places where the steps before them issue the loads of their own tile, so a tile starts with its first operands in LDS.  The
-  // epilogue touches no LDS and runs while the next tile's loads land.  What this replaces: of the 15 us that a tile of six K steps took
-  // (128 experts x 2048 x 768), 1 us went into finding the tile, 2 - 2.5 into the wait for its first operands, 4 into the epilogue
-  // and 0.5 into starting the workgroup; now 12 us, of them 2.8 for the epilogue (vector arithmetic: 3.5 instructions for each of 256 sums).
+  // epilogue touches no LDS and runs while the next tile's loads land.  Tiles one per workgroup pay for finding the tile, for its first
+  // operands, for an epilogue through LDS and for the start of the workgroup with nothing else running on the CU.  Four full tiles of six steps per
+  // CU (128 x 256 rows x 2048 x 768, cold weights): 83.9 -> 75.8 us; with skewed sizes 102.6 -> 90.2; 16384 rows x 8192 x 1024 142.7 -> 132.4; even from K = 4096 on.
   // A K that is no multiple of the step ends in a step over the last kBK bytes of the rows: what the step before has
-  // consumed already is cleared in the fragments of both operands.
+  // consumed already is cleared in the fragments of both operands.  (The codes then stand at the end of the instruction's k positions, in
+  // other tiles in front; the sums are the same bit for bit.)
   using Chain = TileChain<TS>;
   using Scales = TileScales<TS>;
 
@@ -888,7 +892,7 @@ struct GemmTile {
     c.advance();
   }
 
-  // DIRECT: row of fragment row tm that this lane stores, and its first column of the fragment pair 2 t, 2 t + 1
+  // DIRECT: first of the 16 rows of the tile that m fragment tm of this wave holds.
   template <bool ILV>
   MSLK_AMD_DEVINL static int direct_row(int tm) {
     const int wm = wave_id() / TS::WN;
@@ -921,9 +925,11 @@ struct GemmTile {
   // FMV < FM: only that many m fragments of a wave have valid rows, dealt to the wave rows round-robin.
   // A lane's eight columns are 16 of 64 bytes that one fragment pair gives each of 16 rows.  Two pairs make a 128-byte line: the lanes
   // of rows 0 - 7 and 8 - 15 exchange one of their two pieces (row_ror:8), so that one store writes whole lines of eight rows and the
-  // next those of the other eight, past the L2.  Half lines were slow past the L2 (64 x 512 rows x 2048 x 768: 81 against 62 us), and left to the L2
-  // they displaced operands: eight groups of 1500 rows and 56 of 40 as a list, x 4096 x 4096, 365 us (333 now), 64 groups of 16384
-  // rows x 2816 x 2880 220 (203), 64 x 150 rows x 4096 x 2048 124 (115); 64 x 300 rows x 4096 x 768 102 (95), of cold weights.
+  // next those of the other eight, past the L2.  Cold weights, in us: half lines past the L2 / half lines or whole ones left to the L2 (the same
+  // within 2 %) / as it is: 128 x 256 rows x 2048 x 768 88 / 78 / 76, 64 groups of 16384 rows x 2816 x 2880 208 / 209 / 198, 64 x 150 rows x 4096 x 2048 123 / 124 /
+  // 115, 64 x 300 x 4096 x 768 104 / 104 / 94, a list of eight groups of 1500 rows and 56 of 40, x 4096 x 4096, 345 / 367 / 337: output left to the L2 displaces
+  // operands.  Where the operands of a pass fit beside it, it is 4 - 6 % better there: 64 x 512 rows x 2048 x 768 78 / 66 / 70, 32 groups of 16384 rows x 4096 x
+  // 1408 122 / 108 / 113.
   template <bool ALL, int FMV>
   MSLK_AMD_DEVINL void epilogue_direct(v4f (&acc)[TS::FN][TS::FM], const Scales& sc, uint16_t* y, int m_rem, int n_rem, int N) {
     constexpr bool ILV = FMV < TS::FM;
